@@ -110,6 +110,7 @@ static void model_create(Model& mm, const hoefem_model_desc* d) {
     m->scatter.build(m->pattern, m->ne, eoff.data(), m->conn.data(), m->colors, 2);
     // device data
     m->pattern.upload(m->stream);
+    m->grid.build(m->pattern, nullptr, grid_device_cus(), m->stream);
     m->scatter.upload(m->stream);
     m->d_vertices.upload(m->vertices, m->stream);
     std::vector<int32_t> soa((size_t)n * m->ne);
@@ -653,14 +654,16 @@ static hoefem_status sim_step(Sim& s, double t, double dt, double* u, double* v,
 // ends on the device. Scenes therefore never wait for each other, and each scene's u and v are the
 // ones sim_step gives it, bit for bit. A scene whose single-step attempt fails continues alone with
 // the substepping of sim_step once the others are done.
-// Scenes go to CG pools by size (DOFs below 2e4, below 8e4, larger), each on its own stream, so the
-// iterations of small systems do not wait for the launches the large ones lengthen.
+// Scenes whose systems fit the resident grid share its pool; the others go to CG pools by size (DOFs below
+// 2e4, below 8e4, larger), each on its own stream, so the iterations of small systems do not wait for
+// the launches the large ones lengthen.
 constexpr int BATCH_POOLS = 3;
 constexpr int64_t BATCH_POOL_DOFS[BATCH_POOLS - 1] = {20000, 80000};
 
 struct Batch {
     std::vector<Sim*> sims;
     CgBatch cg[BATCH_POOLS];
+    GridBatch grid;
     std::vector<hipEvent_t> ev;  // one per scene
     ~Batch() {
         for (hipEvent_t e : ev) (void)hipEventDestroy(e);
@@ -703,17 +706,20 @@ static void batch_step(Batch& B, const double* dt, double* const* u, double* con
     }
     const bool fp32 = B.sims[0]->fp32_jacobian();
     std::vector<int> pool_of(ns);
-    int pool_size[BATCH_POOLS] = {};
+    int pool_size[BATCH_POOLS + 1] = {};
     for (size_t i = 0; i < ns; ++i) {
-        const int64_t ndof = 3 * B.sims[i]->model->nv;
+        const Sim& s = *B.sims[i];
+        const int64_t ndof = 3 * s.model->nv;
         int c = 0;
         while (c < BATCH_POOLS - 1 && ndof >= BATCH_POOL_DOFS[c]) ++c;
+        if ((s.schwarz ? s.schwarz->grid : s.model->grid).W) c = BATCH_POOLS;  // the resident grid's
         pool_of[i] = c;
         pool_size[c] += 1;
     }
-    std::unique_ptr<CgPool> pools[BATCH_POOLS];
+    std::unique_ptr<CgPool> pools[BATCH_POOLS + 1];
     for (int c = 0; c < BATCH_POOLS; ++c)
         if (pool_size[c]) pools[c] = make_cg_pool(B.cg[c], fp32, pool_size[c]);
+    if (pool_size[BATCH_POOLS]) pools[BATCH_POOLS] = make_grid_pool(B.grid, fp32);
     std::vector<BatchScene> q(ns);
     const auto t0 = std::chrono::steady_clock::now();
     auto elapsed_ms = [&]() {
@@ -800,7 +806,7 @@ static void batch_step(Batch& B, const double* dt, double* const* u, double* con
         mark(i);
     }
     std::vector<int> ended;
-    std::vector<int> owner[BATCH_POOLS];  // scene of every pool system
+    std::vector<int> owner[BATCH_POOLS + 1];  // scene of every pool system
     const double c = 1e-4, alpha_min = 1e-6;
     const double initial[3] = {1.0, 0.75, 0.5};
     while (true) {
@@ -866,7 +872,7 @@ static void batch_step(Batch& B, const double* dt, double* const* u, double* con
             }
         }
         bool any_ended = false;
-        for (int pc = 0; pc < BATCH_POOLS; ++pc) {
+        for (int pc = 0; pc <= BATCH_POOLS; ++pc) {
             if (!pools[pc]) continue;
             ended.clear();
             pools[pc]->progress(ended);

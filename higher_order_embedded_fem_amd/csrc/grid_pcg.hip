@@ -1,0 +1,1048 @@
+// Preconditioned conjugate gradient (fenris/src/cg.rs:377-482) as one resident grid: the whole solve of
+// a system that fits the chip's register files and L2s runs in one launch (in chunks of iterations), its
+// work-groups exchanging vectors and dot products through memory instead of through kernel boundaries.
+//
+// Why. The two-kernel iteration of solver.hip costs 5-9 us per kernel on the smallest systems (launch,
+// descriptor, status, partial sums, row entries, columns and gathered vectors: a chain of dependent memory
+// reads that starts anew in every kernel) and reads every matrix value from the Infinity Cache in every
+// iteration on the larger ones. Here the matrix values, the columns and the vectors of a work-group's rows
+// stay in its registers and LDS between iterations; an iteration moves one vector entry per node and
+// phase, and its chain is: store own entries, post a partial sum, poll the others', load the neighbours'.
+//
+// Split. Work-group b owns a contiguous range of nodes and their rows of A and P, at most 170 nodes (one
+// vector component per thread). Thread t holds a run of consecutive 3x3 blocks of those rows (sA of A, then
+// sP of P), so every thread has the same work whatever the row lengths are; where a run leaves a row it
+// writes the row's partial sum to LDS, and the thread of each row component adds its row's partials in
+// order. The first N blocks of a thread stay in registers, the rest is re-read in every iteration from a
+// work-group-private, coalesced copy (L2-resident up to about 30 MB).
+//
+// Iteration k (z, p, r: own entries in registers, own and neighbour entries in LDS):
+//   A  p <- z + beta p for own and neighbour nodes (every work-group computes its neighbours' p itself, so
+//      only z is exchanged); Ap = A p; publish Ap; exchange p.Ap
+//   B  x += alpha p, r <- r - alpha Ap (neighbours' r likewise); z = P r; publish z; exchange z.r, |r|^2
+// The stopping tests and their order are those of the two-kernel path.
+//
+// Exchange. Vector entries and partial sums are stored and loaded with agent scope (write-through stores,
+// loads past the L2), so no cache is written back or invalidated, and every value is its own flag: an entry
+// holds a sentinel (a signalling NaN, which no arithmetic yields) until its owner stores it, and its
+// readers poll it. A phase thus costs one trip of a store and one of a load, the vector entries' beside the
+// partial sums'. Every work-group adds all partial sums in the same order, so all agree on alpha, beta and
+// the stopping tests bit for bit. Four sets of entries are used in turn. A work-group stores its entries of
+// phase m and the sentinel into those of phase m + 2: their previous use, phase m - 2, has been read by all
+// (they posted phase m - 1 after it), and the sentinel is in memory before the work-group posts phase m + 1
+// (its waves wait for their older stores, s_waitcnt vmcnt(0), before the stores of a phase), so
+// before anyone can poll phase m + 2.
+//
+// Residency. The work-groups wait for each other, so all of a launch's must be resident: launches are
+// admitted against the device's number of CUs (GridSlots below), one work-group per CU. Every wait is
+// bounded (GRID_POLL_LIMIT); a launch that cannot make progress ends with an error status and the caller
+// falls back to the two-kernel path.
+#include <algorithm>
+#include <cmath>
+#include <condition_variable>
+#include <map>
+#include <mutex>
+#include <system_error>
+#include <thread>
+#include <type_traits>
+
+#include "grid_pcg.hpp"
+
+namespace hoefem {
+
+namespace {
+
+constexpr unsigned long long GRID_EMPTY = 0x7ff4deadbeef0001ull;  // slot sentinel
+constexpr int GRID_POLL_LIMIT = 1 << 21;                           // about 2 s of polling
+constexpr int GRID_WAVES = GRID_THREADS / 64;
+// copies of the partial sums, each read by an eighth of the work-groups: 256 work-groups polling one array
+// queue at its few memory channels (3.1 us per exchange at 256 work-groups against 2.4 with 8 copies)
+constexpr int GRID_COPIES = 8;
+
+__device__ inline double agent_load(const double* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void agent_store(double* p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+    return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// the sum over the wavefront's lanes, the same in every lane (register lane shifts, no LDS)
+__device__ inline double wave_total(double v) {
+    v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: lane 15 of each row of 16 holds the row's sum
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+    v = dpp_add<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3: lane 63 holds the total
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+__device__ inline float fmav(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ inline double fmav(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// f(0), f(1), .. f(N - 1) with compile-time indices (register arrays stay in registers)
+template <int N, class F>
+__device__ __forceinline__ void unrolled(F&& f) {
+    if constexpr (N > 0) {
+        unrolled<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
+
+__device__ inline bool is_empty(double v) { return (unsigned long long)__double_as_longlong(v) == GRID_EMPTY; }
+
+// A barrier that orders LDS accesses only: global stores and loads in flight are not waited for
+__device__ inline void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// A thread's run of consecutive blocks of its work-group's rows: the block (node, j) it stands at
+struct Run {
+    int node, j, k, left;
+    int64_t base;
+};
+
+}  // namespace
+
+// N blocks of a thread in registers: 10 of FP64 (180 of the 256 registers that two waves per SIMD leave a
+// thread) or 16 of FP32, the next S.nlds in LDS; pairs of register blocks share one uniform test and have
+// their LDS reads in flight together.
+// K systems in one launch (descriptors in the kernel arguments), their work-groups one after the other.
+template <class VT, int N, int K>
+__global__ __launch_bounds__(GRID_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_grid_pcg(
+    const GridSegs<VT, K> all) {
+#pragma clang fp contract(off)
+#define INLINE __attribute__((always_inline))
+    extern __shared__ double lds[];
+    __shared__ double s_w[GRID_WAVES][2];
+    __shared__ double s_tot[2];
+    __shared__ int s_bad;
+    __shared__ double s_x[GRID_THREADS], s_v[GRID_THREADS], s_d[GRID_THREADS];  // own x; Ap or z; diagonal entries
+    __shared__ uint32_t s_rows[2][GRID_THREADS];  // own component's partial sums: first | count << 16
+    int b = (int)blockIdx.x, seg = 0;
+    while (seg + 1 < K && b >= all.seg[seg].W) b -= all.seg[seg++].W;  // uniform
+    const GridSeg<VT>& S = all.seg[seg];
+    const int W = S.W;
+    const GridWg g = S.wg[b];
+    int sA = __builtin_amdgcn_readfirstlane(g.sA), nS = __builtin_amdgcn_readfirstlane(g.sA + g.sP);
+    const int nR = N + S.nlds;
+    double* s_p = lds;                          // p: own nodes, then A's halo
+    double* s_r = s_p + 3 * (g.nown + g.nhA);   // r: own nodes, then P's halo
+    double* s_part = s_r + 3 * (g.nown + g.nhP);
+    VT* s_blk = reinterpret_cast<VT*>(lds + S.blk_off);  // the LDS-held blocks, [block][entry][thread]
+    int t = threadIdx.x;
+
+    // ---- the thread's blocks: values, packed columns, and the mask of blocks that end a row or the run
+    static_assert(N % 2 == 0, "blocks are taken in pairs");
+    VT v[N][9];
+    constexpr int NL = GRID_LDS_SLOTS, NC = (N + NL) / 2;  // columns of the register and LDS blocks, in pairs
+    uint32_t cp[NC];
+#pragma unroll
+    for (int s = 0; s < NC; ++s) cp[s] = 0;
+    uint32_t mask = 0, pos;  // pos: the run's first partial sum of A | of P << 16
+    {
+        const uint16_t* col = S.col + g.col_off;
+        VT* ws = S.ws + g.ws_off;
+        const int64_t th = (int64_t)b * GRID_THREADS + t;
+        const GridStart stA = S.start[2 * th], stP = S.start[2 * th + 1];
+        pos = (uint32_t)stA.pos | (uint32_t)stP.pos << 16;
+        Run R;
+        const int32_t *nptr, *rowptr;
+        const uint8_t* single;
+        const VT* vals;
+        auto open = [&](const GridStart& st, int slots, int blocks, const int32_t* np, const int32_t* rp,
+                        const uint8_t* dg, const VT* va) INLINE {
+            nptr = np;
+            rowptr = rp;
+            single = dg;
+            vals = va;
+            R.node = st.node;
+            R.j = st.j;
+            R.left = min(slots, max(0, blocks - t * slots));
+            R.k = 0;
+            if (R.left > 0) {
+                R.k = nptr[R.node + 1] - nptr[R.node];
+                R.base = rowptr[3 * (int64_t)R.node];
+            }
+        };
+        // the run's next block into u[9] (zeros past its end); true where it ends a row or the run
+        auto next = [&](VT* u) INLINE -> bool {
+            if (R.left <= 0) {
+#pragma unroll
+                for (int c = 0; c < 9; ++c) u[c] = VT(0);
+                return false;
+            }
+            const VT* src = vals + R.base + 3 * R.j;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) u[3 * i + c] = src[3 * (int64_t)R.k * i + c];
+            R.left -= 1;
+            R.j += 1;
+            const bool end = R.j == R.k;
+            if (end && R.left > 0) {
+                R.j = 0;
+                do {
+                    R.node += 1;
+                    R.k = single && single[R.node] ? 0 : nptr[R.node + 1] - nptr[R.node];
+                } while (R.k == 0);
+                R.base = rowptr[3 * (int64_t)R.node];
+            }
+            return end || R.left == 0;
+        };
+        open(stA, sA, g.nbA, S.jnptr, S.jrowptr, nullptr, S.A);
+        unrolled<N>([&](auto I) INLINE {
+            constexpr int s = I;
+            if (s < nS) {
+                if (s == sA) open(stP, g.sP, g.nbP, S.pnptr, S.prowptr, S.pdiag, S.P);
+                if (next(v[s])) mask |= 1u << s;
+                cp[s / 2] |= (uint32_t)col[s * GRID_THREADS + t] << (16 * (s & 1));
+            } else {
+#pragma unroll
+                for (int c = 0; c < 9; ++c) v[s][c] = VT(0);
+            }
+        });
+        for (int s = N; s < nS; ++s) {
+            if (s == sA) open(stP, g.sP, g.nbP, S.pnptr, S.prowptr, S.pdiag, S.P);
+            VT u[9];
+            if (next(u)) mask |= 1u << s;
+            VT* dst = s < nR ? s_blk + (s - N) * 9 * GRID_THREADS : ws + (int64_t)(s - nR) * 9 * GRID_THREADS;
+#pragma unroll
+            for (int c = 0; c < 9; ++c) dst[c * GRID_THREADS + t] = u[c];
+        }
+        unrolled<NL>([&](auto I) INLINE {
+            constexpr int s = N + I;
+            if (s < nR && s < nS) cp[s / 2] |= (uint32_t)col[s * GRID_THREADS + t] << (16 * (s & 1));
+        });
+    }
+    // ---- own component: the partial sums of its rows, the entry of a diagonal row of the preconditioner
+    constexpr uint32_t DIAG = 0xffffffffu;
+    if (t < 3 * g.nown) {
+        const uint16_t* rp = S.rp + g.rp_off + t / 3;
+        s_rows[0][t] = (uint32_t)rp[0] | (uint32_t)(rp[1] - rp[0]) << 16;
+        s_rows[1][t] = (uint32_t)rp[g.nown + 1] | (uint32_t)(rp[g.nown + 2] - rp[g.nown + 1]) << 16;
+        const int64_t node = g.node0 + t / 3;
+        const int64_t dof = 3 * (int64_t)g.node0 + t;
+        if (S.dinv) {
+            s_rows[1][t] = DIAG;
+            s_d[t] = S.dinv[dof];
+        } else if (S.pdiag[node]) {
+            s_rows[1][t] = DIAG;
+            s_d[t] = (double)S.P[S.prowptr[3 * node + t % 3]];
+        }
+        s_x[t] = S.x[dof];
+    }
+    if (t == 0) s_bad = 0;
+
+    // s_part <- partial row sums of the blocks [s0, s1) times the vector sx
+    auto products = [&](int s0, int s1, const double* sx, int at) INLINE {
+        VT y0 = VT(0), y1 = VT(0), y2 = VT(0);
+        auto flush = [&](int s) INLINE {
+            if ((mask >> s) & 1u) {
+                double* d = s_part + 3 * at;
+                d[0] = (double)y0;
+                d[1] = (double)y1;
+                d[2] = (double)y2;
+                ++at;
+                y0 = y1 = y2 = VT(0);
+            }
+        };
+        auto add = [&](const VT* u, VT c0, VT c1, VT c2) INLINE {
+            y0 = fmav(u[2], c2, fmav(u[1], c1, fmav(u[0], c0, y0)));
+            y1 = fmav(u[5], c2, fmav(u[4], c1, fmav(u[3], c0, y1)));
+            y2 = fmav(u[8], c2, fmav(u[7], c1, fmav(u[6], c0, y2)));
+        };
+        unrolled<N / 2>([&](auto I) INLINE {
+            constexpr int s = 2 * I;
+            if (s + 2 <= s0 || s >= s1) return;  // uniform
+            const double* xa = sx + (cp[s / 2] & 0xffffu);
+            const double* xb = sx + (cp[s / 2] >> 16);
+            const bool ina = s >= s0, inb = s + 1 < s1;
+            // a slot of the other phase may hold a column past this phase's vector: read entry 0 instead
+            if (!ina) xa = sx;
+            if (!inb) xb = sx;
+            const VT c0 = VT(xa[0]), c1 = VT(xa[1]), c2 = VT(xa[2]);
+            const VT e0 = VT(xb[0]), e1 = VT(xb[1]), e2 = VT(xb[2]);
+            if (ina) {
+                add(v[s], c0, c1, c2);
+                flush(s);
+            }
+            if (inb) {
+                add(v[s + 1], e0, e1, e2);
+                flush(s + 1);
+            }
+        });
+        unrolled<NL>([&](auto I) INLINE {
+            constexpr int s = N + I;
+            if (s < s0 || s >= s1 || s >= nR) return;  // uniform
+            const double* xx = sx + (s & 1 ? cp[s / 2] >> 16 : cp[s / 2] & 0xffffu);
+            VT u[9];
+#pragma unroll
+            for (int c = 0; c < 9; ++c) u[c] = s_blk[(I * 9 + c) * GRID_THREADS + t];
+            add(u, VT(xx[0]), VT(xx[1]), VT(xx[2]));
+            flush(s);
+        });
+        if (s1 > nR) {
+            const uint16_t* col = S.col + g.col_off;
+            const VT* ws = S.ws + g.ws_off;
+            for (int s = max(nR, s0); s < s1; ++s) {
+                const double* xx = sx + col[s * GRID_THREADS + t];
+                VT u[9];
+#pragma unroll
+                for (int c = 0; c < 9; ++c) u[c] = ws[((s - nR) * 9 + c) * GRID_THREADS + t];
+                add(u, VT(xx[0]), VT(xx[1]), VT(xx[2]));
+                flush(s);
+            }
+        }
+    };
+    // the own component's row sum: its partials in order, eight in flight (reads past them stay in s_part,
+    // which has GRID_SPARE entries more)
+    auto row_sum = [&](uint32_t rows) INLINE {
+        const double* d = s_part + 3 * (rows & 0xffffu) + t % 3;
+        double s = 0.0;
+        for (int n = (int)(rows >> 16); n > 0; n -= 8, d += 24) {
+            double e[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) e[i] = d[3 * i];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s += i < n ? e[i] : 0.0;
+        }
+        return s;
+    };
+    uint32_t phase = S.phase;
+    constexpr int H = 4;  // halo entries of a thread taken in during the exchange
+    double hq[H];
+    // Publishes the own components (val; sets of the phase), the work-group's sums v0 (and v1), and takes in
+    // the totals over all work-groups and the thread's first H halo components of off[0..n). False if
+    // a value did not arrive in time. Begins with all stores of the previous phase complete and ends
+    // with a barrier.
+    auto exchange = [&](double val, double v0, double v1, int nv, const int32_t* off, int n, double& t0,
+                        double& t1) INLINE -> bool {
+        double* vec = S.vec + (int64_t)(phase & 3u) * S.ndof;
+        {
+            double* clean = S.vec + (int64_t)((phase + 2) & 3u) * S.ndof;
+            const uint32_t dof = 3 * (uint32_t)g.node0 + t;
+            if (t < 3 * g.nown) {
+                agent_store(vec + dof, val);
+                agent_store(clean + dof, __longlong_as_double((long long)GRID_EMPTY));
+            }
+            if (t < 2 * GRID_COPIES)
+                agent_store((double*)&S.slots[(((phase + 2) & 3u) * 2 * GRID_COPIES + t) * W + b],
+                            __longlong_as_double((long long)GRID_EMPTY));
+        }
+        const int wid = t >> 6, lane = t & 63;
+        v0 = wave_total(v0);
+        if (nv > 1) v1 = wave_total(v1);
+        if (lane == 0) {
+            s_w[wid][0] = v0;
+            s_w[wid][1] = v1;
+        }
+        lds_barrier();
+        bool missing = true;
+        if (wid < nv) {  // wave w: value w
+            unsigned long long* sl = S.slots + ((phase & 3u) * 2 + wid) * GRID_COPIES * W;
+            double s = 0.0;
+#pragma unroll
+            for (int w = 0; w < GRID_WAVES; ++w) s += s_w[w][wid];
+            if (lane < GRID_COPIES) agent_store((double*)&sl[lane * W + b], s);
+            sl += (b % GRID_COPIES) * W;
+            double got[GRID_MAX_WG / 64];
+            for (int i = 0; missing && i < GRID_POLL_LIMIT; ++i) {
+                missing = false;
+#pragma unroll
+                for (int q = 0; q < GRID_MAX_WG / 64; ++q) {
+                    const int w = lane + 64 * q;
+                    got[q] = 0.0;
+                    if (w < W) got[q] = agent_load((const double*)&sl[w]);
+                }
+#pragma unroll
+                for (int q = 0; q < GRID_MAX_WG / 64; ++q) missing |= is_empty(got[q]);
+                missing = __any(missing);
+            }
+            s = 0.0;
+#pragma unroll
+            for (int q = 0; q < GRID_MAX_WG / 64; ++q) s += got[q];
+            s = wave_total(s);
+            if (lane == 0) {
+                s_tot[wid] = s;
+                if (missing) s_bad = 1;
+            }
+        }
+        missing = true;
+        for (int i = 0; missing && i < GRID_POLL_LIMIT; ++i) {
+            missing = false;
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                const int j = t + h * GRID_THREADS;
+                if (j < n) hq[h] = agent_load(vec + off[j]);
+            }
+#pragma unroll
+            for (int h = 0; h < H; ++h) missing |= t + h * GRID_THREADS < n && is_empty(hq[h]);
+        }
+        if (missing) s_bad = 1;
+        lds_barrier();
+        t0 = s_tot[0];
+        t1 = s_tot[1];
+        ++phase;
+        return s_bad == 0;
+    };
+    // dst[j] <- fn(dst[j], halo component j): the first H of a thread from hq, the others from the phase's vector
+    auto take = [&](double* dst, const int32_t* off, int n, auto fn) INLINE {
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            const int j = t + h * GRID_THREADS;
+            if (j < n) dst[j] = fn(dst[j], hq[h]);
+        }
+        const double* vec = S.vec + (int64_t)((phase - 1) & 3u) * S.ndof;
+        for (int j = t + H * GRID_THREADS; j < n; j += GRID_THREADS) {
+            double q = agent_load(vec + off[j]);
+            for (int i = 0; is_empty(q) && i < GRID_POLL_LIMIT; ++i) q = agent_load(vec + off[j]);
+            if (is_empty(q)) s_bad = 1;
+            dst[j] = fn(dst[j], q);
+        }
+    };
+    const int32_t* haloA = S.halo + g.halo_off;
+    const int32_t* haloP = haloA + 3 * g.nhA;
+    double* hp = s_p + 3 * g.nown;
+    double* hr = s_r + 3 * g.nown;
+    int status = GRID_RUNNING;
+    bool alive = true;
+    double zTr = 0.0, rr = 0.0, zprev = 1.0, bnorm = 0.0;
+    int64_t k = 0;
+    bool first = !S.resume;  // the preamble: r = b - A x, z = P r, by the loop's own products and exchanges
+    {
+        const int64_t dof = 3 * (int64_t)g.node0 + t;
+        if (first) {
+            if (t < 3 * g.nown) s_p[t] = s_x[t];
+            for (int j = t; j < 3 * g.nhA; j += GRID_THREADS) hp[j] = S.x[haloA[j]];
+        } else {
+            const GridState st = *S.state;
+            zTr = st.zTr;
+            rr = st.rr;
+            zprev = st.zprev;
+            bnorm = st.bnorm;
+            k = st.k;
+            // p <- z + beta p is the loop's first update: its halo z by way of hq and, past H, of p itself
+            const double beta = k == 0 ? 0.0 : zTr / zprev;
+            const double *zs = S.save, *rs = zs + S.ndof, *ps = rs + S.ndof;
+            for (int j = t; j < 3 * g.nhA; j += GRID_THREADS) hp[j] = fmav(beta, ps[haloA[j]], zs[haloA[j]]);
+            for (int j = t; j < 3 * g.nhP; j += GRID_THREADS) hr[j] = rs[haloP[j]];
+            if (t < 3 * g.nown) {
+                s_r[t] = rs[dof];
+                s_p[t] = ps[dof];
+                s_v[t] = zs[dof];
+            }
+        }
+    }
+    bool resumed = !first;
+    const int64_t k_end = k + S.chunk;
+    // What is formed from these (LDS addresses, tests of the mask's bits) is formed where it is used, not kept in
+    // registers over the loop, which the blocks fill
+    auto opaque = [&]() INLINE {
+        asm volatile("" : "+v"(t), "+v"(mask), "+v"(pos), "+s"(sA), "+s"(nS));
+#pragma unroll
+        for (int s = 0; s < NC; ++s) asm volatile("" : "+v"(cp[s]));
+    };
+    while (true) {
+        opaque();
+        const bool own = t < 3 * g.nown;
+        if (!first) {
+            // the stopping tests on r_k
+            if (bnorm == 0.0)
+                status = GRID_ZERO_RHS;
+            else if (sqrt(rr) <= S.tol * bnorm)
+                status = GRID_CONVERGED;
+            else if (S.max_iter >= 0 && k >= S.max_iter)
+                status = HOEFEM_ERROR_CG_MAX_ITERATIONS;
+            if (status != GRID_RUNNING || (k == k_end && !resumed)) break;
+            const double beta = k == 0 ? 0.0 : zTr / zprev;
+            if (!resumed) take(hp, haloA, 3 * g.nhA, [&](double d, double q) INLINE { return fmav(beta, d, q); });
+            if (own) s_p[t] = fmav(beta, s_p[t], s_v[t]);
+            resumed = false;
+        }
+        lds_barrier();
+        products(0, sA, s_p, pos & 0xffffu);
+        lds_barrier();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the previous phase's stores
+        double ap = 0.0, v0 = 0.0, v1 = 0.0, pAp, none;
+        if (own) {
+            ap = row_sum(s_rows[0][t]);
+            v0 = s_p[t] * ap;
+            if (first) {
+                const double rhs = S.b[3 * (uint32_t)g.node0 + t];
+                ap = rhs - ap;
+                s_r[t] = ap;
+                v0 = rhs * rhs;
+            }
+            s_v[t] = ap;
+        }
+        alive = exchange(ap, v0, 0.0, 1, haloP, 3 * g.nhP, pAp, none);
+        if (!alive) break;
+        if (first) {
+            bnorm = sqrt(pAp);
+            take(hr, haloP, 3 * g.nhP, [](double, double q) INLINE { return q; });
+            for (int j = t; j < 3 * g.nhA; j += GRID_THREADS) hp[j] = 0.0;
+            if (own) s_p[t] = 0.0;
+        } else {
+            if (pAp <= 0.0)
+                status = HOEFEM_ERROR_CG_INDEFINITE_OPERATOR;
+            else if (zTr <= 0.0)
+                status = HOEFEM_ERROR_CG_INDEFINITE_PRECONDITIONER;
+            if (status != GRID_RUNNING) break;
+            const double alpha = zTr / pAp;
+            take(hr, haloP, 3 * g.nhP, [&](double d, double q) INLINE { return fmav(-alpha, q, d); });
+            if (own) {
+                s_x[t] = fmav(alpha, s_p[t], s_x[t]);
+                s_r[t] = fmav(-alpha, s_v[t], s_r[t]);
+            }
+            zprev = zTr;
+            ++k;
+        }
+        opaque();
+        lds_barrier();
+        products(sA, nS, s_r, pos >> 16);
+        lds_barrier();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        double z = 0.0;
+        v0 = v1 = 0.0;
+        if (own) {
+            const double r = s_r[t];
+            const uint32_t rows = s_rows[1][t];
+            if (rows != DIAG)
+                z = row_sum(rows);
+            else
+                z = S.dinv ? s_d[t] * r : (double)(VT(s_d[t]) * VT(r));
+            s_v[t] = z;
+            v0 = z * r;
+            v1 = r * r;
+        }
+        alive = exchange(z, v0, v1, 2, haloA, 3 * g.nhA, zTr, rr);
+        if (!alive) break;
+        first = false;
+    }
+    if (!alive) {  // x keeps its last saved value
+        if (t == 0) S.host->failed = 1;
+        return;
+    }
+    if (t < 3 * g.nown) {
+        const int64_t dof = 3 * (int64_t)g.node0 + t;
+        S.x[dof] = status == GRID_ZERO_RHS ? 0.0 : s_x[t];
+        if (status == GRID_RUNNING) {
+            S.save[dof] = s_v[t];
+            S.save[dof + S.ndof] = s_r[t];
+            S.save[dof + 2 * S.ndof] = s_p[t];
+        }
+    }
+    if (b == 0 && t == 0) {
+        *S.state = GridState{zTr, rr, zprev, bnorm, k};
+        S.host->iters = k;
+        S.host->phase = phase;
+        S.host->status = status;
+    }
+#undef INLINE
+}
+
+// ------------------------------------------------------------------ plan
+// W: a phase's exchange grows from 2.9 us at 8 work-groups to 5.1 us at 256 while its products shrink with
+// 1/W (about 0.13 us per block of a thread), so small systems take few work-groups: enough for
+// GRID_BLOCKS_PER_THREAD blocks per thread, at least 8, at most the CUs.
+constexpr int GRID_BLOCKS_PER_THREAD = 6;
+constexpr int GRID_MAX_SLOTS = 32;                 // bits of a thread's row-end mask
+constexpr size_t GRID_MAX_LDS = 143 * 1024;  // beside 16.3 KiB of fixed arrays
+constexpr int GRID_MAX_NODES = GRID_THREADS / 3;   // per work-group
+constexpr int GRID_SPARE = 8;                      // spare partial sums (row_sum)
+
+void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStream_t s) {
+    W = 0;
+    const int64_t nn = J.num_nodes;
+    if (nn == 0 || cus < 8) return;
+    auto ka = [&](int64_t v) { return J.nptr[v + 1] - J.nptr[v]; };
+    auto kp = [&](int64_t v) { return !P || P->diag_only[v] ? 0 : P->nptr[v + 1] - P->nptr[v]; };
+    int64_t total = 0;
+    for (int64_t v = 0; v < nn; ++v) total += ka(v) + kp(v);
+    const int wmax = std::min(cus, GRID_MAX_WG);
+    if (nn > (int64_t)wmax * GRID_MAX_NODES || total > (int64_t)wmax * GRID_THREADS * GRID_MAX_SLOTS) return;
+    int64_t w = (total + (int64_t)GRID_THREADS * GRID_BLOCKS_PER_THREAD - 1) / ((int64_t)GRID_THREADS * GRID_BLOCKS_PER_THREAD);
+    w = std::max<int64_t>(w, (nn + GRID_MAX_NODES - 1) / GRID_MAX_NODES);
+    w = std::min<int64_t>(std::max<int64_t>((w + 7) / 8 * 8, 8), wmax);
+    w = std::min(w, nn);
+    // Contiguous node ranges: the fewest blocks per thread that w ranges allow, then the evenest ranges (blocks,
+    // and a few blocks' worth per node) with that many. Both by filling range after range up to a cap.
+    std::vector<int64_t> cut;
+    auto fill = [&](int64_t slots, int64_t cap) -> bool {
+        cut.assign(1, 0);
+        int64_t a = 0, p = 0;
+        for (int64_t v = 0; v < nn; ++v) {
+            const int64_t a1 = a + ka(v), p1 = p + kp(v), n1 = v + 1 - cut.back();
+            const bool full = n1 > GRID_MAX_NODES || a1 + p1 + 4 * n1 > cap ||
+                              (a1 + GRID_THREADS - 1) / GRID_THREADS + (p1 + GRID_THREADS - 1) / GRID_THREADS > slots;
+            if (full && n1 > 1) {
+                if ((int64_t)cut.size() == w) return false;
+                cut.push_back(v);
+                a = ka(v);
+                p = kp(v);
+            } else if (full) {
+                return false;  // a node by itself is too much
+            } else {
+                a = a1;
+                p = p1;
+            }
+        }
+        cut.push_back(nn);
+        return true;
+    };
+    int64_t slots = std::max<int64_t>(1, total / (w * GRID_THREADS));
+    while (slots <= GRID_MAX_SLOTS && !fill(slots, INT64_MAX)) ++slots;
+    if (slots > GRID_MAX_SLOTS) return;
+    int64_t lo = (total + 4 * nn) / w, hi = total + 4 * nn;  // hi fits
+    while (lo < hi) {
+        const int64_t mid = lo + (hi - lo) / 2;
+        if (fill(slots, mid))
+            hi = mid;
+        else
+            lo = mid + 1;
+    }
+    fill(slots, hi);
+    w = (int64_t)cut.size() - 1;
+    std::vector<GridWg> wg(w);
+    std::vector<GridStart> start((size_t)2 * w * GRID_THREADS);
+    struct Part {  // of one work-group
+        std::vector<int32_t> halo;
+        std::vector<uint16_t> col, rp;
+        int parts = 0;
+        bool fits = true;
+    };
+    std::vector<Part> part(w);
+    auto work = [&](int64_t b0, int64_t step) {
+        std::vector<int32_t> local(nn, -1), list;
+        for (int64_t b = b0; b < w; b += step) {
+            GridWg& g = wg[b];
+            Part& o = part[b];
+            g = GridWg{};
+            const int64_t n0 = cut[b], n1 = cut[b + 1];
+            g.node0 = (int32_t)n0;
+            g.nown = (int32_t)(n1 - n0);
+            o.fits = g.nown <= GRID_MAX_NODES;
+            for (int ph = 0; ph < 2 && o.fits; ++ph) {
+                const NodePattern* pat = ph == 0 ? &J : P;
+                auto kk = [&](int64_t v) { return ph == 0 ? ka(v) : kp(v); };
+                list.clear();
+                int64_t nb = 0;
+                for (int64_t v = n0; v < n1; ++v) {
+                    const int k = kk(v);
+                    const int32_t* nc = k ? pat->ncol.data() + pat->nptr[v] : nullptr;
+                    nb += k;
+                    for (int j = 0; j < k; ++j) {
+                        const int32_t c = nc[j];
+                        if (local[c] < 0 && (c < n0 || c >= n1)) {
+                            local[c] = 0;
+                            list.push_back(c);
+                        }
+                    }
+                }
+                std::sort(list.begin(), list.end());
+                for (size_t i = 0; i < list.size(); ++i) {
+                    local[list[i]] = g.nown + (int32_t)i;
+                    for (int c = 0; c < 3; ++c) o.halo.push_back(3 * list[i] + c);
+                }
+                const int slots = (int)((nb + GRID_THREADS - 1) / GRID_THREADS);
+                o.fits = slots <= GRID_MAX_SLOTS && 3 * (g.nown + (int64_t)list.size()) <= 65535;
+                int np = 0;  // partial sums so far
+                if (o.fits) {
+                    const size_t c0 = o.col.size();
+                    o.col.resize(c0 + (size_t)slots * GRID_THREADS, 0);
+                    int th = 0, sl = 0;  // the block's thread and its place in the thread's run
+                    for (int64_t v = n0; v < n1; ++v) {
+                        o.rp.push_back((uint16_t)np);
+                        const int k = kk(v);
+                        const int32_t* nc = k ? pat->ncol.data() + pat->nptr[v] : nullptr;
+                        for (int j = 0; j < k; ++j) {
+                            if (sl == 0) start[2 * (b * GRID_THREADS + th) + ph] = GridStart{(int32_t)v, j, np, 0};
+                            const int32_t c = nc[j];
+                            const int32_t l = c >= n0 && c < n1 ? (int32_t)(c - n0) : local[c];
+                            o.col[c0 + (size_t)sl * GRID_THREADS + th] = (uint16_t)(3 * l);
+                            if (j + 1 == k || sl + 1 == slots) ++np;
+                            if (++sl == slots) {
+                                sl = 0;
+                                ++th;
+                            }
+                        }
+                    }
+                    o.rp.push_back((uint16_t)np);
+                }
+                o.parts = std::max(o.parts, np);
+                for (int32_t c : list) local[c] = -1;
+                (ph == 0 ? g.nhA : g.nhP) = (int32_t)list.size();
+                (ph == 0 ? g.sA : g.sP) = slots;
+                (ph == 0 ? g.nbA : g.nbP) = (int32_t)nb;
+            }
+        }
+    };
+    {  // large patterns on a few host threads
+        const int nt = total < 100000 ? 1 : (int)std::min<int64_t>(std::max(1u, std::thread::hardware_concurrency()), 8);
+        std::vector<std::thread> th;
+        try {
+            for (int i = 1; i < nt; ++i) th.emplace_back(work, i, nt);
+        } catch (const std::system_error&) {  // fewer threads than asked for: their shares here
+            for (int i = (int)th.size() + 1; i < nt; ++i) work(i, nt);
+        }
+        work(0, nt);
+        for (std::thread& t : th) t.join();
+    }
+    std::vector<int32_t> halo;
+    std::vector<uint16_t> col, rp;
+    size_t ws = 0;
+    lds_bytes = 0;
+    max_slots = 0;
+    for (int64_t b = 0; b < w; ++b) {
+        GridWg& g = wg[b];
+        const Part& o = part[b];
+        max_slots = std::max(max_slots, g.sA + g.sP);
+        if (!o.fits || max_slots > GRID_MAX_SLOTS) return;
+        g.halo_off = (int64_t)halo.size();
+        g.rp_off = (int64_t)rp.size();
+        g.col_off = (int64_t)col.size();
+        halo.insert(halo.end(), o.halo.begin(), o.halo.end());
+        rp.insert(rp.end(), o.rp.begin(), o.rp.end());
+        col.insert(col.end(), o.col.begin(), o.col.end());
+        lds_bytes = std::max(lds_bytes, sizeof(double) * (size_t)(3 * (2 * g.nown + g.nhA + g.nhP) + 3 * (o.parts + GRID_SPARE)));
+    }
+    if (lds_bytes > GRID_MAX_LDS) return;
+    // blocks past the registers: in the LDS that is left, then in memory (sized for FP64)
+    constexpr size_t SLOT = sizeof(double) * 9 * GRID_THREADS;
+    blk_off = (int)((lds_bytes / sizeof(double) + 1) / 2 * 2);
+    const int over = std::max(0, max_slots - GRID_REG_F64);
+    nlds = (int)std::min<size_t>((size_t)std::min(over, GRID_LDS_SLOTS), (GRID_MAX_LDS - std::min(GRID_MAX_LDS, sizeof(double) * blk_off)) / SLOT);
+    lds_bytes = sizeof(double) * blk_off + SLOT * nlds;
+    for (GridWg& g : wg) {
+        g.ws_off = (int64_t)ws;
+        ws += (size_t)std::max(0, g.sA + g.sP - GRID_REG_F64 - nlds) * 9 * GRID_THREADS;
+    }
+    d_wg.upload(wg, s);
+    d_halo.upload(halo, s);
+    d_col.upload(col, s);
+    d_rp.upload(rp, s);
+    d_start.upload(start, s);
+    d_ws.ensure(ws);
+    d_save.ensure((size_t)3 * 3 * nn);
+    d_state.ensure(1);
+    host.reset(new PinnedBuf<GridResult>(1, hipHostMallocCoherent));
+    *host->p = GridResult{};
+    ndof = 3 * nn;
+    W = (int)w;
+    reset(s);
+}
+
+// ------------------------------------------------------------------ admission
+// CUs of each device taken by resident grids in flight: a launch is admitted when its work-groups (one per
+// CU at most) fit beside those already admitted, so admitted grids are all resident and make progress.
+namespace {
+struct Slots {
+    std::mutex mu;
+    std::condition_variable cv;
+    std::map<int, std::pair<int, int>> dev;  // device -> (CUs, free)
+    std::pair<int, int>& of(int d) {
+        auto it = dev.find(d);
+        if (it == dev.end()) {
+            int n = 0;
+            HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, d));
+            it = dev.emplace(d, std::make_pair(n, n)).first;
+        }
+        return it->second;
+    }
+};
+Slots& slots() {
+    static Slots s;
+    return s;
+}
+}  // namespace
+
+int grid_device_cus() {
+    int d = 0;
+    HIP_CHECK(hipGetDevice(&d));
+    std::lock_guard<std::mutex> lock(slots().mu);
+    return slots().of(d).first;
+}
+
+int grid_free_cus() {
+    int d = 0;
+    HIP_CHECK(hipGetDevice(&d));
+    std::lock_guard<std::mutex> lock(slots().mu);
+    return slots().of(d).second;
+}
+
+bool GridSlots::acquire(int n, bool wait) {
+    release();
+    HIP_CHECK(hipGetDevice(&dev_));
+    std::unique_lock<std::mutex> lock(slots().mu);
+    auto& c = slots().of(dev_);
+    if (n > c.first) return false;
+    if (wait)
+        slots().cv.wait(lock, [&] { return c.second >= n; });
+    else if (c.second < n)
+        return false;
+    c.second -= n;
+    n_ = n;
+    return true;
+}
+
+void GridSlots::release() {
+    if (!n_) return;
+    {
+        std::lock_guard<std::mutex> lock(slots().mu);
+        slots().dev[dev_].second += n_;
+    }
+    n_ = 0;
+    slots().cv.notify_all();
+}
+
+// ------------------------------------------------------------------ launches
+template <class VT>
+GridSeg<VT> grid_segment(const GridPlan& g, Model& m, const VT* A, const Schwarz* P, const double* dinv,
+                         const double* b, double* x, double tol, int64_t max_iter) {
+    GridSeg<VT> S{};
+    S.wg = g.d_wg.get();
+    S.halo = g.d_halo.get();
+    S.col = g.d_col.get();
+    S.rp = g.d_rp.get();
+    S.start = g.d_start.get();
+    S.jnptr = m.pattern.d_nptr.get();
+    S.jrowptr = m.pattern.d_rowptr.get();
+    S.A = A;
+    if (P) {
+        S.pnptr = P->P.d_nptr.get();
+        S.prowptr = P->P.d_rowptr.get();
+        S.pdiag = P->P.d_diag_only.get();
+        if constexpr (sizeof(VT) == sizeof(double))
+            S.P = P->d_vals.get();
+        else
+            S.P = P->d_vals32.get();
+    } else {
+        S.dinv = dinv;
+    }
+    S.b = b;
+    S.x = x;
+    S.vec = reinterpret_cast<double*>(g.d_slots.get() + (size_t)8 * GRID_COPIES * g.W);
+    S.save = g.d_save.get();
+    S.ndof = g.ndof;
+    S.ws = reinterpret_cast<VT*>(g.d_ws.get());
+    S.slots = g.d_slots.get();
+    S.state = g.d_state.get();
+    S.host = g.host->p;
+    S.W = g.W;
+    S.phase = g.phase;
+    S.nlds = g.nlds;
+    S.blk_off = g.blk_off;
+    S.tol = tol;
+    S.max_iter = max_iter;
+    return S;
+}
+template GridSeg<double> grid_segment<double>(const GridPlan&, Model&, const double*, const Schwarz*, const double*,
+                                              const double*, double*, double, int64_t);
+template GridSeg<float> grid_segment<float>(const GridPlan&, Model&, const float*, const Schwarz*, const double*,
+                                            const double*, double*, double, int64_t);
+
+template <class VT>
+constexpr int grid_reg() {
+    return sizeof(VT) == sizeof(double) ? GRID_REG_F64 : GRID_REG_F32;
+}
+
+template <class VT, int K>
+void grid_launch(const GridSegs<VT, K>& all, int wgs, size_t lds, hipStream_t s) {
+    auto* k = &k_grid_pcg<VT, grid_reg<VT>(), K>;
+    raise_lds_limit((const void*)k, lds);
+    k<<<dim3((unsigned)wgs), dim3(GRID_THREADS), lds, s>>>(all);
+    check_launch("k_grid_pcg");
+}
+template void grid_launch<double, GRID_SEGS>(const GridSegs<double, GRID_SEGS>&, int, size_t, hipStream_t);
+template void grid_launch<float, GRID_SEGS>(const GridSegs<float, GRID_SEGS>&, int, size_t, hipStream_t);
+
+template <class VT>
+bool grid_solve(GridPlan& g, Model& m, const VT* A, const Schwarz* P, const double* dinv, const double* b, double* x,
+                double tol, int64_t max_iter, int64_t* iterations, hoefem_status* status) {
+    GridSegs<VT, 1> all;
+    GridSeg<VT>& S = all.seg[0];
+    S = grid_segment<VT>(g, m, A, P, dinv, b, x, tol, max_iter);
+    S.chunk = GRID_CHUNK;
+    while (true) {
+        volatile GridResult* h = g.host->p;
+        h->status = GRID_RUNNING;
+        h->failed = 0;
+        {
+            GridSlots slots;
+            if (!slots.acquire(g.W, true)) return false;
+            grid_launch(all, g.W, g.lds_bytes, m.stream);
+            HIP_CHECK(hipStreamSynchronize(m.stream));
+        }
+        if (h->failed) {
+            g.reset(m.stream);
+            return false;
+        }
+        g.phase = S.phase = h->phase;
+        *iterations = h->iters;
+        if (h->status != GRID_RUNNING) break;
+        S.resume = 1;
+    }
+    const int st = g.host->p->status;
+    *status = st == GRID_CONVERGED || st == GRID_ZERO_RHS ? HOEFEM_OK : (hoefem_status)st;
+    return true;
+}
+template bool grid_solve<double>(GridPlan&, Model&, const double*, const Schwarz*, const double*, const double*,
+                                 double*, double, int64_t, int64_t*, hoefem_status*);
+template bool grid_solve<float>(GridPlan&, Model&, const float*, const Schwarz*, const double*, const double*,
+                                double*, double, int64_t, int64_t*, hoefem_status*);
+
+// ------------------------------------------------------------------ many systems
+GridBatch::~GridBatch() {
+    for (Lane& l : lanes) {
+        if (l.s) (void)hipStreamSynchronize(l.s);
+        if (l.done) (void)hipEventDestroy(l.done);
+        if (l.s) (void)hipStreamDestroy(l.s);
+    }
+}
+
+namespace {
+// The resident-grid solves of a batch. Waiting systems are launched together, in the order they came, as far
+// as their work-groups fit the free CUs, for GRID_BATCH_CHUNK iterations (so that CUs of systems that end
+// soon come free); launches go to a few lanes (streams), so systems that come later run beside the earlier
+// ones. A system that is not done goes on in a later launch; its arithmetic does not depend on where its launches
+// are cut, so x, iteration count and status equal a solve by itself bit for bit.
+template <class VT>
+struct GridPoolT final : CgPool {
+    struct Item {
+        CgBatchSystem q;
+        GridPlan* g;
+        GridSeg<VT> seg;
+    };
+    GridBatch& B;
+    std::vector<Item> items;
+    std::vector<int> waiting;
+    GridSlots slots[GRID_LANES];
+    std::vector<int> running[GRID_LANES];
+
+    explicit GridPoolT(GridBatch& b) : B(b) {
+        for (GridBatch::Lane& l : B.lanes)
+            if (!l.s) {
+                HIP_CHECK(hipStreamCreateWithFlags(&l.s, hipStreamNonBlocking));
+                HIP_CHECK(hipEventCreateWithFlags(&l.done, hipEventDisableTiming));
+            }
+    }
+    ~GridPoolT() override {
+        for (int l = 0; l < GRID_LANES; ++l)
+            if (!running[l].empty()) (void)hipStreamSynchronize(B.lanes[l].s);
+    }
+    int join(const CgBatchSystem& q) override {
+        Item it{q, q.P ? &q.P->grid : &q.m->grid, {}};
+        it.q.iterations = 0;
+        it.q.status = HOEFEM_OK;
+        it.seg = grid_segment<VT>(*it.g, *q.m, (const VT*)q.A, q.P, q.P ? nullptr : q.w->diag_inv.get(), q.b, q.x, q.tol,
+                                  q.max_iter);
+        it.seg.chunk = GRID_BATCH_CHUNK;
+        items.push_back(it);
+        waiting.push_back((int)items.size() - 1);
+        return (int)items.size() - 1;
+    }
+    const CgBatchSystem& system(int id) const override { return items[id].q; }
+    bool idle() const override {
+        for (const auto& r : running)
+            if (!r.empty()) return false;
+        return waiting.empty();
+    }
+    void ended_launch(int lane, std::vector<int>& ended) {
+        slots[lane].release();
+        std::vector<int> again;
+        for (int id : running[lane]) {
+            Item& it = items[id];
+            volatile GridResult* h = it.g->host->p;
+            if (h->failed) {  // solved from the start by the two kernels
+                it.g->reset(B.lanes[lane].s);
+                HIP_CHECK(hipMemsetAsync(it.q.x, 0, sizeof(double) * it.g->ndof, it.q.m->stream));
+                it.q.w->use_grid = false;
+                it.q.status = pcg_solve(*it.q.m, *it.q.w, (const VT*)it.q.A, it.q.P, it.q.b, it.q.x, it.q.tol,
+                                        it.q.max_iter, &it.q.iterations);
+                it.q.w->use_grid = true;
+                HIP_CHECK(hipStreamSynchronize(it.q.m->stream));
+                ended.push_back(id);
+                continue;
+            }
+            it.g->phase = it.seg.phase = h->phase;
+            if (h->status == GRID_RUNNING) {
+                it.seg.resume = 1;
+                again.push_back(id);
+                continue;
+            }
+            it.q.iterations = h->iters;
+            it.q.status = h->status == GRID_CONVERGED || h->status == GRID_ZERO_RHS ? HOEFEM_OK : (hoefem_status)h->status;
+            ended.push_back(id);
+        }
+        running[lane].clear();
+        waiting.insert(waiting.begin(), again.begin(), again.end());
+    }
+    void progress(std::vector<int>& ended) override {
+        for (int l = 0; l < GRID_LANES; ++l)
+            if (!running[l].empty()) {
+                const hipError_t e = hipEventQuery(B.lanes[l].done);
+                if (e == hipErrorNotReady) continue;
+                HIP_CHECK(e);
+                ended_launch(l, ended);
+            }
+        for (int l = 0; l < GRID_LANES && !waiting.empty(); ++l) {
+            if (!running[l].empty()) continue;
+            // as many waiting systems as fit, at least the first
+            int wgs = 0, n = 0;
+            const int cus = grid_free_cus();
+            while (n < (int)waiting.size() && n < GRID_SEGS && wgs + items[waiting[n]].g->W <= cus)
+                wgs += items[waiting[n++]].g->W;
+            if (n == 0 || !slots[l].acquire(wgs, false)) break;
+            GridSegs<VT, GRID_SEGS> all{};
+            size_t lds = 0;
+            const hipStream_t s = B.lanes[l].s;
+            for (int k = 0; k < n; ++k) {
+                Item& it = items[waiting[k]];
+                volatile GridResult* h = it.g->host->p;
+                h->status = GRID_RUNNING;
+                h->failed = 0;
+                if (!it.seg.resume) HIP_CHECK(hipMemsetAsync(it.q.x, 0, sizeof(double) * it.g->ndof, s));
+                it.seg.phase = it.g->phase;
+                all.seg[k] = it.seg;
+                lds = std::max(lds, it.g->lds_bytes);
+                running[l].push_back(waiting[k]);
+            }
+            waiting.erase(waiting.begin(), waiting.begin() + n);
+            grid_launch(all, wgs, lds, s);
+            HIP_CHECK(hipEventRecord(B.lanes[l].done, s));
+        }
+    }
+};
+}  // namespace
+
+std::unique_ptr<CgPool> make_grid_pool(GridBatch& B, bool fp32) {
+    if (fp32) return std::unique_ptr<CgPool>(new GridPoolT<float>(B));
+    return std::unique_ptr<CgPool>(new GridPoolT<double>(B));
+}
+
+__global__ void k_grid_clear(int64_t n, unsigned long long* __restrict__ p) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = GRID_EMPTY;
+}
+
+void GridPlan::reset(hipStream_t s) {
+    const int64_t n = (int64_t)8 * GRID_COPIES * W + 4 * ndof;
+    d_slots.ensure((size_t)n);
+    k_grid_clear<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(n, d_slots.get());
+    check_launch("k_grid_clear");
+    phase = 0;
+}
+
+}  // namespace hoefem

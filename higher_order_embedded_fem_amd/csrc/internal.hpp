@@ -166,6 +166,50 @@ struct KernelProf {
     ~KernelProf();
 };
 
+// ------------------------------------------------------------------ resident-grid PCG (grid_pcg.hip)
+// One work-group's share of a system: a contiguous range of nodes with their rows of A and P.
+struct GridWg {
+    int32_t node0, nown;
+    int32_t nhA, nhP;            // halo nodes of its rows of A and of P
+    int32_t sA, sP;              // blocks of A and of P per thread
+    int32_t nbA, nbP;            // blocks of A and of P
+    int64_t halo_off;            // vector offsets of the halo components (A's, then P's)
+    int64_t col_off;             // local column offsets, [block of a thread][thread]
+    int64_t rp_off;              // partial-sum ranges of the rows (nown + 1 for A, nown + 1 for P)
+    int64_t ws_off;              // its blocks past the register-held ones
+};
+struct GridStart {               // first block of a thread's run and its first partial sum
+    int32_t node, j, pos, pad;
+};
+struct GridState {               // iteration state between launches
+    double zTr, rr, zprev, bnorm;
+    int64_t k;
+};
+struct GridResult {              // pinned: written by the kernel
+    int32_t status, failed;
+    uint32_t phase, pad;
+    int64_t iters;
+};
+// How a matrix pattern (and its preconditioner's) is split over the grid, with the buffers of a solve.
+// W == 0: the system does not fit and takes the two-kernel path.
+struct GridPlan {
+    int W = 0, max_slots = 0, nlds = 0, blk_off = 0;
+    uint32_t phase = 0;
+    int64_t ndof = 0;
+    size_t lds_bytes = 0;
+    DevBuf<GridWg> d_wg;
+    DevBuf<int32_t> d_halo;
+    DevBuf<uint16_t> d_col, d_rp;
+    DevBuf<GridStart> d_start;
+    DevBuf<double> d_ws, d_save;
+    DevBuf<unsigned long long> d_slots;  // partial sums, then the exchanged vectors (four sets each)
+    DevBuf<GridState> d_state;
+    std::unique_ptr<PinnedBuf<GridResult>> host;
+    void build(const NodePattern& J, const NodePattern* P, int cus, hipStream_t s);
+    void reset(hipStream_t s);  // after a failed launch
+};
+int grid_device_cus();
+
 // ------------------------------------------------------------------ model
 struct DeviceQuadrature {
     DevBuf<int32_t> off;  // [E + 1]
@@ -182,6 +226,7 @@ struct Model {
     std::vector<std::vector<int32_t>> colors[2];  // pass -> color -> element ids
     NodePattern pattern;
     BlockScatter scatter;                         // element blocks -> pattern, color order
+    GridPlan grid;                                // resident-grid solves with the Jacobi preconditioner
     double mass_reg = 0.0;
     int material = 0;                 // dev::MAT_* (elastic model wrapping Stable Neo-Hookean)
     double inversion_threshold = 0.0; // InvertibleMaterial threshold
@@ -219,6 +264,7 @@ struct Schwarz {
     std::vector<int32_t> nodes, untreated;
     std::vector<std::vector<int32_t>> colors;
     NodePattern P;
+    GridPlan grid;                 // resident-grid solves of the model's matrix with this preconditioner
     BlockScatter scatter;          // blocks -> P pattern
     std::vector<int32_t> jslot;    // per block entry (a, c): local index of node c in J's nbr(node a)
     DevBuf<int32_t> d_jslot, d_untreated, d_nodes;
@@ -265,6 +311,7 @@ struct CgWork {
     hipGraphExec_t batch_exec = nullptr;
     std::vector<const void*> batch_key;
     bool use_graphs = true;
+    bool use_grid = true;  // the resident grid where the system fits it (grid_pcg.hip)
     PinnedBuf<CgScalars> h_scalars{3};  // final readback (slot 2)
     PinnedBuf<int> h_status{1, hipHostMallocCoherent};  // the solve's status, written by the kernel that ends it
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -392,6 +439,20 @@ struct CgPool {
     virtual bool idle() const = 0;
 };
 std::unique_ptr<CgPool> make_cg_pool(CgBatch& B, bool fp32, int capacity);
+// The same for systems that fit the resident grid (grid_pcg.hip): streams of its launches
+constexpr int GRID_LANES = 3;
+struct GridBatch {
+    struct Lane {
+        hipStream_t s = nullptr;
+        hipEvent_t done = nullptr;
+    };
+    Lane lanes[GRID_LANES];
+    GridBatch() = default;
+    GridBatch(const GridBatch&) = delete;
+    GridBatch& operator=(const GridBatch&) = delete;
+    ~GridBatch();
+};
+std::unique_ptr<CgPool> make_grid_pool(GridBatch& B, bool fp32);
 // the Jacobi diagonal of A into w.diag_inv on the model stream (zero diagonal entries flagged in m.d_err)
 void launch_jacobi_diag(Model& m, CgWork& w, const void* A, bool fp32);
 

@@ -61,6 +61,7 @@ void schwarz_setup(Schwarz& s, Model& m, int64_t nsub, const int64_t* off, const
         if (v < 0 || v >= m.nv || !s.P.diag_only[v])
             throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "untreated node must not belong to a subdomain");
     s.P.upload(m.stream);
+    s.grid.build(m.pattern, &s.P, grid_device_cus(), m.stream);
     s.scatter.upload(m.stream);
     s.d_jslot.upload(s.jslot, m.stream);
     s.d_untreated.upload(s.untreated, m.stream);

@@ -1,5 +1,6 @@
-// Preconditioned conjugate gradient (fenris/src/cg.rs:377-482) as two fused kernels per
-// iteration, with the iteration state (zTr, alpha, beta, status) kept on the device:
+// Preconditioned conjugate gradient (fenris/src/cg.rs:377-482). Systems that fit the chip's registers and LDS
+// run as one resident grid (grid_pcg.hip); the others, the learned correction, harvesting and timed solves
+// as two fused kernels per iteration, with the iteration state (zTr, alpha, beta, status) kept on the device:
 //   A-kernel: [sum zTr, |r|^2 of the previous B-kernel; convergence / max-iteration status;
 //             beta] p <- z + beta p (on the fly, double-buffered), Ap = A p, partial pAp
 //   B-kernel: [sum pAp; indefiniteness status; alpha] x += alpha p, r <- r - alpha Ap
@@ -18,7 +19,7 @@
 
 #include <hip/hip_ext.h>
 
-#include "internal.hpp"
+#include "grid_pcg.hpp"
 
 namespace hoefem {
 
@@ -1195,6 +1196,12 @@ static hoefem_status pcg_solve_t(Model& m, CgWork& w, const VT* Avals, const VT*
     if (FLEX && JAC) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "the learned correction needs the Schwarz preconditioner");
     if (FLEX && (lv->na < 1 || lv->na > CG_MAX_BLOCKS))
         throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "number of aggregates out of range");
+    // the resident grid takes every plain solve that fits it; per-iteration hooks (kernel timing, snapshots)
+    // and the flexible variant keep the two kernels
+    GridPlan& grid = Pre ? Pre->grid : m.grid;
+    if (grid.W && !FLEX && !h && !m.prof && w.use_grid &&
+        grid_solve<VT>(grid, m, Avals, Pre, Pre ? nullptr : w.diag_inv.get(), b, x, tol, max_iter, iterations, &st))
+        return st;
 #define CG_CASE(ga, gb, j, f)                                                                            \
     if (GA == ga && GB == gb && JAC == j && FLEX == f) {                                                 \
         cg_launch_all<ga, gb, j, f, VT>(m, w, A, Pm, b, x, tol, max_iter, iterations, &st, h, lv);        \
@@ -1336,6 +1343,10 @@ hoefem_status pcg_solve_noalloc(Model& m, const double* Avals, Schwarz* Pre, con
         check_launch("k_jacobi_diag");
         if (read_and_clear_err(m) & KERR_ZERO_DIAG) throw Error(HOEFEM_ERROR_SINGULAR, "Diagonal matrix is not invertible.");
     }
+    GridPlan& grid = Pre ? Pre->grid : m.grid;
+    hoefem_status st = HOEFEM_OK;
+    if (grid.W && grid_solve<double>(grid, m, Avals, Pre, Pre ? nullptr : base + NA_DIAG, b, x, tol, max_iter, iterations, &st))
+        return st;
 #define NA_CASE(ga, gb, j) \
     if (GA == ga && GB == gb && (Pre == nullptr) == j) return cg_launch_noalloc<ga, gb, j>(m, base, A, Pm, b, x, tol, max_iter, iterations);
     NA_CASE(8, 8, true) NA_CASE(16, 8, true) NA_CASE(32, 8, true)
