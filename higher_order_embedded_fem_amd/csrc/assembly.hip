@@ -817,28 +817,49 @@ __global__ void k_dirichlet_rows(const int32_t* __restrict__ bc_nodes, int64_t n
 }
 
 // ------------------------------------------------------------------ material (batched)
-__global__ void k_material(int mat, double thr, double mu, double lambda, int64_t nq, const double* __restrict__ F,
-                           double* __restrict__ P, double* __restrict__ dP, int* err) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nq) return;
+// One lane per deformation gradient, MT_PTS of them per work-group. A lane's 9 or 81 values are contiguous in
+// memory, so lanes accessing them directly are 72 or 648 bytes apart and every store instruction touches 64
+// lines; F, P and dP/dF pass through LDS instead, where a lane's odd stride is free of bank conflicts, and
+// move to and from memory as the contiguous runs they are. 200,003 points (158 MB): 151 us with direct
+// accesses; this takes 47 us. With stress alone the LDS holds 9 values per
+// point, with the tangent 81 (41 KB per 64 points: three work-groups per CU).
+constexpr int MT_PTS = 64;
+template <int MAT>
+__global__ __launch_bounds__(MT_PTS) void k_material(double thr, double mu, double lambda, int64_t nq,
+                                                     const double* __restrict__ F, double* __restrict__ P,
+                                                     double* __restrict__ dP, int* err) {
+    extern __shared__ double s_m[];  // MT_PTS x 81 (or x 9 without dP)
+    const int64_t q0 = (int64_t)blockIdx.x * MT_PTS;
+    const int t = threadIdx.x, n = (int)(nq - q0 < MT_PTS ? nq - q0 : MT_PTS);
+    for (int i = t; i < 9 * n; i += MT_PTS) s_m[i] = F[9 * q0 + i];
+    __syncthreads();
     double f[9];
-    for (int k = 0; k < 9; ++k) f[k] = F[9 * q + k];
+    if (t < n)
+        for (int k = 0; k < 9; ++k) f[k] = s_m[9 * t + k];
+    __syncthreads();
+    bool ok = true;
     if (P) {
-        double p[9];
-        if (!material_stress(mat, thr, mu, lambda, f, p)) {
-            atomicOr(err, KERR_SINGULAR);
-            for (int k = 0; k < 9; ++k) p[k] = 0.0;
+        if (t < n) {
+            double p[9];
+            ok = material_stress(MAT, thr, mu, lambda, f, p);
+            for (int k = 0; k < 9; ++k) s_m[9 * t + k] = ok ? p[k] : 0.0;
         }
-        for (int k = 0; k < 9; ++k) P[9 * q + k] = p[k];
+        __syncthreads();
+        for (int i = t; i < 9 * n; i += MT_PTS) P[9 * q0 + i] = s_m[i];
+        __syncthreads();
     }
     if (dP) {
-        double d[81];
-        if (!material_dpdf(mat, thr, mu, lambda, f, d)) {
-            atomicOr(err, KERR_SINGULAR);
-            for (int k = 0; k < 81; ++k) d[k] = 0.0;
+        if (t < n) {
+            double* d = s_m + 81 * t;
+            if (!material_dpdf(MAT, thr, mu, lambda, f, d)) {
+                ok = false;
+                for (int k = 0; k < 81; ++k) d[k] = 0.0;
+            }
         }
-        for (int k = 0; k < 81; ++k) dP[81 * q + k] = d[k];
+        __syncthreads();
+        for (int i = t; i < 81 * n; i += MT_PTS) dP[81 * q0 + i] = s_m[i];
     }
+    if (!ok) *err = KERR_SINGULAR;  // pinned host word; every writer stores the same value
 }
 
 // Stable Neo-Hookean energy density of nq deformation gradients (column-major F[9 q .. 9 q + 8])
@@ -1087,17 +1108,20 @@ void material_energy(double mu, double lambda, int64_t nq, const double* F, doub
 
 void material_eval(int mat, double thr, double mu_r, double lambda_r, int64_t nq, const double* F, double* P,
                    double* dPdF) {
-    DevBuf<int> err;
-    err.alloc(1);
-    HIP_CHECK(hipMemset(err.get(), 0, sizeof(int)));
+    // the error word, written by the kernel into host memory: one per thread, for the life of the process
+    static thread_local PinnedBuf<int>* err = nullptr;
+    if (!err) err = new PinnedBuf<int>(1, hipHostMallocCoherent);
+    volatile int* h = err->p;
+    *h = 0;
     if (nq > 0) {
-        hipLaunchKernelGGL(k_material, dim3((unsigned)((nq + 127) / 128)), dim3(128), 0, nullptr, mat, thr, mu_r, lambda_r, nq, F,
-                           P, dPdF, err.get());
+        const unsigned g = (unsigned)((nq + MT_PTS - 1) / MT_PTS);
+        const uint32_t lds = (uint32_t)(sizeof(double) * MT_PTS * (dPdF ? 81 : 9));
+        HOEFEM_MATERIAL_DISPATCH(mat, hipLaunchKernelGGL(k_material<MK>, dim3(g), dim3(MT_PTS), lds, nullptr, thr, mu_r,
+                                                         lambda_r, nq, F, P, dPdF, err->p));
         check_launch("k_material");
     }
-    int h = 0;
-    HIP_CHECK(hipMemcpy(&h, err.get(), sizeof(int), hipMemcpyDeviceToHost));
-    if (h & KERR_SINGULAR) throw Error(HOEFEM_ERROR_SINGULAR, "singular deformation gradient");
+    HIP_CHECK(hipStreamSynchronize(nullptr));
+    if (*h & KERR_SINGULAR) throw Error(HOEFEM_ERROR_SINGULAR, "singular deformation gradient");
 }
 
 void rotation_svd_eval(int64_t nq, const double* F, double* U, double* S, double* Vt) {
