@@ -483,8 +483,7 @@ __global__ __launch_bounds__(EIG_THREADS) void k_psd_certify(const int32_t* __re
 // (Higham, "Functions of Matrices", SIAM 2008, sec. 5.3). Every X_k is a polynomial in B, so the
 // eigenvectors are B's and each eigenvalue x follows the scalar map: x in (0, 1] goes to 1, x < 0
 // to -1, x = 0 stays. PSD_NS_ITERS steps settle every eigenvalue with |lambda| >= 1.5^-59 |B|_F
-// (~4e-11 |B|_F); smaller ones contribute at most |lambda| to the error. The block is dim x dim
-// in LDS padded to a multiple of 4; products in 4 x 4 register tiles, one or two per thread.
+// (~4e-11 |B|_F); smaller ones contribute at most |lambda| to the error.
 constexpr int PSD_NS_ITERS = 64;
 
 __device__ inline void tile_gemm(const double* __restrict__ X, const double* __restrict__ Y, int dp, int ld, int ti,
@@ -506,22 +505,29 @@ __device__ inline void tile_gemm(const double* __restrict__ X, const double* __r
     }
 }
 
+// One block per work-group of four wavefronts, X and T in LDS as NT x NT tiles of 16 x 16 (dim <= 16 NT, zero
+// padding), the products on v_mfma_f64_16x16x4 (lane layout as in k_spd_inverse_mf). X, X^2 and
+// X (3 I - X^2) / 2 are symmetric, so an iteration computes the tiles on and below the diagonal and
+// mirrors their lower triangle; X and T are exactly symmetric, as their reads along rows for both operands need (an
+// antisymmetric part would double with every iteration): 2 NT (NT + 1) / 2 tiles of 4 NT instructions, dealt to the wavefronts in turn. Bound by the
+// matrix cores (64 cycles per instruction and SIMD): 3840 blocks of 60 x 60 are 79M instructions, 2.0 ms at the
+// peak rate. 560 blocks of 60 x 60 take 918 us; 3307 us with 4 x 4 register tiles on the vector units, 1804 us with the
+// products' operands read down columns.
+template <int NT>
 __global__ __launch_bounds__(EIG_THREADS) void k_psd_newton_schulz(const int32_t* __restrict__ msz,
                                                                    const int64_t* __restrict__ val_off,
                                                                    double* __restrict__ blocks,
-                                                                   const int* __restrict__ need, int ldpad) {
+                                                                   const int* __restrict__ need) {
     if (need[blockIdx.x] == 0) return;
+    constexpr int PD = 16 * NT, LD = PD + 1, LOWER = NT * (NT + 1) / 2, PER = (LOWER + 3) / 4;
     extern __shared__ double lds[];
     __shared__ double s_red[EIG_THREADS];
     const int64_t b = blockIdx.x;
     const int dim = 3 * msz[b];
-    const int dp = (dim + 3) & ~3;
-    const int ld = ldpad;  // >= dp
-    const int nt = dp / 4, ntiles = nt * nt;
     double* X = lds;
-    double* T = lds + (size_t)dp * ld;
+    double* T = lds + PD * LD;
     double* blk = blocks + val_off[b];
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, w = t >> 6, l = t & 63;
     double loc = 0.0;
     for (int idx = t; idx < dim * dim; idx += EIG_THREADS) {
         const double v = blk[idx];
@@ -530,77 +536,78 @@ __global__ __launch_bounds__(EIG_THREADS) void k_psd_newton_schulz(const int32_t
     const double nrm = sqrt(block_sum(loc, s_red));
     if (nrm == 0.0) return;  // uniform
     const double inv = 1.0 / nrm;
-    for (int idx = t; idx < dp * dp; idx += EIG_THREADS) {
-        const int r = idx / dp, c = idx % dp;
-        X[r * ld + c] = (r < dim && c < dim) ? 0.5 * (blk[r * dim + c] + blk[c * dim + r]) * inv : 0.0;
-    }
+    // dst = s (B + B^T) / 2
+    auto load = [&](double* dst, double s) {
+        for (int idx = t; idx < PD * PD; idx += EIG_THREADS) {
+            const int r = idx / PD, c = idx % PD;
+            dst[r * LD + c] = (r < dim && c < dim) ? 0.5 * (blk[r * dim + c] + blk[c * dim + r]) * s : 0.0;
+        }
+    };
+    load(X, inv);  // symmetric: both sums of two commute
     __syncthreads();
-    double acc[2][4][4];
+    // tile (ti, tj) of A B for a symmetric A, whose operand A(r, k) is read as A(k, r), along a row as B's is
+    auto product = [&](const double* A, const double* B, int ti, int tj) {
+        sgj_double4 acc = {0.0, 0.0, 0.0, 0.0};
+        const double* pa = A + (l >> 4) * LD + 16 * ti + (l & 15);
+        const double* pb = B + (l >> 4) * LD + 16 * tj + (l & 15);
+#pragma unroll
+        for (int ks = 0; ks < 4 * NT; ++ks)  // entries past dim are zero
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[4 * ks * LD], pb[4 * ks * LD], acc, 0, 0, 0);
+        return acc;
+    };
+    // the tiles on and below the diagonal, tile n = ti (ti + 1) / 2 + tj to wavefront n % 4
+    auto each_tile = [&](auto f) {
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int n = 4 * q + w;
+            if (n >= LOWER) break;  // uniform over the wavefront
+            int ti = 0;
+            while ((ti + 1) * (ti + 2) / 2 <= n) ++ti;
+            f(q, ti, n - ti * (ti + 1) / 2);
+        }
+    };
+    sgj_double4 acc[PER];
     for (int it = 0; it < PSD_NS_ITERS; ++it) {
         // T = X X
-        for (int q = 0; q < 2; ++q) {
-            const int tile = t + q * EIG_THREADS;
-            if (tile < ntiles) tile_gemm(X, X, dp, ld, tile / nt, tile % nt, acc[q]);
-        }
-        for (int q = 0; q < 2; ++q) {
-            const int tile = t + q * EIG_THREADS;
-            if (tile < ntiles) {
-                const int ti = tile / nt, tj = tile % nt;
+        each_tile([&](int, int ti, int tj) {
+            const sgj_double4 d = product(X, X, ti, tj);
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) T[(4 * ti + a) * ld + 4 * tj + c] = acc[q][a][c];
+            for (int v = 0; v < 4; ++v) {
+                const int r = 16 * ti + 4 * v + (l >> 4), c = 16 * tj + (l & 15);
+                if (ti != tj || r >= c) T[r * LD + c] = T[c * LD + r] = d[v];
             }
-        }
+        });
         __syncthreads();
-        // X <- 1.5 X - 0.5 X T
-        for (int q = 0; q < 2; ++q) {
-            const int tile = t + q * EIG_THREADS;
-            if (tile < ntiles) tile_gemm(X, T, dp, ld, tile / nt, tile % nt, acc[q]);
-        }
+        // X <- 1.5 X - 0.5 X T, stored once every product has read X
+        each_tile([&](int q, int ti, int tj) { acc[q] = product(X, T, ti, tj); });
         __syncthreads();
-        for (int q = 0; q < 2; ++q) {
-            const int tile = t + q * EIG_THREADS;
-            if (tile < ntiles) {
-                const int ti = tile / nt, tj = tile % nt;
+        each_tile([&](int q, int ti, int tj) {
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        double* x = &X[(4 * ti + a) * ld + 4 * tj + c];
-                        *x = 1.5 * *x - 0.5 * acc[q][a][c];
-                    }
+            for (int v = 0; v < 4; ++v) {
+                const int r = 16 * ti + 4 * v + (l >> 4), c = 16 * tj + (l & 15);
+                if (ti != tj || r >= c) X[r * LD + c] = X[c * LD + r] = 1.5 * X[r * LD + c] - 0.5 * acc[q][v];
             }
-        }
+        });
         __syncthreads();
     }
-    // P = (B + B S) / 2 with B = nrm X_0: X_0 back into T, then the product
-    for (int idx = t; idx < dp * dp; idx += EIG_THREADS) {
-        const int r = idx / dp, c = idx % dp;
-        T[r * ld + c] = (r < dim && c < dim) ? 0.5 * (blk[r * dim + c] + blk[c * dim + r]) : 0.0;
-    }
+    // P = (B + B S) / 2: B back into T, B S into the block, then symmetrized (B S is symmetric in exact arithmetic)
+    load(T, 1.0);
     __syncthreads();
-    for (int q = 0; q < 2; ++q) {
-        const int tile = t + q * EIG_THREADS;
-        if (tile < ntiles) tile_gemm(T, X, dp, ld, tile / nt, tile % nt, acc[q]);
-    }
-    __syncthreads();
-    for (int q = 0; q < 2; ++q) {
-        const int tile = t + q * EIG_THREADS;
-        if (tile < ntiles) {
-            const int ti = tile / nt, tj = tile % nt;
-            for (int a = 0; a < 4; ++a)
-                for (int c = 0; c < 4; ++c) {
-                    const int r = 4 * ti + a, cc = 4 * tj + c;
-                    if (r < dim && cc < dim) X[r * ld + cc] = 0.5 * (T[r * ld + cc] + acc[q][a][c]);
-                }
+    for (int n = w; n < NT * NT; n += 4) {
+        const int ti = n / NT, tj = n % NT;
+        const sgj_double4 d = product(T, X, ti, tj);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = 16 * ti + 4 * v + (l >> 4), c = 16 * tj + (l & 15);
+            if (r < dim && c < dim) blk[r * dim + c] = 0.5 * (T[r * LD + c] + d[v]);
         }
     }
+    __syncthreads();  // the work-group's stores are visible to it
+    for (int idx = t; idx < dim * dim; idx += EIG_THREADS) X[(idx / dim) * LD + idx % dim] = blk[idx];
     __syncthreads();
-    // symmetrize on the way out (B S is symmetric in exact arithmetic)
     for (int idx = t; idx < dim * dim; idx += EIG_THREADS) {
         const int r = idx / dim, c = idx % dim;
-        blk[idx] = 0.5 * (X[r * ld + c] + X[c * ld + r]);
+        blk[idx] = 0.5 * (X[r * LD + c] + X[c * LD + r]);
     }
 }
 
@@ -1199,14 +1206,20 @@ void launch_element_psd_projection(Model& m) {
     hipLaunchKernelGGL(k_psd_certify, dim3((unsigned)m.ne), dim3(EIG_THREADS), lds_c, m.stream, m.d_elem_m.get(),
                        m.d_elem_off.get(), (const double*)m.d_ke.get(), m.d_elem_need.get(), ld_c);
     check_launch("k_psd_certify");
-    const int dp = (dim + 3) & ~3;
-    const int ld_ns = dp + 1;
-    const size_t lds_ns = (size_t)2 * dp * ld_ns * sizeof(double);
-    if (lds_ns > 120 * 1024 || (dp / 4) * (dp / 4) > 2 * EIG_THREADS)
-        throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "element matrix too large for the projection");
-    raise_lds_limit((const void*)k_psd_newton_schulz, 120 * 1024);
-    hipLaunchKernelGGL(k_psd_newton_schulz, dim3((unsigned)m.ne), dim3(EIG_THREADS), lds_ns, m.stream,
-                       m.d_elem_m.get(), m.d_elem_off.get(), m.d_ke.get(), (const int*)m.d_elem_need.get(), ld_ns);
+    const int nt = (dim + 15) / 16;
+    const size_t lds_ns = (size_t)2 * 16 * nt * (16 * nt + 1) * sizeof(double);  // 149 KB at 81 x 81
+    auto run = [&](auto kernel) {
+        raise_lds_limit((const void*)kernel, lds_ns);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)m.ne), dim3(EIG_THREADS), lds_ns, m.stream, m.d_elem_m.get(),
+                           m.d_elem_off.get(), m.d_ke.get(), (const int*)m.d_elem_need.get());
+    };
+    switch (nt) {
+        case 1: run(&k_psd_newton_schulz<1>); break;
+        case 2: run(&k_psd_newton_schulz<2>); break;
+        case 4: run(&k_psd_newton_schulz<4>); break;
+        case 6: run(&k_psd_newton_schulz<6>); break;
+        default: throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "element matrix size without a projection kernel");
+    }
     check_launch("k_psd_newton_schulz");
 }
 
