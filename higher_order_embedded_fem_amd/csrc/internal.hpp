@@ -274,12 +274,12 @@ struct Schwarz {
     DevBuf<float> d_vals32;        // P values (FP32)
     DevBuf<double> d_blocks;       // gathered / inverted blocks (always FP64)
     DevBuf<int> d_fallback;        // per block: 1 if the Gauss-Jordan path rejected it (eigen path)
-    // blocks above SCHWARZ_SMALL_DIM: blocked Gauss-Jordan in global memory (32 x 32 MFMA tiles)
+    // blocks above SCHWARZ_SMALL_DIM: blocked Gauss-Jordan in global memory (64 x 64 tiles)
     int small_max_dim = 0, large_max_dim = 0;
     std::vector<int32_t> large;    // their block indices
     DevBuf<int32_t> d_large;
-    DevBuf<int64_t> d_colp_off;    // per large block: offset of its column-panel copy (dim x 32)
-    DevBuf<double> d_piv, d_colp, d_lnorm;  // pivot tile inverses, column panels, |B|_F^2 and |B^-1|_F^2
+    DevBuf<int64_t> d_panel_off;   // per large block: offset of its panels (64 x 64 tiles)
+    DevBuf<double> d_piv, d_panels, d_lnorm;  // pivot tile inverses, column and row panels, partial norms
 };
 constexpr int SCHWARZ_SMALL_DIM = 96;  // blocks up to this size: register Gauss-Jordan / LDS eigen paths
 

@@ -40,8 +40,8 @@ void schwarz_setup(Schwarz& s, Model& m, int64_t nsub, const int64_t* off, const
     s.jslot.resize(s.scatter.slot.size());
     s.small_max_dim = s.large_max_dim = 0;
     s.large.clear();
-    std::vector<int64_t> colp_off;
-    int64_t colp_total = 0;
+    std::vector<int64_t> panel_off;
+    int64_t panel_total = 0;
     for (int64_t b = 0; b < nsub; ++b) {
         const int32_t* g = s.nodes.data() + s.off[b];
         const int mb = (int)(s.off[b + 1] - s.off[b]);
@@ -50,8 +50,8 @@ void schwarz_setup(Schwarz& s, Model& m, int64_t nsub, const int64_t* off, const
         if (3 * mb > SCHWARZ_SMALL_DIM) {
             s.large.push_back((int32_t)b);
             s.large_max_dim = std::max(s.large_max_dim, 3 * mb);
-            colp_off.push_back(colp_total);
-            colp_total += (int64_t)3 * mb * 32;
+            panel_off.push_back(panel_total);
+            panel_total += ((int64_t)3 * mb + 63) / 64 * 64 * 64;  // 64 x 64 tiles
         } else {
             s.small_max_dim = std::max(s.small_max_dim, 3 * mb);
         }
@@ -78,10 +78,11 @@ void schwarz_setup(Schwarz& s, Model& m, int64_t nsub, const int64_t* off, const
     s.d_fallback.ensure(std::max<int64_t>(nsub, 1));
     if (!s.large.empty()) {
         s.d_large.upload(s.large, m.stream);
-        s.d_colp_off.upload(colp_off, m.stream);
-        s.d_piv.ensure(s.large.size() * 32 * 32);
-        s.d_colp.ensure((size_t)colp_total);
-        s.d_lnorm.ensure(2 * s.large.size() * BGJ_NORM_SPLIT);
+        s.d_panel_off.upload(panel_off, m.stream);
+        s.d_piv.ensure(s.large.size() * 64 * 64);
+        s.d_panels.ensure((size_t)2 * panel_total);
+        const size_t nt = ((size_t)s.large_max_dim + 63) / 64;
+        s.d_lnorm.ensure(s.large.size() * (BGJ_NORM_SPLIT + nt * (nt + 1) / 2));
     }
 }
 
@@ -301,53 +302,55 @@ __global__ __launch_bounds__(EIG_THREADS) void k_spd_inverse(const int32_t* __re
 
 typedef double sgj_double4 __attribute__((ext_vector_type(4)));
 
-// The same inversion on the matrix cores: in-place blocked Gauss-Jordan over NT x NT tiles of 16 x 16
-// (dim <= 16 NT; the padding is the identity), one work-group of four wavefronts per block, the block
-// in LDS (row stride LD = 16 NT + 1). For each diagonal tile k:
-//   D = A_kk^-1        wavefront 0, pivot by pivot (the pivots are those of the unblocked elimination,
-//                      so a non-positive one marks the block exactly as k_spd_inverse does)
-//   A_kj = D A_kj      (j != k)
-//   A_ij -= A_ik A_kj  (i, j != k; the new A_kj, the old A_ik)
-//   A_ik = -A_ik D     (i != k);  A_kk = D
-// The tile products run on v_mfma_f64_16x16x4 (lane l: A operand X(l % 16, 4 s + l / 16), B operand
-// Y(4 s + l / 16, l % 16), result item v = (4 v + l / 16, l % 16)), the tiles of each step dealt to
-// the wavefronts in turn. The certificate and the symmetrized write-back are k_spd_inverse's.
-template <int NT>
-__global__ __launch_bounds__(EIG_THREADS) void k_spd_inverse_mf(const int32_t* __restrict__ msz,
-                                                                const int64_t* __restrict__ val_off,
-                                                                double* __restrict__ blocks, int* __restrict__ fallback) {
-    constexpr int PD = 16 * NT, LD = PD + 1;
-    extern __shared__ double s_a[];  // [PD][LD]
-    __shared__ double s_red[EIG_THREADS];
-    __shared__ int s_bad;
-    const int64_t b = blockIdx.x;
-    const int dim = 3 * msz[b];
-    if (dim > SCHWARZ_SMALL_DIM || dim > PD) {  // handled by the blocked path in global memory
-        if (threadIdx.x == 0) fallback[b] = 4;
-        return;
+// v of lane p of each row of 16 lanes, in all of the row's lanes
+template <int P>
+__device__ inline double row_lane(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x150 + P, 0xf, 0xf, false);  // row_newbcast
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + P, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ inline double lane_value(double v, int lane) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_ds_bpermute(4 * lane, (int)b), hi = __builtin_amdgcn_ds_bpermute(4 * lane, (int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// One pivot of the in-register inversion of a 16 x 16 tile by a wavefront (lane l: column l % 16, rows
+// 4 (l / 16) .. + 3 in a[4]); false if the pivot is not positive, uniformly.
+template <int P>
+__device__ inline bool gj_pivot(double (&a)[4], int l) {
+    constexpr int G = P / 4, M = P % 4;
+    const long long pb = __double_as_longlong(a[M]);
+    const int plo = __builtin_amdgcn_readlane((int)pb, 16 * G + P), phi = __builtin_amdgcn_readlane((int)(pb >> 32), 16 * G + P);
+    const double piv = __longlong_as_double(((long long)phi << 32) | (unsigned)plo);
+    if (!(piv > 0.0) || !isfinite(piv)) return false;
+    const double ip = 1.0 / piv;
+    const int j = l & 15, g = l >> 4;
+    const double row = lane_value(a[M], 16 * G + j);  // a(P, j)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const double col = row_lane<P>(a[m]);  // a(i, P), i = 4 g + m
+        const bool ip_row = g == G && m == M, ip_col = j == P;
+        a[m] = ip_row ? (ip_col ? ip : row * ip) : (ip_col ? -col * ip : a[m] - col * row * ip);
     }
+    return true;
+}
+template <int P>
+__device__ inline bool gj_pivots(double (&a)[4], int l) {
+    if constexpr (P == 16)
+        return true;
+    else
+        return gj_pivot<P>(a, l) && gj_pivots<P + 1>(a, l);
+}
+
+// The elimination of k_spd_inverse_mf, in place on the NT x NT tiles in s_a (row stride 16 NT + 1; rows and
+// columns past dim are the identity's), by the NW wavefronts of a work-group. s_bad: LDS, 0. Ends with a
+// barrier; false if a pivot is not positive.
+template <int NT, int NW>
+__device__ inline bool gj_tiles(double* s_a, int dim, int& s_bad) {
+    constexpr int LD = 16 * NT + 1;
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
-    double* blk = blocks + val_off[b];
-    for (int idx = t; idx < PD * PD; idx += EIG_THREADS) {
-        const int i = idx / PD, j = idx % PD;
-        s_a[i * LD + j] = (i < dim && j < dim) ? blk[(int64_t)i * dim + j] : (i == j ? 1.0 : 0.0);
-    }
-    if (t == 0) s_bad = 0;
-    __syncthreads();
-    // |.|_F^2 and |.|_inf of the block's dim x dim part
-    auto norms = [&](double& f2, double& finf) {
-        double loc = 0.0, row = 0.0;
-        for (int idx = t; idx < dim * dim; idx += EIG_THREADS) {
-            const double x = s_a[(idx / dim) * LD + idx % dim];
-            loc += x * x;
-        }
-        if (t < dim)
-            for (int j = 0; j < dim; ++j) row += fabs(s_a[t * LD + j]);
-        f2 = block_sum(loc, s_red);
-        finf = block_max(row, s_red);
-    };
-    double nb2, nbinf;
-    norms(nb2, nbinf);
     // C = (neg ? -1 : 1) X Y (+ Cin), 16 x 16 tiles at (xr, xc), (yr, yc) of s_a
     auto tile_mul = [&](int xr, int xc, int yr, int yc, bool neg, sgj_double4 acc) {
 #pragma unroll
@@ -369,62 +372,114 @@ __global__ __launch_bounds__(EIG_THREADS) void k_spd_inverse_mf(const int32_t* _
         return acc;
     };
     const sgj_double4 zero = {0.0, 0.0, 0.0, 0.0};
+    constexpr int O = NT - 1;  // tiles other than kt
+#pragma unroll 1
     for (int kt = 0; kt < NT && 16 * kt < dim; ++kt) {
         const int K = 16 * kt;
-        if (w == 0) {  // D = A_kk^-1 in place, one wavefront: its LDS accesses take effect in order
-            for (int p = 0; p < 16; ++p) {
-                const double piv = s_a[(K + p) * LD + K + p];
-                if (!(piv > 0.0) || !isfinite(piv)) {
-                    if (l == 0) s_bad = 1;
-                    break;
-                }
-                const double ip = 1.0 / piv;
-                double nv[4];
+        auto other = [&](int n) { return 16 * (n < kt ? n : n + 1); };
+        if (w == 0) {  // D = A_kk^-1 in one wavefront's registers
+            double a[4];
+            double* src = s_a + (K + 4 * (l >> 4)) * LD + K + (l & 15);
 #pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const int e = l + 64 * m, i = e >> 4, j = e & 15;
-                    const double aij = s_a[(K + i) * LD + K + j];
-                    const double aip = s_a[(K + i) * LD + K + p], apj = s_a[(K + p) * LD + K + j];
-                    nv[m] = (i == p && j == p) ? ip : (i == p ? apj * ip : (j == p ? -aip * ip : aij - aip * apj * ip));
-                }
-                __builtin_amdgcn_wave_barrier();
+            for (int m = 0; m < 4; ++m) a[m] = src[m * LD];
+            if (gj_pivots<0>(a, l)) {
 #pragma unroll
-                for (int m = 0; m < 4; ++m) {
-                    const int e = l + 64 * m;
-                    s_a[(K + (e >> 4)) * LD + K + (e & 15)] = nv[m];
-                }
-                __builtin_amdgcn_wave_barrier();
+                for (int m = 0; m < 4; ++m) src[m * LD] = a[m];
+            } else if (l == 0) {
+                s_bad = 1;
             }
         }
         __syncthreads();
-        if (s_bad) {  // the same in every thread: uniform exit
-            if (t == 0) fallback[b] = 1;
-            return;
-        }
+        if (s_bad) return false;  // the same in every thread
         // row panel A_kj = D A_kj: the tile's old values are read (by its wavefront) before it is written
-        for (int j = 0, n = 0; j < NT; ++j) {
-            if (j == kt) continue;
-            if ((n++ & 3) == w) tile_store(K, 16 * j, tile_mul(K, K, K, 16 * j, false, zero));
+#pragma unroll 1
+        for (int n = w; n < O; n += NW) tile_store(K, other(n), tile_mul(K, K, K, other(n), false, zero));
+        __syncthreads();
+#pragma unroll 1
+        for (int n = w; n < O * O; n += NW) {
+            const int i = other(n / (O ? O : 1)), j = other(n % (O ? O : 1));
+            tile_store(i, j, tile_mul(i, K, K, j, true, tile_load(i, j)));
         }
         __syncthreads();
-        for (int i = 0, n = 0; i < NT; ++i) {
-            if (i == kt) continue;
-            for (int j = 0; j < NT; ++j) {
-                if (j == kt) continue;
-                if ((n++ & 3) == w) tile_store(16 * i, 16 * j, tile_mul(16 * i, K, K, 16 * j, true, tile_load(16 * i, 16 * j)));
+#pragma unroll 1
+        for (int n = w; n < O; n += NW) tile_store(other(n), K, tile_mul(other(n), K, K, K, true, zero));
+        __syncthreads();
+    }
+    return true;
+}
+
+// The same inversion on the matrix cores: in-place blocked Gauss-Jordan over NT x NT tiles of 16 x 16
+// (dim <= 16 NT; the padding is the identity), one work-group of NW wavefronts per block, the block
+// in LDS (row stride LD = 16 NT + 1). For each diagonal tile k:
+//   D = A_kk^-1        wavefront 0, in registers, pivot by pivot (the pivots are those of the unblocked
+//                      elimination, so a non-positive one marks the block exactly as k_spd_inverse does)
+//   A_kj = D A_kj      (j != k)
+//   A_ij -= A_ik A_kj  (i, j != k; the new A_kj, the old A_ik)
+//   A_ik = -A_ik D     (i != k);  A_kk = D
+// The tile products run on v_mfma_f64_16x16x4 (lane l: A operand X(l % 16, 4 s + l / 16), B operand
+// Y(4 s + l / 16, l % 16), result item v = (4 v + l / 16, l % 16)), the tiles of each step dealt to
+// the wavefronts in turn. The certificate and the symmetrized write-back are k_spd_inverse's. Blocks of one or
+// two tiles (Tet4, Hex8, Tet10) take a wavefront each: their steps have one tile product.
+template <int NT, int NW>
+__global__ __launch_bounds__(64 * NW) void k_spd_inverse_mf(const int32_t* __restrict__ msz,
+                                                            const int64_t* __restrict__ val_off,
+                                                            double* __restrict__ blocks, int* __restrict__ fallback) {
+    constexpr int PD = 16 * NT, LD = PD + 1, THREADS = 64 * NW;
+    extern __shared__ double s_a[];  // [PD][LD]
+    __shared__ double s_red[2][NW];
+    __shared__ int s_bad;
+    const int64_t b = blockIdx.x;
+    const int dim = 3 * msz[b];
+    if (dim > SCHWARZ_SMALL_DIM || dim > PD) {  // handled by the blocked path in global memory
+        if (threadIdx.x == 0) fallback[b] = 4;
+        return;
+    }
+    const int t = threadIdx.x;
+    double* blk = blocks + val_off[b];
+    for (int idx = t; idx < PD * PD; idx += THREADS) {
+        const int i = idx / PD, j = idx % PD;
+        s_a[i * LD + j] = (i < dim && j < dim) ? blk[(int64_t)i * dim + j] : (i == j ? 1.0 : 0.0);
+    }
+    if (t == 0) s_bad = 0;
+    __syncthreads();
+    // |.|_F^2 and |.|_inf of the block's dim x dim part, a row per lane; ends with a barrier
+    auto norms = [&](double& f2, double& finf) {
+        double loc = 0.0, row = 0.0;
+        for (int r = t; r < dim; r += THREADS) {
+            double sum = 0.0;
+            for (int j = 0; j < dim; ++j) {
+                const double x = s_a[r * LD + j];
+                loc += x * x;
+                sum += fabs(x);
             }
+            row = fmax(row, sum);
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+            loc += __shfl_xor(loc, off, 64);
+            row = fmax(row, __shfl_xor(row, off, 64));
+        }
+        if ((t & 63) == 0) {
+            s_red[0][t >> 6] = loc;
+            s_red[1][t >> 6] = row;
         }
         __syncthreads();
-        for (int i = 0, n = 0; i < NT; ++i) {
-            if (i == kt) continue;
-            if ((n++ & 3) == w) tile_store(16 * i, K, tile_mul(16 * i, K, K, K, true, zero));
+        f2 = finf = 0.0;
+        for (int w = 0; w < NW; ++w) {
+            f2 += s_red[0][w];
+            finf = fmax(finf, s_red[1][w]);
         }
         __syncthreads();
+    };
+    double nb2, nbinf;
+    norms(nb2, nbinf);
+    if (!gj_tiles<NT, NW>(s_a, dim, s_bad)) {  // the same in every thread: uniform exit
+        if (t == 0) fallback[b] = 1;
+        return;
     }
     double ni2, niinf;
     norms(ni2, niinf);
     const double cert = fmin(sqrt(nb2) * sqrt(ni2), nbinf * niinf);
-    for (int idx = t; idx < dim * dim; idx += EIG_THREADS) {
+    for (int idx = t; idx < dim * dim; idx += THREADS) {
         const int i = idx / dim, j = idx % dim;
         blk[(int64_t)i * dim + j] = 0.5 * (s_a[i * LD + j] + s_a[j * LD + i]);
     }
@@ -855,47 +910,32 @@ __global__ __launch_bounds__(EIG_THREADS) void k_jacobi_inverse(const int32_t* _
 }
 
 // ------------------------------------------------------------------ blocks above 96 x 96
-// Blocked Gauss-Jordan inversion in global memory, 32 x 32 tiles, all large blocks of an update
-// together. For panel k (rows / columns 32k ..): (1) the pivot tile A_kk is inverted in LDS
-// (P = A_kk^-1, unpivoted: every pivot is a diagonal entry of a Schur complement, positive iff the
-// block is positive definite); (2) the row panel A_kj <- P A_kj (j != k) and a copy C of the old
-// column panel A_ik (i != k); (3) A_ij -= C_i A_kj (i, j != k), A_ik <- -C_i P, A_kk <- P. Steps 2
-// and 3 multiply 32 x 32 tiles on v_mfma_f64_16x16x4 (each of four wavefronts a 16 x 16 quarter).
+// Blocked Gauss-Jordan inversion in global memory, 64 x 64 tiles, all large blocks of an update
+// together. The block and every intermediate matrix are known from their lower triangles: with S the panels
+// eliminated so far, M_ij is symmetric between tiles that are both in S or both not, and
+// M_ji = -M_ij^T between one in S and one not. So only tiles on and below the diagonal are read and written.
+// For panel k:
+//   (1) P = A_kk^-1 in LDS (gj_tiles: unpivoted; every pivot is a diagonal entry of a Schur complement,
+//       positive iff the block is positive definite);
+//   (2) for every tile t != k: C_t = A_tk (t > k as stored; t < k, already eliminated: -A_kt^T) and
+//       R_t = M_kt = s_t P C_t^T, s_t = 1 for t > k and -1 for t < k; stored as M_tk = -R_t^T (t > k) or
+//       M_kt = R_t (t < k), M_kk = P, and C and R as panels for (3);
+//   (3) M_ij = A_ij - C_i R_j for tiles i >= j other than k.
+// The products run on v_mfma_f64_16x16x4. (3) is bound by memory: it reads and writes half a block once per
+// panel, 51 blocks of 570 x 570 (132 MB, held by the Infinity Cache) in 9 panels; 32 x 32 tiles over whole blocks
+// moved four times as much (18 panels; 64 us per panel, 2.1 ms per update).
 // The inverse is accepted when |B|_F |B^-1|_F < SPD_COND_LIMIT (an upper bound of kappa_2): the
-// eigenvalue clamp is then inactive and B^+ = B^-1; it is symmetrized as in k_spd_inverse. A block
-// without that certificate (indefinite or too ill-conditioned) raises KERR_SCHWARZ: large blocks have
-// no eigen fallback.
-constexpr int BT = 32, BTP = 33;  // tile size, LDS row stride
+// eigenvalue clamp is then inactive and B^+ = B^-1. A block without that certificate (indefinite or too
+// ill-conditioned) raises KERR_SCHWARZ: large blocks have no eigen fallback.
+constexpr int BT = 64, BTP = 65;  // tile size, LDS row stride
 
-typedef double bgj_double4 __attribute__((ext_vector_type(4)));
-
-// dst(32 x 32 tile in LDS) = src rows r0.., cols c0.. of a row-major dim x dim block, zero outside
-__device__ inline void bgj_load(double* dst, const double* src, int dim, int r0, int c0, double sign) {
-    for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
-        const int r = idx / BT, c = idx % BT;
-        dst[r * BTP + c] = (r0 + r < dim && c0 + c < dim) ? sign * src[(int64_t)(r0 + r) * dim + c0 + c] : 0.0;
-    }
-}
-
-// acc (this wavefront's 16 x 16 quarter (si, sj) of a 32 x 32 tile) += A B, A and B 32 x 32 in LDS
-__device__ inline void bgj_mfma(bgj_double4& acc, const double* A, const double* B, int si, int sj) {
-    const int l = threadIdx.x & 63;
-#pragma unroll
-    for (int ks = 0; ks < BT / 4; ++ks) {
-        const double a = A[(16 * si + (l & 15)) * BTP + 4 * ks + (l >> 4)];
-        const double b = B[(4 * ks + (l >> 4)) * BTP + 16 * sj + (l & 15)];
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-    }
-}
-
-// |B|_F^2 (which = 0) or |B^-1|_F^2 (which = 1) of every large block in BGJ_NORM_SPLIT partial sums:
-// work-group (l, y) sums the y-th contiguous chunk of block l's entries into
-// out[(2 l + which) BGJ_NORM_SPLIT + y]; k_bgj_finish adds the partials in order.
+// |B|_F^2 of every large block in BGJ_NORM_SPLIT partial sums: work-group (l, y) sums the y-th contiguous
+// chunk of block l's entries into out[y] of the block's partials; k_bgj_check adds the partials in order.
 __global__ __launch_bounds__(EIG_THREADS) void k_bgj_norm(const int32_t* __restrict__ large,
                                                           const int32_t* __restrict__ msz,
                                                           const int64_t* __restrict__ val_off,
                                                           const double* __restrict__ blocks, double* __restrict__ out,
-                                                          int which) {
+                                                          int stride) {
     __shared__ double s_red[EIG_THREADS];
     const int b = large[blockIdx.x];
     const int dim = 3 * msz[b];
@@ -906,200 +946,270 @@ __global__ __launch_bounds__(EIG_THREADS) void k_bgj_norm(const int32_t* __restr
     double loc = 0.0;
     for (int64_t idx = c0 + threadIdx.x; idx < c1; idx += EIG_THREADS) loc += blk[idx] * blk[idx];
     const double tot = block_sum(loc, s_red);
-    if (threadIdx.x == 0) out[(2 * (int64_t)blockIdx.x + which) * BGJ_NORM_SPLIT + blockIdx.y] = tot;
+    if (threadIdx.x == 0) out[(int64_t)blockIdx.x * stride + blockIdx.y] = tot;
 }
 
-// (1) P = A_kk^-1 for every large block with a panel k
+// (1) P = A_kk^-1 by a work-group whose s_a (stride BTP) holds A_kk (bk x bk, its lower triangle mirrored,
+// the padding the identity); false, in every thread, and an error if the block is not positive definite
+__device__ inline bool bgj_invert(double* s_a, int bk, int& s_bad, double* out, int* err) {
+    if (threadIdx.x == 0) s_bad = 0;
+    __syncthreads();
+    if (!gj_tiles<BT / 16, 4>(s_a, bk, s_bad)) {
+        if (threadIdx.x == 0) atomicOr(err, KERR_SCHWARZ);
+        return false;
+    }
+    for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
+        const int r = idx / BT, c = idx % BT;
+        out[idx] = 0.5 * (s_a[r * BTP + c] + s_a[c * BTP + r]);
+    }
+    return true;
+}
+
+// panel 0's pivot tile of every large block; the others' are inverted where the update finishes them
 __global__ __launch_bounds__(EIG_THREADS) void k_bgj_pivot(const int32_t* __restrict__ large,
                                                            const int32_t* __restrict__ msz,
                                                            const int64_t* __restrict__ val_off,
                                                            const double* __restrict__ blocks, double* __restrict__ piv,
-                                                           int* __restrict__ fallback, int* err, int k) {
-    __shared__ double T[BT * BTP];
-    __shared__ double s_row[BT], s_col[BT];
+                                                           int* __restrict__ fallback, int* err) {
+    __shared__ double s_a[BT * BTP];
+    __shared__ int s_bad;
     const int lb = blockIdx.x, b = large[lb];
     const int dim = 3 * msz[b];
-    if (BT * k >= dim || fallback[b] != 4) return;
-    const int bk = min(BT, dim - BT * k);
+    if (fallback[b] != 4) return;
+    const int bk = min(BT, dim);
     const double* blk = blocks + val_off[b];
     for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
         const int r = idx / BT, c = idx % BT;
-        T[r * BTP + c] = (r < bk && c < bk) ? blk[(int64_t)(BT * k + r) * dim + BT * k + c] : (r == c ? 1.0 : 0.0);
+        const int i = max(r, c), j = min(r, c);  // the lower triangle's entry
+        s_a[r * BTP + c] = i < bk ? blk[(int64_t)i * dim + j] : (r == c ? 1.0 : 0.0);
     }
-    __syncthreads();
-    for (int p = 0; p < bk; ++p) {
-        if (threadIdx.x < BT) {
-            s_row[threadIdx.x] = T[p * BTP + threadIdx.x];
-            s_col[threadIdx.x] = T[threadIdx.x * BTP + p];
-        }
-        __syncthreads();
-        const double pv = s_row[p];
-        if (!(pv > 0.0) || !isfinite(pv)) {  // uniform: the block is not positive definite
-            if (threadIdx.x == 0) {
-                fallback[b] = 5;
-                atomicOr(err, KERR_SCHWARZ);
-            }
-            return;
-        }
-        const double ip = 1.0 / pv;
-        for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
-            const int r = idx / BT, c = idx % BT;
-            double v = T[r * BTP + c];
-            if (r == p && c == p)
-                v = ip;
-            else if (r == p)
-                v = s_row[c] * ip;
-            else if (c == p)
-                v = -s_col[r] * ip;
-            else
-                v -= s_col[r] * s_row[c] * ip;
-            T[r * BTP + c] = v;
-        }
-        __syncthreads();
-    }
-    double* out = piv + (int64_t)lb * BT * BT;
-    for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) out[idx] = T[(idx / BT) * BTP + idx % BT];
+    if (!bgj_invert(s_a, bk, s_bad, piv + (int64_t)lb * BT * BT, err) && threadIdx.x == 0) fallback[b] = 5;
 }
 
-// (2) row panel A_kj <- P A_kj and the copy C_j = A_jk of the column panel, tile j != k
+// acc[2 a + c] += the 16 x 16 tiles (2 si + a, 2 sj + c) of A B (64 x 64 in LDS): a wavefront's 32 x 32 quarter
+__device__ inline void bgj_mfma(sgj_double4 (&acc)[4], const double* A, const double* B, int si, int sj) {
+    const int l = threadIdx.x & 63;
+    const double* pa = A + (32 * si + (l & 15)) * BTP + (l >> 4);
+    const double* pb = B + (l >> 4) * BTP + 32 * sj + (l & 15);
+#pragma unroll 4
+    for (int ks = 0; ks < BT / 4; ++ks) {
+        const double a0 = pa[4 * ks], a1 = pa[16 * BTP + 4 * ks];
+        const double b0 = pb[4 * ks * BTP], b1 = pb[4 * ks * BTP + 16];
+        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[1], 0, 0, 0);
+        acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[2], 0, 0, 0);
+        acc[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[3], 0, 0, 0);
+    }
+}
+
+// f(row, column, acc item) over the wavefront's quarter of a 64 x 64 tile
+template <class F>
+__device__ inline void bgj_each(int si, int sj, F f) {
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) f(32 * si + 16 * (q >> 1) + 4 * v + (l >> 4), 32 * sj + 16 * (q & 1) + (l & 15), q, v);
+}
+
+// (2) the panels C_t and R_t of tile t and the block's new tile; colp and rowp hold 64 x 64 tiles, zero past dim
 __global__ __launch_bounds__(EIG_THREADS) void k_bgj_panel(const int32_t* __restrict__ large,
                                                            const int32_t* __restrict__ msz,
                                                            const int64_t* __restrict__ val_off,
                                                            double* __restrict__ blocks, const double* __restrict__ piv,
-                                                           double* __restrict__ colp,
-                                                           const int64_t* __restrict__ colp_off,
+                                                           double* __restrict__ colp, double* __restrict__ rowp,
+                                                           const int64_t* __restrict__ panel_off,
                                                            const int* __restrict__ fallback, int k) {
-    __shared__ double sP[BT * BTP], sR[BT * BTP];
+    extern __shared__ double lds[];
+    double *sP = lds, *sC = lds + BT * BTP;  // sC: C_t^T
     const int lb = blockIdx.x, b = large[lb], t = blockIdx.y;
     const int dim = 3 * msz[b];
     const int nt = (dim + BT - 1) / BT;
-    if (BT * k >= dim || t >= nt || t == k || fallback[b] != 4) return;
+    if (BT * k >= dim || t >= nt || fallback[b] != 4) return;
     double* blk = blocks + val_off[b];
-    // the column panel's tile (rows 32 t.., columns 32 k..), before step 3 overwrites it
-    double* C = colp + colp_off[lb];
+    const double* P = piv + (int64_t)lb * BT * BT;
+    if (t == k) {
+        for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
+            const int r = BT * k + idx / BT, c = BT * k + idx % BT;
+            if (r < dim && c < dim) blk[(int64_t)r * dim + c] = P[idx];
+        }
+        return;
+    }
     for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
         const int r = idx / BT, c = idx % BT;
-        if (BT * t + r < dim && BT * k + c < dim)
-            C[(int64_t)(BT * t + r) * BT + c] = blk[(int64_t)(BT * t + r) * dim + BT * k + c];
+        sP[r * BTP + c] = P[idx];
+        // the stored tile: rows of the larger tile index
+        const int gr = BT * max(t, k) + r, gc = BT * min(t, k) + c;
+        const double v = gr < dim && gc < dim ? blk[(int64_t)gr * dim + gc] : 0.0;
+        if (t > k)
+            sC[c * BTP + r] = v;
+        else
+            sC[r * BTP + c] = -v;
     }
-    const double* P = piv + (int64_t)lb * BT * BT;
-    for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) sP[(idx / BT) * BTP + idx % BT] = P[idx];
-    bgj_load(sR, blk, dim, BT * k, BT * t, 1.0);
     __syncthreads();
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, si = w >> 1, sj = w & 1;
-    bgj_double4 acc = {0.0, 0.0, 0.0, 0.0};
-    bgj_mfma(acc, sP, sR, si, sj);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int r = BT * k + 16 * si + 4 * v + (l >> 4), c = BT * t + 16 * sj + (l & 15);
-        if (r < dim && c < dim) blk[(int64_t)r * dim + c] = acc[v];
+    double* C = colp + panel_off[lb] + (int64_t)t * BT * BT;
+    double* R = rowp + panel_off[lb] + (int64_t)t * BT * BT;
+    for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) C[idx] = sC[(idx % BT) * BTP + idx / BT];
+    const int w = threadIdx.x >> 6, si = w >> 1, sj = w & 1;
+    sgj_double4 acc[4] = {};
+    bgj_mfma(acc, sP, sC, si, sj);
+    const double sign = t > k ? 1.0 : -1.0;
+    bgj_each(si, sj, [&](int r, int c, int q, int v) {
+        const double x = sign * acc[q][v];
+        R[r * BT + c] = x;
+        if (t < k && BT * k + r < dim && BT * t + c < dim) blk[(int64_t)(BT * k + r) * dim + BT * t + c] = x;
+    });
+    if (t < k) return;
+    __syncthreads();  // M_tk = -R_t^T by way of sC, so that its rows are stored contiguously
+    bgj_each(si, sj, [&](int r, int c, int q, int v) { sC[c * BTP + r] = -acc[q][v]; });
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
+        const int r = BT * t + idx / BT, c = BT * k + idx % BT;
+        if (r < dim && c < dim) blk[(int64_t)r * dim + c] = sC[(idx / BT) * BTP + idx % BT];
     }
 }
 
-// (3) A_ij -= C_i A_kj (i, j != k), A_ik = -C_i P, A_kk = P
+// tile pair of index n among those on and below the diagonal
+__device__ inline void bgj_lower(int n, int& i, int& j) {
+    i = (int)((sqrtf(8.0f * (float)n + 1.0f) - 1.0f) * 0.5f);
+    while ((i + 1) * (i + 2) / 2 <= n) ++i;
+    while (i * (i + 1) / 2 > n) --i;
+    j = n - i * (i + 1) / 2;
+}
+
+// (3) M_ij = A_ij - C_i R_j, tiles i >= j other than k. The work-group of tile (k + 1, k + 1), among the first to
+// start, goes on to invert it: the next panel's pivot, 28 us (41 us one pivot at a time through LDS), runs beside the
+// other tiles' updates. Two work-groups per CU by their LDS, so its registers cost the others nothing.
 __global__ __launch_bounds__(EIG_THREADS) void k_bgj_update(const int32_t* __restrict__ large,
                                                             const int32_t* __restrict__ msz,
                                                             const int64_t* __restrict__ val_off,
-                                                            double* __restrict__ blocks, const double* __restrict__ piv,
-                                                            const double* __restrict__ colp,
-                                                            const int64_t* __restrict__ colp_off,
-                                                            const int* __restrict__ fallback, int k, int ntm) {
-    __shared__ double sA[BT * BTP], sB[BT * BTP];
+                                                            double* __restrict__ blocks, const double* __restrict__ colp,
+                                                            const double* __restrict__ rowp,
+                                                            const int64_t* __restrict__ panel_off,
+                                                            double* __restrict__ piv, const int* __restrict__ fallback,
+                                                            int* err, int k) {
+    extern __shared__ double lds[];
+    __shared__ int s_bad;
+    double *sA = lds, *sB = lds + BT * BTP;
     const int lb = blockIdx.x, b = large[lb];
-    const int ti = blockIdx.y / ntm, tj = blockIdx.y % ntm;
     const int dim = 3 * msz[b];
-    const int nt = (dim + BT - 1) / BT;
-    if (BT * k >= dim || ti >= nt || tj >= nt || (ti == k && tj != k) || fallback[b] != 4) return;
+    int ti, tj, n = (int)blockIdx.y;
+    const int next = (k + 1) * (k + 2) / 2 + k + 1;  // tile (k + 1, k + 1), swapped with tile 0
+    if (next < (int)gridDim.y && (n == 0 || n == next)) n = next - n;
+    bgj_lower(n, ti, tj);
+    if (BT * k >= dim || BT * ti >= dim || ti == k || tj == k || fallback[b] != 4) return;
     double* blk = blocks + val_off[b];
-    const double* P = piv + (int64_t)lb * BT * BT;
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, si = w >> 1, sj = w & 1;
-    bgj_double4 acc = {0.0, 0.0, 0.0, 0.0};
-    if (ti == k) {  // tj == k: the pivot tile becomes P
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[v] = P[(16 * si + 4 * v + (l >> 4)) * BT + 16 * sj + (l & 15)];
-    } else {
-        // -C_i: the column panel copy, rows 32 ti..
-        const double* C = colp + colp_off[lb];
-        for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
-            const int r = idx / BT, c = idx % BT;
-            sA[r * BTP + c] = (BT * ti + r < dim && BT * k + c < dim) ? -C[(int64_t)(BT * ti + r) * BT + c] : 0.0;
-        }
-        if (tj == k) {
-            for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) sB[(idx / BT) * BTP + idx % BT] = P[idx];
-        } else {
-            bgj_load(sB, blk, dim, BT * k, BT * tj, 1.0);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int r = BT * ti + 16 * si + 4 * v + (l >> 4), c = BT * tj + 16 * sj + (l & 15);
-                acc[v] = (r < dim && c < dim) ? blk[(int64_t)r * dim + c] : 0.0;
-            }
-        }
-        __syncthreads();
-        bgj_mfma(acc, sA, sB, si, sj);
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const int r = BT * ti + 16 * si + 4 * v + (l >> 4), c = BT * tj + 16 * sj + (l & 15);
-        if (r < dim && c < dim) blk[(int64_t)r * dim + c] = acc[v];
-    }
-}
-
-// certificate and symmetrization: tile pairs (ti <= tj) of every large block
-__global__ __launch_bounds__(EIG_THREADS) void k_bgj_finish(const int32_t* __restrict__ large,
-                                                            const int32_t* __restrict__ msz,
-                                                            const int64_t* __restrict__ val_off,
-                                                            double* __restrict__ blocks, const double* __restrict__ lnorm,
-                                                            int* __restrict__ fallback, int* err, int ntm) {
-    __shared__ double sA[BT * BTP], sB[BT * BTP];
-    const int lb = blockIdx.x, b = large[lb];
-    const int ti = blockIdx.y / ntm, tj = blockIdx.y % ntm;
-    const int dim = 3 * msz[b];
-    const int nt = (dim + BT - 1) / BT;
-    if (ti >= nt || tj >= nt || ti > tj || fallback[b] != 4) return;
-    double n2[2] = {0.0, 0.0};  // the partial sums of k_bgj_norm, in order
-    for (int w = 0; w < 2; ++w)
-        for (int y = 0; y < BGJ_NORM_SPLIT; ++y) n2[w] += lnorm[(2 * (int64_t)lb + w) * BGJ_NORM_SPLIT + y];
-    const double cert = sqrt(n2[0]) * sqrt(n2[1]);
-    if (!(cert < SPD_COND_LIMIT)) {  // uniform over the block's work-groups
-        if (threadIdx.x == 0 && ti == 0 && tj == 0) atomicOr(err, KERR_SCHWARZ);
-        return;
-    }
-    double* blk = blocks + val_off[b];
-    bgj_load(sA, blk, dim, BT * ti, BT * tj, 1.0);
-    bgj_load(sB, blk, dim, BT * tj, BT * ti, 1.0);
-    __syncthreads();
+    const int w = threadIdx.x >> 6, si = w >> 1, sj = w & 1;
+    const double* C = colp + panel_off[lb] + (int64_t)ti * BT * BT;
+    const double* R = rowp + panel_off[lb] + (int64_t)tj * BT * BT;
+    sgj_double4 acc[4];
+    bgj_each(si, sj, [&](int r, int c, int q, int v) {
+        const int gr = BT * ti + r, gc = BT * tj + c;
+        acc[q][v] = gr < dim && gc < dim ? blk[(int64_t)gr * dim + gc] : 0.0;
+    });
     for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
         const int r = idx / BT, c = idx % BT;
-        const double v = 0.5 * (sA[r * BTP + c] + sB[c * BTP + r]);
-        if (BT * ti + r < dim && BT * tj + c < dim) blk[(int64_t)(BT * ti + r) * dim + BT * tj + c] = v;
-        if (BT * tj + c < dim && BT * ti + r < dim) blk[(int64_t)(BT * tj + c) * dim + BT * ti + r] = v;
+        sA[r * BTP + c] = -C[idx];
+        sB[r * BTP + c] = R[idx];
     }
+    __syncthreads();
+    bgj_mfma(acc, sA, sB, si, sj);
+    bgj_each(si, sj, [&](int r, int c, int q, int v) {
+        const int gr = BT * ti + r, gc = BT * tj + c;
+        if (gr < dim && gc < dim) blk[(int64_t)gr * dim + gc] = acc[q][v];
+    });
+    if (n != next) return;
+    const int bk = min(BT, dim - BT * (k + 1));
+    __syncthreads();  // sA has been read
+    bgj_each(si, sj, [&](int r, int c, int q, int v) {
+        if (r < c) return;
+        const double x = r < bk ? acc[q][v] : (r == c ? 1.0 : 0.0);
+        sA[r * BTP + c] = x;
+        sA[c * BTP + r] = x;
+    });
+    bgj_invert(sA, bk, s_bad, piv + (int64_t)lb * BT * BT, err);
+}
+
+// The inverse's upper triangle from its lower one (the diagonal tiles averaged with their transposes), and
+// the tile pair's share of |B^-1|_F^2 into the block's partials after the BGJ_NORM_SPLIT of |B|_F^2
+__global__ __launch_bounds__(EIG_THREADS) void k_bgj_mirror(const int32_t* __restrict__ large,
+                                                            const int32_t* __restrict__ msz,
+                                                            const int64_t* __restrict__ val_off,
+                                                            double* __restrict__ blocks, double* __restrict__ lnorm,
+                                                            const int* __restrict__ fallback, int stride) {
+    __shared__ double sA[BT * BTP];
+    __shared__ double s_red[EIG_THREADS];
+    const int lb = blockIdx.x, b = large[lb];
+    const int dim = 3 * msz[b];
+    int ti, tj;
+    bgj_lower((int)blockIdx.y, ti, tj);
+    if (BT * ti >= dim || fallback[b] != 4) return;
+    double* blk = blocks + val_off[b];
+    for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
+        const int r = idx / BT, c = idx % BT, gr = BT * ti + r, gc = BT * tj + c;
+        sA[r * BTP + c] = gr < dim && gc < dim ? blk[(int64_t)gr * dim + gc] : 0.0;
+    }
+    __syncthreads();
+    double loc = 0.0;
+    for (int idx = threadIdx.x; idx < BT * BT; idx += EIG_THREADS) {
+        const int r = idx / BT, c = idx % BT, gr = BT * tj + r, gc = BT * ti + c;  // entry (r, c) of tile (tj, ti)
+        const double x = ti == tj ? 0.5 * (sA[r * BTP + c] + sA[c * BTP + r]) : sA[c * BTP + r];
+        loc += x * x;
+        if (gr < dim && gc < dim) blk[(int64_t)gr * dim + gc] = x;
+    }
+    const double tot = block_sum(loc, s_red);
+    if (threadIdx.x == 0) lnorm[(int64_t)lb * stride + BGJ_NORM_SPLIT + blockIdx.y] = ti == tj ? tot : 2.0 * tot;
+}
+
+// the certificate of every large block from its norms' partial sums
+__global__ __launch_bounds__(64) void k_bgj_check(const int32_t* __restrict__ large, const int32_t* __restrict__ msz,
+                                                  const double* __restrict__ lnorm, const int* __restrict__ fallback,
+                                                  int* err, int stride) {
+    const int lb = blockIdx.x, b = large[lb];
+    if (fallback[b] != 4) return;
+    const int nt = (3 * msz[b] + BT - 1) / BT, parts = nt * (nt + 1) / 2;
+    const double* n2 = lnorm + (int64_t)lb * stride;
+    double nb = 0.0, ni = 0.0;
+    for (int y = threadIdx.x; y < BGJ_NORM_SPLIT; y += 64) nb += n2[y];
+    for (int y = threadIdx.x; y < parts; y += 64) ni += n2[BGJ_NORM_SPLIT + y];
+    for (int off = 32; off > 0; off >>= 1) {
+        nb += __shfl_xor(nb, off, 64);
+        ni += __shfl_xor(ni, off, 64);
+    }
+    if (threadIdx.x == 0 && !(sqrt(nb) * sqrt(ni) < SPD_COND_LIMIT)) atomicOr(err, KERR_SCHWARZ);
 }
 
 static void schwarz_update_large(Schwarz& s) {
     Model& m = *s.model;
     const hipStream_t st = m.stream;
     const unsigned nl = (unsigned)s.large.size();
-    const int ntm = (s.large_max_dim + BT - 1) / BT;
+    const int ntm = (s.large_max_dim + BT - 1) / BT, lower = ntm * (ntm + 1) / 2;
+    const int stride = BGJ_NORM_SPLIT + lower;
     const int32_t* lg = s.d_large.get();
     const int32_t* msz = s.scatter.d_m.get();
     const int64_t* vo = s.scatter.d_val_off.get();
+    const int64_t* po = s.d_panel_off.get();
+    const int* fb = s.d_fallback.get();
+    double* colp = s.d_panels.get();
+    double* rowp = colp + s.d_panels.n / 2;
+    const size_t lds = (size_t)2 * BT * BTP * sizeof(double);
+    raise_lds_limit((const void*)k_bgj_panel, lds);
+    raise_lds_limit((const void*)k_bgj_update, lds);
     hipLaunchKernelGGL(k_bgj_norm, dim3(nl, BGJ_NORM_SPLIT), dim3(EIG_THREADS), 0, st, lg, msz, vo,
-                       (const double*)s.d_blocks.get(), s.d_lnorm.get(), 0);
+                       (const double*)s.d_blocks.get(), s.d_lnorm.get(), stride);
+    hipLaunchKernelGGL(k_bgj_pivot, dim3(nl), dim3(EIG_THREADS), 0, st, lg, msz, vo, (const double*)s.d_blocks.get(),
+                       s.d_piv.get(), s.d_fallback.get(), m.d_err.get());
     for (int k = 0; k < ntm; ++k) {
-        hipLaunchKernelGGL(k_bgj_pivot, dim3(nl), dim3(EIG_THREADS), 0, st, lg, msz, vo,
-                           (const double*)s.d_blocks.get(), s.d_piv.get(), s.d_fallback.get(), m.d_err.get(), k);
-        hipLaunchKernelGGL(k_bgj_panel, dim3(nl, (unsigned)ntm), dim3(EIG_THREADS), 0, st, lg, msz, vo,
-                           s.d_blocks.get(), (const double*)s.d_piv.get(), s.d_colp.get(),
-                           (const int64_t*)s.d_colp_off.get(), (const int*)s.d_fallback.get(), k);
-        hipLaunchKernelGGL(k_bgj_update, dim3(nl, (unsigned)(ntm * ntm)), dim3(EIG_THREADS), 0, st, lg, msz, vo,
-                           s.d_blocks.get(), (const double*)s.d_piv.get(), (const double*)s.d_colp.get(),
-                           (const int64_t*)s.d_colp_off.get(), (const int*)s.d_fallback.get(), k, ntm);
+        hipLaunchKernelGGL(k_bgj_panel, dim3(nl, (unsigned)ntm), dim3(EIG_THREADS), lds, st, lg, msz, vo,
+                           s.d_blocks.get(), (const double*)s.d_piv.get(), colp, rowp, po, fb, k);
+        hipLaunchKernelGGL(k_bgj_update, dim3(nl, (unsigned)lower), dim3(EIG_THREADS), lds, st, lg, msz, vo,
+                           s.d_blocks.get(), (const double*)colp, (const double*)rowp, po, s.d_piv.get(),
+                           s.d_fallback.get(), m.d_err.get(), k);
     }
-    hipLaunchKernelGGL(k_bgj_norm, dim3(nl, BGJ_NORM_SPLIT), dim3(EIG_THREADS), 0, st, lg, msz, vo,
-                       (const double*)s.d_blocks.get(), s.d_lnorm.get(), 1);
-    hipLaunchKernelGGL(k_bgj_finish, dim3(nl, (unsigned)(ntm * ntm)), dim3(EIG_THREADS), 0, st, lg, msz, vo,
-                       s.d_blocks.get(), (const double*)s.d_lnorm.get(), s.d_fallback.get(), m.d_err.get(), ntm);
+    hipLaunchKernelGGL(k_bgj_mirror, dim3(nl, (unsigned)lower), dim3(EIG_THREADS), 0, st, lg, msz, vo,
+                       s.d_blocks.get(), s.d_lnorm.get(), fb, stride);
+    hipLaunchKernelGGL(k_bgj_check, dim3(nl), dim3(64), 0, st, lg, msz, (const double*)s.d_lnorm.get(), fb,
+                       m.d_err.get(), stride);
     check_launch("blocked Gauss-Jordan");
 }
 
@@ -1138,11 +1248,19 @@ static void schwarz_update_t(Schwarz& s, const VJ* J) {
         // ones by the register Gauss-Jordan (Hex27 cylinder's 81 x 81: 869 vs 938 us on the matrix cores,
         // whose LDS round trips and serial diagonal tiles dominate at that size)
         if (dim <= 64) {
-            const size_t lds = (size_t)64 * 65 * sizeof(double);
-            raise_lds_limit((const void*)k_spd_inverse_mf<4>, lds);
-            hipLaunchKernelGGL(k_spd_inverse_mf<4>, dim3((unsigned)s.nsub), dim3(EIG_THREADS), lds, st,
-                               s.scatter.d_m.get(), s.scatter.d_val_off.get(), s.d_blocks.get(), s.d_fallback.get());
-            check_launch("k_spd_inverse_mf");
+            auto run = [&](auto kernel, int nt, int nw) {
+                const size_t lds = (size_t)16 * nt * (16 * nt + 1) * sizeof(double);
+                raise_lds_limit((const void*)kernel, lds);
+                hipLaunchKernelGGL(kernel, dim3((unsigned)s.nsub), dim3(64 * nw), lds, st, s.scatter.d_m.get(),
+                                   s.scatter.d_val_off.get(), s.d_blocks.get(), s.d_fallback.get());
+                check_launch("k_spd_inverse_mf");
+            };
+            if (dim <= 16)
+                run(&k_spd_inverse_mf<1, 1>, 1, 1);
+            else if (dim <= 32)
+                run(&k_spd_inverse_mf<2, 1>, 2, 1);
+            else
+                run(&k_spd_inverse_mf<4, 4>, 4, 4);
         } else {
             hipLaunchKernelGGL(k_spd_inverse<6>, dim3((unsigned)s.nsub), dim3(EIG_THREADS), 0, st, s.scatter.d_m.get(),
                                s.scatter.d_val_off.get(), s.d_blocks.get(), s.d_fallback.get());

@@ -16,6 +16,49 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
+# Nodes per subdomain: 3 m on both sides of every multiple of 16 and 64 that a kernel's tiles end at, alone and
+# mixed in one operator (nodes of several subdomains, and of none, included). The matrix's
+# condition number is 192, so inverses of at most 450 rows agree to 192 * 450 eps = 2e-11.
+SIZES = [(1, 2, 3), (4, 5, 5), (5, 6, 9, 10), (10, 11, 16, 21), (21, 22, 31, 32), (33, 42, 43, 64), (64, 85, 86),
+         (127, 128, 150), (1, 21, 32, 33, 65, 107)]
+
+
+@pytest.mark.parametrize("sizes", SIZES, ids=lambda s: "-".join(map(str, s)))
+def test_block_inverses_at_tile_edges(sizes):
+    from higher_order_embedded_fem_amd import fem
+
+    sc = scenes.cube_scene(3, scenes.TET10)
+    om = O.Model(sc)
+    rp, col, J = rest_jacobian(sc, om, seed=2)
+    rng = np.random.default_rng(sum(sizes))
+    sets = [np.sort(rng.choice(sc.num_vertices, m, replace=False)) for m in sizes]
+    so = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    sn = np.concatenate(sets).astype(np.int32)
+    rest = np.setdiff1d(np.arange(sc.num_vertices), sn).astype(np.int32)
+    sc = dataclasses.replace(sc, subdomain_offsets=so, subdomain_nodes=sn, untreated_nodes=rest)
+    gsw = fem.SchwarzPreconditioner.from_scene(fem.ElasticityModel(sc), sc)
+    prp, pcol = gsw.pattern()
+    treated = np.isin(np.repeat(np.arange(sc.ndof) // 3, np.diff(prp)), sn)
+    expected = lapack_P(rp, col, J, prp, pcol, so, sn)
+    for _ in range(2):  # an update leaves nothing behind for the next
+        gsw.update(dev(J))
+        P = host(gsw.values())
+        assert rel(P[treated], expected[treated]) < 1e-10
+    # the largest subdomain's last DOF: its pivot is the elimination's last
+    d = 3 * int(sets[-1][-1]) + 2
+    bad = J.copy()
+    bad[rp[d] + np.searchsorted(col[rp[d]:rp[d + 1]], d)] = -1.0 * np.abs(J).max()
+    L = _lib.load()
+    status = L.hoefem_schwarz_update(gsw.h, dev(bad).data_ptr())
+    if 3 * max(sizes) > 96:
+        assert status == 3 and b"not certified" in L.hoefem_last_error()
+    else:  # indefinite small blocks take the eigenvalue path
+        assert status == 0
+        assert rel(host(gsw.values())[treated], lapack_P(rp, col, bad, prp, pcol, so, sn)[treated]) < 1e-10
+    gsw.update(dev(J))
+    assert np.array_equal(host(gsw.values()), P)
+
+
 # Element matrices of 12, 24, 30, 60 (twice) and 81 rows, indefinite ones among them. The iteration leaves
 # eigenvalues below 4e-11 |K_e| undecided, at most 81 of them: 81 * 4e-11 < 4e-9 of an element's norm, and rounding
 # far below.
