@@ -515,174 +515,60 @@ __global__ __launch_bounds__(256) void k_element_mass(int64_t ne, const int32_t*
 }
 
 // ------------------------------------------------------------------ block gather
-// One 64-lane work-group owns the row block (3 rows) of pattern node v and accumulates the
-// incident element blocks in color order in LDS (add_element_row_to_csr_row semantics,
-// fenris/src/assembly.rs:1042-1075, without the linear search: slots are precomputed).
-// mode 0: values = (values or 0) + sum; mode 1: values = (0 + c * sum) + 1 * M (J combination,
-// simulation_toolbox/src/fem/system_assembly.rs:196-235).
-// A row block wider than `chunk` neighbour nodes (large Schwarz subdomains) is done in column
-// chunks of `chunk` nodes, each a pass over the incident blocks; every entry still receives its
-// terms in color order, so the sums do not depend on the chunking.
-constexpr int GATHER_CHUNK = 896;  // 9 * 896 doubles = 63 KiB of LDS
-// threads of k_block_gather: four waves share a node row, so a row of hundreds of blocks (the
-// Schwarz operator of large subdomains) is not walked by one wave
-constexpr int GB_THREADS = 256;
-template <class TB, class TV>
-__global__ __launch_bounds__(GB_THREADS) void k_block_gather(
-    const int32_t* __restrict__ nptr, const int32_t* __restrict__ rowptr, const uint8_t* __restrict__ diag_only,
-    const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_blk, const int32_t* __restrict__ inc_loc,
-    const int32_t* __restrict__ msz, const int64_t* __restrict__ val_off, const int64_t* __restrict__ slot_off,
-    const int32_t* __restrict__ slot, const TB* __restrict__ blocks, TV* __restrict__ values, int mode,
-    double c, const double* __restrict__ M, int zero_first, const double* __restrict__ D2, double cd, double cm,
-    int chunk) {
-    extern __shared__ double s_rb[];
-    const int64_t v = blockIdx.x;
-    const int t = threadIdx.x;
-    if (diag_only[v]) return;
-    const int k = nptr[v + 1] - nptr[v];
-    if (k == 0) return;
-    const int rw = 3 * k;
-    const int64_t r0 = rowptr[3 * v];
-    // rows 3v, 3v+1, 3v+2 are contiguous: row i starts at r0 + i * rw
-    for (int c0 = 0; c0 < k; c0 += chunk) {
-        const int cw = min(chunk, k - c0);
-        const int cr = 3 * cw;  // a row's width within the chunk
-        const int R = 3 * cr;
-        for (int idx = t; idx < R; idx += GB_THREADS) {
-            const int i = idx / cr, cc = idx % cr;
-            s_rb[idx] = (zero_first || mode == 1) ? 0.0 : (double)values[r0 + i * rw + 3 * c0 + cc];
-        }
-        __syncthreads();
-        for (int it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
-            const int b = inc_blk[it], a = inc_loc[it];
-            const int mb = msz[b];
-            const int bw = 3 * mb;
-            const TB* base = blocks + val_off[b] + (int64_t)(3 * a) * bw;
-            const int32_t* sl = slot + slot_off[b] + (int64_t)a * mb;
-            for (int idx = t; idx < 3 * bw; idx += GB_THREADS) {
-                const int i = idx / bw, cc = idx % bw;
-                const int bb = cc / 3, jj = cc % 3;
-                const int col = sl[bb] - c0;
-                if (col >= 0 && col < cw) s_rb[i * cr + 3 * col + jj] += (double)base[idx];
-            }
-            __syncthreads();
-        }
-        for (int idx = t; idx < R; idx += GB_THREADS) {
-            const int i = idx / cr, cc = idx % cr;
-            const int64_t o = r0 + i * rw + 3 * c0 + cc;
-            const double s = s_rb[idx];
-            if (mode == 0)
-                values[o] = (TV)s;
-            else {
-                // compute_jacobian_combination_into (system_assembly.rs:197-235): the terms in the order
-                // stiffness, damping, mass
-                double v2 = 0.0;
-                v2 += c * s;
-                if (D2) v2 += cd * D2[o];
-                if (M) v2 += cm * M[o];
-                values[o] = (TV)v2;
-            }
-        }
-        __syncthreads();  // the next chunk reuses s_rb
+// values (+)= the sums of the dense blocks (element matrices, Schwarz block inverses), add_element_row_to_csr_row
+// semantics (fenris/src/assembly.rs:1042-1075): every CSR entry adds its terms in color order. A lane owns
+// one column of a 3x3 node block, its three entries, and reads their terms through the block's list of
+// places in the staging, built once with the pattern; the lanes of a wavefront cover neighbouring columns of
+// a row, so stores are contiguous and loads are runs of the blocks' rows. A wavefront waits for
+// three dependent reads (the list's bounds, the places, the values) whatever the number of terms, most
+// blocks having one or two, and every lane's reads are independent: bound by memory traffic.
+// mode 0: values = (values or 0) + sum; mode 1: values = (0 + c sum) + cd D2 + cm M (J combination,
+// simulation_toolbox/src/fem/system_assembly.rs:196-235, its terms in that order).
+constexpr int BS_THREADS = 256;
+template <class TB, class TV, bool UNIFORM>
+__global__ __launch_bounds__(BS_THREADS) void k_block_sum(
+    int64_t nblk, const BlockScatter::Dest* __restrict__ dest, const int32_t* __restrict__ term_ptr,
+    const uint32_t* __restrict__ term, const int32_t* __restrict__ term_row, int row_stride,
+    const TB* __restrict__ blocks, TV* __restrict__ values, int mode, double c, const double* __restrict__ M,
+    int zero_first, const double* __restrict__ D2, double cd, double cm) {
+    const int64_t i = (int64_t)blockIdx.x * BS_THREADS + threadIdx.x;
+    const int64_t B = i / 3;
+    if (B >= nblk) return;
+    const int j = (int)(i - 3 * B);
+    const BlockScatter::Dest d = dest[B];
+    const int q0 = term_ptr[B], q1 = term_ptr[B + 1];
+    if (d.row == 0) return;
+    const int64_t o = (int64_t)d.pos + j, o1 = o + d.row, o2 = o1 + d.row;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    if (!zero_first && mode == 0) {
+        s0 = (double)values[o];
+        s1 = (double)values[o1];
+        s2 = (double)values[o2];
     }
-}
-
-// The same gather with the incident blocks' metadata held one incidence per lane (moved by
-// shuffles instead of loaded per block) and each block's row values and slots loaded one block
-// ahead, so a node row's blocks cost one memory latency between them instead of three. For blocks of
-// at most 28 nodes (3 rows x 3m <= 256 values, four per lane) and rows that fit the LDS at once;
-// every entry receives its terms in the same order as in k_block_gather.
-constexpr int GP_VALS = 4;
-template <class TB, class TV>
-__global__ __launch_bounds__(64) void k_block_gather_pf(
-    const int32_t* __restrict__ nptr, const int32_t* __restrict__ rowptr, const uint8_t* __restrict__ diag_only,
-    const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_blk, const int32_t* __restrict__ inc_loc,
-    const int32_t* __restrict__ msz, const int64_t* __restrict__ val_off, const int64_t* __restrict__ slot_off,
-    const int32_t* __restrict__ slot, const TB* __restrict__ blocks, TV* __restrict__ values, int mode,
-    double c, const double* __restrict__ M, int zero_first, const double* __restrict__ D2, double cd, double cm) {
-    extern __shared__ double s_rb[];
-    const int64_t v = blockIdx.x;
-    const int t = threadIdx.x;
-    if (diag_only[v]) return;
-    const int k = nptr[v + 1] - nptr[v];
-    if (k == 0) return;
-    const int rw = 3 * k, R = 3 * rw;
-    const int64_t r0 = rowptr[3 * v];
-    const int i0 = inc_ptr[v], ninc = inc_ptr[v + 1] - i0;
-    // lane j holds incidence j (at most 64, checked by the launch)
-    int a_l = 0, mb_l = 0;
-    int64_t vo_l = 0, so_l = 0;
-    if (t < ninc) {
-        const int b = inc_blk[i0 + t];
-        a_l = inc_loc[i0 + t];
-        mb_l = msz[b];
-        vo_l = val_off[b];
-        so_l = slot_off[b];
+#pragma unroll 2
+    for (int q = q0; q < q1; ++q) {
+        const TB* src = blocks + 3 * (int64_t)term[q] + j;
+        const int64_t r = UNIFORM ? row_stride : term_row[q];
+        s0 += (double)src[0];
+        s1 += (double)src[r];
+        s2 += (double)src[2 * r];
     }
-    for (int idx = t; idx < R; idx += 64) s_rb[idx] = (zero_first || mode == 1) ? 0.0 : (double)values[r0 + idx];
-    // incidence j's row values and slots: every lane loads (a lane past the block's 3 x 3m values
-    // re-reads its first one and does not use it), so the loads in flight are counted statically and
-    // adding one incidence waits only for its own loads
-    auto fetch = [&](int j, double* vv, int* ss, int& bwj) {
-        const int a = __shfl(a_l, j, 64), mb = __shfl(mb_l, j, 64);
-        const int64_t vo = __shfl(vo_l, j, 64), so = __shfl(so_l, j, 64);
-        const int bw = 3 * mb;
-        bwj = bw;
-        const TB* base = blocks + vo + (int64_t)(3 * a) * bw;
-        const int32_t* sl = slot + so + (int64_t)a * mb;
-#pragma unroll
-        for (int q = 0; q < GP_VALS; ++q) {
-            const int idx = t + 64 * q;
-            const int id = idx < 3 * bw ? idx : 0;
-            vv[q] = (double)base[id];
-            ss[q] = sl[(id % bw) / 3];
-        }
+    if (mode == 0) {
+        values[o] = (TV)s0;
+        values[o1] = (TV)s1;
+        values[o2] = (TV)s2;
+        return;
+    }
+    auto combine = [&](double sum, int64_t at) {
+        double v = 0.0;
+        v += c * sum;
+        if (D2) v += cd * D2[at];
+        if (M) v += cm * M[at];
+        return (TV)v;
     };
-    // two incidence buffers used in turn (no register copy between them, which would wait for the
-    // loads): the next incidence's loads are in flight while this one's values are added
-    double av[GP_VALS] = {0.0, 0.0, 0.0, 0.0}, bv[GP_VALS] = {0.0, 0.0, 0.0, 0.0};
-    int as[GP_VALS] = {0, 0, 0, 0}, bs[GP_VALS] = {0, 0, 0, 0};
-    int abw = 0, bbw = 0;
-    auto add = [&](const double* vv, const int* ss, int bw) {
-#pragma unroll
-        for (int q = 0; q < GP_VALS; ++q) {
-            const int idx = t + 64 * q;
-            if (idx < 3 * bw) {
-                const int i = idx / bw, cc = idx % bw;
-                s_rb[i * rw + 3 * ss[q] + cc % 3] += vv[q];
-            }
-        }
-    };
-    // The work-group is one wavefront, whose LDS accesses take effect in program order: the row's sums
-    // need no s_barrier, only a compiler barrier that keeps the LDS accesses of consecutive incidences
-    // in order (an s_barrier's fence would also wait for the loads of the incidence ahead). The fetches
-    // are unconditional inside the block (the last incidence again past the end), so every path reaches
-    // the loop with the same loads in flight and each addition waits only for its own incidence.
-    if (ninc > 0) {
-        fetch(0, av, as, abw);
-        __builtin_amdgcn_wave_barrier();
-        for (int j = 0; j < ninc; j += 2) {
-            fetch(min(j + 1, ninc - 1), bv, bs, bbw);
-            add(av, as, abw);
-            __builtin_amdgcn_wave_barrier();
-            fetch(min(j + 2, ninc - 1), av, as, abw);
-            if (j + 1 < ninc) add(bv, bs, bbw);
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-    for (int idx = t; idx < R; idx += 64) {
-        const int64_t o = r0 + idx;
-        const double sum = s_rb[idx];
-        if (mode == 0)
-            values[o] = (TV)sum;
-        else {
-            double v2 = 0.0;  // stiffness, damping, mass (system_assembly.rs:197-235)
-            v2 += c * sum;
-            if (D2) v2 += cd * D2[o];
-            if (M) v2 += cm * M[o];
-            values[o] = (TV)v2;
-        }
-    }
+    values[o] = combine(s0, o);
+    values[o1] = combine(s1, o1);
+    values[o2] = combine(s2, o2);
 }
 
 // f += sum of element force blocks in color order (one thread per node)
@@ -960,28 +846,19 @@ template <class TB, class TV>
 void launch_block_gather(const NodePattern& pat, const BlockScatter& sc, const TB* blocks, TV* values, int mode,
                          double c, const double* M, bool zero_first, hipStream_t s, const double* D2, double cd,
                          double cm, KernelProf* prof) {
-    if (pat.num_nodes == 0) return;
-    if (pat.max_nbr <= GATHER_CHUNK && 9 * sc.max_m <= 64 * GP_VALS && sc.max_inc <= 64) {
-        const size_t lds = (size_t)9 * std::max(pat.max_nbr, 1) * sizeof(double);
-        launch_timed(prof, k_block_gather_pf<TB, TV>, dim3((unsigned)pat.num_nodes), dim3(64), (uint32_t)lds, s,
-                     (const int32_t*)pat.d_nptr.get(), (const int32_t*)pat.d_rowptr.get(),
-                     (const uint8_t*)pat.d_diag_only.get(), (const int32_t*)sc.d_inc_ptr.get(),
-                     (const int32_t*)sc.d_inc_blk.get(), (const int32_t*)sc.d_inc_loc.get(),
-                     (const int32_t*)sc.d_m.get(), (const int64_t*)sc.d_val_off.get(),
-                     (const int64_t*)sc.d_slot_off.get(), (const int32_t*)sc.d_slot.get(), blocks, values, mode, c,
-                     M, zero_first ? 1 : 0, D2, cd, cm);
-        check_launch("k_block_gather_pf");
-        return;
-    }
-    const int chunk = std::min(std::max(pat.max_nbr, 1), GATHER_CHUNK);
-    const size_t lds = (size_t)9 * chunk * sizeof(double);
-    launch_timed(prof, k_block_gather<TB, TV>, dim3((unsigned)pat.num_nodes), dim3(GB_THREADS), (uint32_t)lds, s,
-                 (const int32_t*)pat.d_nptr.get(), (const int32_t*)pat.d_rowptr.get(),
-                 (const uint8_t*)pat.d_diag_only.get(), (const int32_t*)sc.d_inc_ptr.get(),
-                 (const int32_t*)sc.d_inc_blk.get(), (const int32_t*)sc.d_inc_loc.get(), (const int32_t*)sc.d_m.get(),
-                 (const int64_t*)sc.d_val_off.get(), (const int64_t*)sc.d_slot_off.get(),
-                 (const int32_t*)sc.d_slot.get(), blocks, values, mode, c, M, zero_first ? 1 : 0, D2, cd, cm, chunk);
-    check_launch("k_block_gather");
+    const int64_t nblk = (int64_t)sc.dest.size();
+    if (nblk == 0) return;
+    auto run = [&](auto kernel) {
+        launch_timed(prof, kernel, dim3((unsigned)((3 * nblk + BS_THREADS - 1) / BS_THREADS)), dim3(BS_THREADS), 0, s, nblk,
+                     (const BlockScatter::Dest*)sc.d_dest.get(), (const int32_t*)sc.d_term_ptr.get(),
+                     (const uint32_t*)sc.d_term.get(), (const int32_t*)sc.d_term_row.get(), sc.row_stride, blocks,
+                     values, mode, c, M, zero_first ? 1 : 0, D2, cd, cm);
+    };
+    if (sc.row_stride)
+        run(&k_block_sum<TB, TV, true>);
+    else
+        run(&k_block_sum<TB, TV, false>);
+    check_launch("k_block_sum");
 }
 template void launch_block_gather<double, double>(const NodePattern&, const BlockScatter&, const double*,
                                                   double*, int, double, const double*, bool, hipStream_t,

@@ -141,7 +141,20 @@ struct BlockScatter {
     std::vector<int32_t> inc_ptr;   // per pattern node
     int max_inc = 0;                // most incident blocks of one node
     std::vector<int32_t> inc_blk, inc_loc;  // incident (block, local node) in color order
-    DevBuf<int32_t> d_m, d_slot, d_inc_ptr, d_inc_blk, d_inc_loc;
+    // The same incidences seen from the pattern's node blocks (ncol entries): where block B's 3x3 values go,
+    // and where its terms lie in the staging, in color order: term q in [term_ptr[B], term_ptr[B + 1]) has its
+    // first value at 3 * term[q] and its rows term_row[q] apart (row_stride for all when block sizes agree)
+    struct Dest {
+        int32_t pos, row;  // first value, distance of the rows (0: a diagonal-only node's entry, not written)
+    };
+    std::vector<Dest> dest;
+    std::vector<int32_t> term_ptr, term_row;
+    std::vector<uint32_t> term;
+    int row_stride = 0;
+    DevBuf<Dest> d_dest;
+    DevBuf<int32_t> d_term_ptr, d_term_row;
+    DevBuf<uint32_t> d_term;
+    DevBuf<int32_t> d_m, d_inc_ptr, d_inc_blk, d_inc_loc;
     DevBuf<int64_t> d_val_off, d_slot_off;
     void build(const NodePattern& pat, int64_t nblocks, const int64_t* off, const int32_t* nodes,
                const std::vector<std::vector<int32_t>>* colors, int ncolor_lists);

@@ -310,11 +310,52 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
                     inc_loc[fill[v]] = a;
                     fill[v]++;
                 }
+    // the terms of every node block: each node's incidences in order, counted and placed by slot
+    row_stride = nb > 0 ? 3 * m[0] : 0;
+    for (int64_t b = 0; b < nb; ++b)
+        if (3 * m[b] != row_stride) row_stride = 0;
+    const int64_t nblk = pat.ncol.size(), nterms = slot_off[nb];
+    if (nterms > INT32_MAX || val_off[nb] / 3 > UINT32_MAX)
+        throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "too many element block entries");
+    dest.resize(nblk);
+    term_ptr.assign(nblk + 1, 0);
+    term.resize(nterms);
+    term_row.resize(row_stride ? 0 : nterms);
+    std::vector<int32_t> at;
+    for (int64_t v = 0; v < pat.num_nodes; ++v) {
+        const int32_t b0 = pat.nptr[v], k = pat.nptr[v + 1] - b0;
+        for (int j = 0; j < k; ++j)
+            dest[b0 + j] = pat.diag_only[v] ? Dest{0, 0} : Dest{pat.rowptr[3 * v] + 3 * j, 3 * k};
+        int32_t* count = term_ptr.data() + b0 + 1;
+        for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
+            const int32_t b = inc_blk[it], mb = m[b];
+            const int32_t* sl = slot.data() + slot_off[b] + (int64_t)inc_loc[it] * mb;
+            for (int c = 0; c < mb; ++c) count[sl[c]]++;
+        }
+        at.resize(k);
+        for (int j = 0; j < k; ++j) {
+            at[j] = term_ptr[b0 + j];
+            term_ptr[b0 + j + 1] += term_ptr[b0 + j];
+        }
+        for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
+            const int32_t b = inc_blk[it], mb = m[b], a = inc_loc[it];
+            const int32_t* sl = slot.data() + slot_off[b] + (int64_t)a * mb;
+            const uint32_t base = (uint32_t)(val_off[b] / 3 + (int64_t)(3 * a) * mb);  // of row 3 a, over 3
+            for (int c = 0; c < mb; ++c) {
+                const int32_t q = at[sl[c]]++;
+                term[q] = base + c;
+                if (!row_stride) term_row[q] = 3 * mb;
+            }
+        }
+    }
 }
 
 void BlockScatter::upload(hipStream_t s) {
     d_m.upload(m, s);
-    d_slot.upload(slot, s);
+    d_dest.upload(dest, s);
+    d_term_ptr.upload(term_ptr, s);
+    d_term.upload(term, s);
+    if (!row_stride) d_term_row.upload(term_row, s);
     d_inc_ptr.upload(inc_ptr, s);
     d_inc_blk.upload(inc_blk, s);
     d_inc_loc.upload(inc_loc, s);
