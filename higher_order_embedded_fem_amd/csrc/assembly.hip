@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "fem_device.hpp"
+#include "gather_device.hpp"
 #include "internal.hpp"
 
 namespace hoefem {
@@ -571,22 +572,14 @@ __global__ __launch_bounds__(BS_THREADS) void k_block_sum(
     values[o2] = combine(s2, o2);
 }
 
-// f += sum of element force blocks in color order (one thread per node)
-__global__ void k_force_gather(int64_t nn, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_blk,
+// f += sum of element force blocks in color order (one thread per DOF)
+__global__ __launch_bounds__(128) void k_force_gather(int64_t nn, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_blk,
                                const int32_t* __restrict__ inc_loc, int n, const double* __restrict__ fe,
                                double* __restrict__ f) {
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t v = i / 3;
     if (v >= nn) return;
-    double a0 = f[3 * v], a1 = f[3 * v + 1], a2 = f[3 * v + 2];
-    for (int it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
-        const double* src = fe + ((int64_t)inc_blk[it] * n + inc_loc[it]) * 3;
-        a0 += src[0];
-        a1 += src[1];
-        a2 += src[2];
-    }
-    f[3 * v] = a0;
-    f[3 * v + 1] = a1;
-    f[3 * v + 2] = a2;
+    f[i] = force_sum(f[i], inc_ptr[v], inc_ptr[v + 1], inc_blk, inc_loc, n, fe, (int)(i - 3 * v));
 }
 
 // ------------------------------------------------------------------ SpMV
@@ -875,7 +868,7 @@ template void launch_block_gather<float, double>(const NodePattern&, const Block
 
 void launch_force_gather(Model& m, double* f) {
     if (m.nv == 0) return;
-    hipLaunchKernelGGL(k_force_gather, dim3((unsigned)((m.nv + 255) / 256)), dim3(256), 0, m.stream, m.nv,
+    hipLaunchKernelGGL(k_force_gather, dim3((unsigned)((3 * m.nv + 127) / 128)), dim3(128), 0, m.stream, m.nv,
                        m.scatter.d_inc_ptr.get(), m.scatter.d_inc_blk.get(), m.scatter.d_inc_loc.get(), m.n,
                        m.d_fe.get(), f);
     check_launch("k_force_gather");

@@ -19,6 +19,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "gather_device.hpp"
 #include "grid_pcg.hpp"
 
 namespace hoefem {
@@ -1867,30 +1868,19 @@ __global__ void k_bc_copy(int64_t ndof, const double* __restrict__ src, const ui
 }
 
 // f = M g + f_int (element forces in color order) - D v, Dirichlet rows zeroed
-// (NewtonCgDynamicSystem::eval_f, newton_cg.rs:441-478); one thread per node
-__global__ void k_node_force(int64_t nn, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_blk,
+// (NewtonCgDynamicSystem::eval_f, newton_cg.rs:441-478); one thread per DOF
+__global__ __launch_bounds__(128) void k_node_force(int64_t nn, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_blk,
                              const int32_t* __restrict__ inc_loc, int n, const double* __restrict__ fe,
                              const double* __restrict__ gforce, const double* __restrict__ dv,
                              const uint8_t* __restrict__ dirmask, double* __restrict__ f) {
 #pragma clang fp contract(off)
-    const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t v = i / 3;
     if (v >= nn) return;
-    double f0 = gforce[3 * v], f1 = gforce[3 * v + 1], f2 = gforce[3 * v + 2];
-    for (int it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
-        const double* src = fe + ((int64_t)inc_blk[it] * n + inc_loc[it]) * 3;
-        f0 += src[0];
-        f1 += src[1];
-        f2 += src[2];
-    }
-    if (dv) {  // f += -D v (spmv_csr with beta = 1, alpha = -1)
-        f0 = f0 - dv[3 * v];
-        f1 = f1 - dv[3 * v + 1];
-        f2 = f2 - dv[3 * v + 2];
-    }
-    if (dirmask[v]) f0 = f1 = f2 = 0.0;
-    f[3 * v] = f0;
-    f[3 * v + 1] = f1;
-    f[3 * v + 2] = f2;
+    const bool fixed = dirmask[v];
+    double s = dev::force_sum(gforce[i], inc_ptr[v], inc_ptr[v + 1], inc_blk, inc_loc, n, fe, (int)(i - 3 * v));
+    if (dv) s = s - dv[i];  // f += -D v (spmv_csr with beta = 1, alpha = -1)
+    f[i] = fixed ? 0.0 : s;
 }
 
 // dst = src * sc  (F <- -dt f, euler.rs:110)
@@ -2103,7 +2093,7 @@ void launch_bc_copy(Model& m, const double* src, const uint8_t* dirmask, const d
 void launch_node_force(Model& m, const double* gforce, const double* dv, const uint8_t* dirmask, double* f) {
     const int64_t nn = m.nv;
     if (nn <= 0) return;
-    launch_timed(prof_slot(m), k_node_force, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, m.stream, nn,
+    launch_timed(prof_slot(m), k_node_force, dim3((unsigned)((3 * nn + 127) / 128)), dim3(128), 0, m.stream, nn,
                  (const int32_t*)m.scatter.d_inc_ptr.get(), (const int32_t*)m.scatter.d_inc_blk.get(),
                  (const int32_t*)m.scatter.d_inc_loc.get(), m.n, (const double*)m.d_fe.get(), gforce, dv, dirmask, f);
     check_launch("k_node_force");
