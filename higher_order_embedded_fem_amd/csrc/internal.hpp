@@ -294,7 +294,7 @@ struct Schwarz {
     DevBuf<int64_t> d_panel_off;   // per large block: offset of its panels (64 x 64 tiles)
     DevBuf<double> d_piv, d_panels, d_lnorm;  // pivot tile inverses, column and row panels, partial norms
 };
-constexpr int SCHWARZ_SMALL_DIM = 96;  // blocks up to this size: register Gauss-Jordan / LDS eigen paths
+constexpr int SCHWARZ_SMALL_DIM = 96;  // blocks up to this size: Gauss-Jordan and eigen paths in LDS
 
 // ------------------------------------------------------------------ CG workspace
 struct CgScalars {

@@ -2,8 +2,8 @@
 // P = sum_s R_s^T B_s^+ R_s + sum_untreated 1 / J_ii, with B_s the restriction of J to the
 // subdomain's DOFs and B_s^+ = V diag(1 / max(|lambda|, 1e-12 max|lambda|)) V^T.
 //
-// Per update: (1) gather every B_s from J (precomputed slots), (2) batched FP64 Gauss-Jordan
-// inversion in LDS, one work-group per block, accepted where it certifies that B_s is positive
+// Per update: (1) gather every B_s from J (precomputed slots) and (2) invert it by batched FP64 Gauss-Jordan
+// in LDS, one work-group per block, accepted where it certifies that B_s is positive
 // definite with kappa_2 < 1e11 (then the eigenvalue clamp is inactive and B_s^+ = B_s^-1),
 // (3) for the remaining blocks, symmetric eigen-decomposition by parallel (round-robin) Jacobi
 // in LDS and recomposition of B_s^+, (4) color-ordered gather of the blocks into P's row
@@ -86,17 +86,18 @@ void schwarz_setup(Schwarz& s, Model& m, int64_t nsub, const int64_t* off, const
     }
 }
 
-// B_s(r, c) = J[3 g_a + i, 3 g_c + j], row-major (3m)^2, always FP64. Work-group (s, y) gathers
-// entries [y SG_CHUNK, (y + 1) SG_CHUNK) of block s, so a block of hundreds of DOFs (the 64-element
+// B_s(r, c) = J[3 g_a + i, 3 g_c + j] of the blocks above 96 x 96 (listed in large), row-major (3m)^2, always
+// FP64 (the smaller ones are gathered where they are inverted). Work-group (s, y) gathers
+// entries [y SG_CHUNK, (y + 1) SG_CHUNK) of the s-th such block, so a block of hundreds of DOFs (the 64-element
 // patches) is spread over many work-groups instead of walking its entries on one.
 constexpr int SG_CHUNK = 2048;
 template <class VJ>
-__global__ void k_schwarz_gather(const int32_t* __restrict__ msz, const int64_t* __restrict__ val_off,
-                                 const int64_t* __restrict__ slot_off, const int64_t* __restrict__ noff,
+__global__ void k_schwarz_gather(const int32_t* __restrict__ large, const int32_t* __restrict__ msz,
+                                 const int64_t* __restrict__ val_off, const int64_t* __restrict__ slot_off, const int64_t* __restrict__ noff,
                                  const int32_t* __restrict__ nodes, const int32_t* __restrict__ jslot,
                                  const int32_t* __restrict__ jrowptr, const VJ* __restrict__ J,
                                  double* __restrict__ blocks) {
-    const int64_t b = blockIdx.x;
+    const int64_t b = large[blockIdx.x];
     const int mb = msz[b], dim = 3 * mb;
     const int c0 = (int)blockIdx.y * SG_CHUNK;
     if (c0 >= dim * dim) return;
@@ -144,160 +145,6 @@ __device__ inline double block_sum(double v, double* s_red) {
     const double r = s_red[0];
     __syncthreads();
     return r;
-}
-
-// Gauss-Jordan inversion of a symmetric block without pivoting, held in registers: the 16 x 16
-// threads own the entries (i, j) with i = 16 r + tr, j = 16 c + tc (r, c < 6, so dim <= 96), and
-// each pivot step broadcasts row k and column k through LDS (double-buffered: one barrier per
-// pivot). Each pivot is a diagonal entry of a Schur complement, so all pivots are positive iff B
-// is positive definite. Results per block (fallback[b]):
-//   0  pivots positive and min(|B|_F |B^-1|_F, |B|_inf |B^-1|_inf) < SPD_COND_LIMIT (both upper
-//      bounds of kappa_2(B) for symmetric B): the clamp of the pseudo-inverse is inactive, so
-//      B^+ = B^-1, and the symmetrized inverse replaces the block;
-//   2  pivots positive, the cheap bound too loose: the inverse replaces the block and
-//      k_spd_power_certify decides with a sharper bound;
-//   1  a pivot not positive: B is kept for the eigen path.
-// RR x RR register tiles per thread: RR = 6 covers blocks up to 96 x 96 (used above 64 x 64; the
-// smaller blocks go to k_spd_inverse_mf on the matrix cores, with the same results per block).
-
-// Pivot row k = 16 R + kt and column k of the register-held block into LDS (owners only).
-template <int R, int RR>
-__device__ inline void gj_publish(const double (&a)[RR][RR], double* srow, double* scol, int tr, int tc, int kt) {
-    if constexpr (R >= RR) return;
-    else {
-    if (tr == kt) {
-#pragma unroll
-        for (int c = 0; c < RR; ++c) srow[16 * c + tc] = a[R][c];
-    }
-    if (tc == kt) {
-#pragma unroll
-        for (int r = 0; r < RR; ++r) scol[16 * r + tr] = a[r][R];
-    }
-    }
-}
-
-// After the rank-1 update: row k -> a_kj / a_kk, column k -> -a_ik / a_kk, the pivot -> 1 / a_kk.
-template <int R, int RR>
-__device__ inline void gj_fix(double (&a)[RR][RR], const double (&rk)[RR], const double (&ck)[RR], double ip, int tr,
-                              int tc, int kt) {
-    if constexpr (R >= RR) return;
-    else {
-    if (tr == kt) {
-#pragma unroll
-        for (int c = 0; c < RR; ++c) a[R][c] = rk[c];
-    }
-    if (tc == kt) {
-#pragma unroll
-        for (int r = 0; r < RR; ++r) a[r][R] = -ck[r] * ip;
-    }
-    if (tr == kt && tc == kt) a[R][R] = ip;
-    }
-}
-
-template <int RR>
-__global__ __launch_bounds__(EIG_THREADS) void k_spd_inverse(const int32_t* __restrict__ msz,
-                                                             const int64_t* __restrict__ val_off,
-                                                             double* __restrict__ blocks, int* __restrict__ fallback) {
-    __shared__ double s_row[2][16 * RR], s_col[2][16 * RR];
-    __shared__ double s_x[RR][EIG_THREADS];  // row-sum partials, then the transpose exchange
-    __shared__ double s_red[EIG_THREADS];
-    const int64_t b = blockIdx.x;
-    const int dim = 3 * msz[b];
-    if (dim > SCHWARZ_SMALL_DIM) {  // handled by the blocked path
-        if (threadIdx.x == 0) fallback[b] = 4;
-        return;
-    }
-    const int t = threadIdx.x, tr = t >> 4, tc = t & 15;
-    double* blk = blocks + val_off[b];
-    double a[RR][RR];
-#pragma unroll
-    for (int r = 0; r < RR; ++r)
-#pragma unroll
-        for (int c = 0; c < RR; ++c) {
-            const int i = 16 * r + tr, j = 16 * c + tc;
-            a[r][c] = (i < dim && j < dim) ? blk[(int64_t)i * dim + j] : 0.0;
-        }
-    // |.|_F^2 and |.|_inf of the register-held matrix
-    auto norms = [&](double& f2, double& finf) {
-        double loc = 0.0, rs[RR];
-#pragma unroll
-        for (int r = 0; r < RR; ++r) {
-            rs[r] = 0.0;
-#pragma unroll
-            for (int c = 0; c < RR; ++c) {
-                loc += a[r][c] * a[r][c];
-                rs[r] += fabs(a[r][c]);
-            }
-        }
-        f2 = block_sum(loc, s_red);  // synchronizes
-        double* part = &s_x[0][0];   // [16 (tc)][96 (row)]
-#pragma unroll
-        for (int r = 0; r < RR; ++r) part[tc * (16 * RR) + 16 * r + tr] = rs[r];
-        __syncthreads();
-        double row = 0.0;
-        if (t < 16 * RR)
-            for (int q = 0; q < 16; ++q) row += part[q * (16 * RR) + t];
-        finf = block_max(row, s_red);  // synchronizes
-    };
-    double nb2, nbinf;
-    norms(nb2, nbinf);
-    for (int k = 0; k < dim; ++k) {
-        const int buf = k & 1, kr = k >> 4, kt = k & 15;
-        // kr is the same in every thread: the switch branches on it instead of selecting per entry
-        switch (kr) {
-            case 0: gj_publish<0, RR>(a, s_row[buf], s_col[buf], tr, tc, kt); break;
-            case 1: gj_publish<1, RR>(a, s_row[buf], s_col[buf], tr, tc, kt); break;
-            case 2: gj_publish<2, RR>(a, s_row[buf], s_col[buf], tr, tc, kt); break;
-            case 3: gj_publish<3, RR>(a, s_row[buf], s_col[buf], tr, tc, kt); break;
-            case 4: gj_publish<4, RR>(a, s_row[buf], s_col[buf], tr, tc, kt); break;
-            default: gj_publish<5, RR>(a, s_row[buf], s_col[buf], tr, tc, kt); break;
-        }
-        __syncthreads();
-        const double piv = s_row[buf][k];
-        if (!(piv > 0.0) || !isfinite(piv)) {  // same value in every thread: uniform exit
-            if (t == 0) fallback[b] = 1;
-            return;
-        }
-        const double ip = 1.0 / piv;
-        double rk[RR], ck[RR];
-#pragma unroll
-        for (int c = 0; c < RR; ++c) rk[c] = s_row[buf][16 * c + tc] * ip;
-#pragma unroll
-        for (int r = 0; r < RR; ++r) ck[r] = s_col[buf][16 * r + tr];
-        // a_ij - a_ik a_kj / a_kk everywhere, then row k -> a_kj / a_kk, column k -> -a_ik / a_kk,
-        // the pivot -> 1 / a_kk
-#pragma unroll
-        for (int r = 0; r < RR; ++r)
-#pragma unroll
-            for (int c = 0; c < RR; ++c) a[r][c] -= ck[r] * rk[c];
-        switch (kr) {
-            case 0: gj_fix<0, RR>(a, rk, ck, ip, tr, tc, kt); break;
-            case 1: gj_fix<1, RR>(a, rk, ck, ip, tr, tc, kt); break;
-            case 2: gj_fix<2, RR>(a, rk, ck, ip, tr, tc, kt); break;
-            case 3: gj_fix<3, RR>(a, rk, ck, ip, tr, tc, kt); break;
-            case 4: gj_fix<4, RR>(a, rk, ck, ip, tr, tc, kt); break;
-            default: gj_fix<5, RR>(a, rk, ck, ip, tr, tc, kt); break;
-        }
-    }
-    double ni2, niinf;
-    norms(ni2, niinf);
-    const double cert = fmin(sqrt(nb2) * sqrt(ni2), nbinf * niinf);
-    // symmetrize: the transpose of entry (r, c) sits in thread (tc, tr) at (c, r); round r
-    // exchanges the entries (r, 0..5)
-    const int partner = tc * 16 + tr;
-#pragma unroll
-    for (int r = 0; r < RR; ++r) {
-#pragma unroll
-        for (int x = 0; x < RR; ++x) s_x[x][t] = a[x][r];
-        __syncthreads();
-#pragma unroll
-        for (int c = 0; c < RR; ++c) {
-            const int i = 16 * r + tr, j = 16 * c + tc;
-            if (i < dim && j < dim) blk[(int64_t)i * dim + j] = 0.5 * (a[r][c] + s_x[c][partner]);
-        }
-        __syncthreads();
-    }
-    if (t == 0) fallback[b] = cert < SPD_COND_LIMIT ? 0 : 2;
 }
 
 typedef double sgj_double4 __attribute__((ext_vector_type(4)));
@@ -372,9 +219,9 @@ __device__ inline bool gj_tiles(double* s_a, int dim, int& s_bad) {
         return acc;
     };
     const sgj_double4 zero = {0.0, 0.0, 0.0, 0.0};
-    constexpr int O = NT - 1;  // tiles other than kt
+    const int O = (dim + 15) / 16 - 1;  // tiles of dim other than kt
 #pragma unroll 1
-    for (int kt = 0; kt < NT && 16 * kt < dim; ++kt) {
+    for (int kt = 0; kt <= O; ++kt) {
         const int K = 16 * kt;
         auto other = [&](int n) { return 16 * (n < kt ? n : n + 1); };
         if (w == 0) {  // D = A_kk^-1 in one wavefront's registers
@@ -397,7 +244,7 @@ __device__ inline bool gj_tiles(double* s_a, int dim, int& s_bad) {
         __syncthreads();
 #pragma unroll 1
         for (int n = w; n < O * O; n += NW) {
-            const int i = other(n / (O ? O : 1)), j = other(n % (O ? O : 1));
+            const int i = other(n / O), j = other(n % O);
             tile_store(i, j, tile_mul(i, K, K, j, true, tile_load(i, j)));
         }
         __syncthreads();
@@ -408,37 +255,65 @@ __device__ inline bool gj_tiles(double* s_a, int dim, int& s_bad) {
     return true;
 }
 
-// The same inversion on the matrix cores: in-place blocked Gauss-Jordan over NT x NT tiles of 16 x 16
-// (dim <= 16 NT; the padding is the identity), one work-group of NW wavefronts per block, the block
-// in LDS (row stride LD = 16 NT + 1). For each diagonal tile k:
-//   D = A_kk^-1        wavefront 0, in registers, pivot by pivot (the pivots are those of the unblocked
-//                      elimination, so a non-positive one marks the block exactly as k_spd_inverse does)
+// Inverse of each small symmetric block B_s(r, c) = J[3 g_a + i, 3 g_c + j], without pivoting, on the matrix cores:
+// in-place blocked Gauss-Jordan over tiles of 16 x 16 (dim <= 16 NT; the padding is the identity), one
+// work-group of NW wavefronts per block, the block gathered from J into LDS (row stride LD = 16 NT + 1). For
+// each diagonal tile k:
+//   D = A_kk^-1        wavefront 0, in registers, pivot by pivot
 //   A_kj = D A_kj      (j != k)
 //   A_ij -= A_ik A_kj  (i, j != k; the new A_kj, the old A_ik)
 //   A_ik = -A_ik D     (i != k);  A_kk = D
 // The tile products run on v_mfma_f64_16x16x4 (lane l: A operand X(l % 16, 4 s + l / 16), B operand
 // Y(4 s + l / 16, l % 16), result item v = (4 v + l / 16, l % 16)), the tiles of each step dealt to
-// the wavefronts in turn. The certificate and the symmetrized write-back are k_spd_inverse's. Blocks of one or
-// two tiles (Tet4, Hex8, Tet10) take a wavefront each: their steps have one tile product.
-template <int NT, int NW>
-__global__ __launch_bounds__(64 * NW) void k_spd_inverse_mf(const int32_t* __restrict__ msz,
-                                                            const int64_t* __restrict__ val_off,
-                                                            double* __restrict__ blocks, int* __restrict__ fallback) {
+// the wavefronts in turn. Every pivot is a diagonal entry of a Schur complement, so all are positive iff B
+// is positive definite. Results per block (fallback[b]):
+//   0  pivots positive and min(|B|_F |B^-1|_F, |B|_inf |B^-1|_inf) < SPD_COND_LIMIT (both upper
+//      bounds of kappa_2(B) for symmetric B): the clamp of the pseudo-inverse is inactive, so
+//      B^+ = B^-1, and the symmetrized inverse is the block's result;
+//   2  pivots positive, the cheap bound too loose: the inverse is stored and
+//      k_spd_power_certify decides with a sharper bound;
+//   1  a pivot not positive: B itself is stored for the eigen path.
+// A block's time is its serial chain (16 pivots per tile, about 200 cycles each, and three rounds of tile
+// products), hidden behind the other blocks of its CU. Blocks of one or two tiles (Tet4, Hex8, Tet10) take a
+// wavefront each: their rounds have one tile product. 1472 blocks of 81 x 81 took 252 us in 6 x 6 register tiles
+// on the vector units with two barriers per pivot, and 65 us to be gathered into memory first; now 190 us
+// together.
+template <class VJ, int NT, int NW>
+__global__ __launch_bounds__(64 * NW) void k_spd_inverse_mf(
+    const int32_t* __restrict__ msz, const int64_t* __restrict__ val_off, const int64_t* __restrict__ slot_off,
+    const int64_t* __restrict__ noff, const int32_t* __restrict__ nodes, const int32_t* __restrict__ jslot,
+    const int32_t* __restrict__ jrowptr, const VJ* __restrict__ J, double* __restrict__ blocks,
+    int* __restrict__ fallback) {
     constexpr int PD = 16 * NT, LD = PD + 1, THREADS = 64 * NW;
     extern __shared__ double s_a[];  // [PD][LD]
     __shared__ double s_red[2][NW];
     __shared__ int s_bad;
     const int64_t b = blockIdx.x;
-    const int dim = 3 * msz[b];
+    const int mb = msz[b], dim = 3 * mb;
     if (dim > SCHWARZ_SMALL_DIM || dim > PD) {  // handled by the blocked path in global memory
         if (threadIdx.x == 0) fallback[b] = 4;
         return;
     }
     const int t = threadIdx.x;
     double* blk = blocks + val_off[b];
+    const int32_t *g = nodes + noff[b], *slot = jslot + slot_off[b];
+    // out[r * ld + c] = B(r, c), a node pair per lane
+    auto gather = [&](double* out, int ld) {
+        for (int p = t; p < mb * mb; p += THREADS) {
+            const int a = p / mb, c = p % mb, k = slot[p];
+            double* o = out + 3 * a * ld + 3 * c;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const VJ* row = J + (k < 0 ? 0 : (int64_t)jrowptr[3 * (int64_t)g[a] + i] + 3 * k);
+#pragma unroll
+                for (int j = 0; j < 3; ++j) o[i * ld + j] = k < 0 ? 0.0 : (double)row[j];
+            }
+        }
+    };
+    gather(s_a, LD);
     for (int idx = t; idx < PD * PD; idx += THREADS) {
         const int i = idx / PD, j = idx % PD;
-        s_a[i * LD + j] = (i < dim && j < dim) ? blk[(int64_t)i * dim + j] : (i == j ? 1.0 : 0.0);
+        if (i >= dim || j >= dim) s_a[i * LD + j] = i == j ? 1.0 : 0.0;
     }
     if (t == 0) s_bad = 0;
     __syncthreads();
@@ -473,6 +348,7 @@ __global__ __launch_bounds__(64 * NW) void k_spd_inverse_mf(const int32_t* __res
     double nb2, nbinf;
     norms(nb2, nbinf);
     if (!gj_tiles<NT, NW>(s_a, dim, s_bad)) {  // the same in every thread: uniform exit
+        gather(blk, dim);
         if (t == 0) fallback[b] = 1;
         return;
     }
@@ -666,7 +542,7 @@ __global__ __launch_bounds__(EIG_THREADS) void k_psd_newton_schulz(const int32_t
     }
 }
 
-// Sharper certificate for the blocks k_spd_inverse marked 2. For symmetric X with eigenvalues
+// Sharper certificate for the blocks k_spd_inverse_mf marked 2. For symmetric X with eigenvalues
 // lambda, |X^8|_F = (sum lambda^16)^(1/2) >= max|lambda|^8, so
 //     |X|_2 <= s |(X / s)^8|_F^(1/8),  s = |X|_F,
 // an upper bound within a factor dim^(1/16) (<= 1.33) of |X|_2 instead of the factor up to dim of
@@ -1234,38 +1110,34 @@ static void schwarz_update_t(Schwarz& s, const VJ* J) {
     Model& m = *s.model;
     const hipStream_t st = m.stream;
     if (s.nsub > 0) {
-        const int64_t gmax = std::max(s.small_max_dim, s.large_max_dim);
-        const unsigned chunks = (unsigned)std::max<int64_t>(1, (gmax * gmax + SG_CHUNK - 1) / SG_CHUNK);
-        k_schwarz_gather<VJ><<<dim3((unsigned)s.nsub, chunks), dim3(256), 0, st>>>(
-            s.scatter.d_m.get(), s.scatter.d_val_off.get(), s.scatter.d_slot_off.get(), s.d_off.get(), s.d_nodes.get(),
-            s.d_jslot.get(), m.pattern.d_rowptr.get(), J, s.d_blocks.get());
-        check_launch("k_schwarz_gather");
+        if (!s.large.empty()) {
+            const int64_t gmax = s.large_max_dim;
+            const unsigned chunks = (unsigned)((gmax * gmax + SG_CHUNK - 1) / SG_CHUNK);
+            k_schwarz_gather<VJ><<<dim3((unsigned)s.large.size(), chunks), dim3(256), 0, st>>>(
+                s.d_large.get(), s.scatter.d_m.get(), s.scatter.d_val_off.get(), s.scatter.d_slot_off.get(), s.d_off.get(),
+                s.d_nodes.get(), s.d_jslot.get(), m.pattern.d_rowptr.get(), J, s.d_blocks.get());
+            check_launch("k_schwarz_gather");
+        }
         const int dim = std::max(3, s.small_max_dim);
         // Gauss-Jordan fast path (blocks up to 96 x 96; it marks the larger ones 4), the sharper
         // certificate for the blocks it could not accept, then the eigen path for the rest; blocks
         // above 96 x 96 go through the blocked path
-        // blocks up to 64 x 64 on the matrix cores (Hex20 cylinder: 93.3 vs 100.3 us per update); larger
-        // ones by the register Gauss-Jordan (Hex27 cylinder's 81 x 81: 869 vs 938 us on the matrix cores,
-        // whose LDS round trips and serial diagonal tiles dominate at that size)
-        if (dim <= 64) {
-            auto run = [&](auto kernel, int nt, int nw) {
-                const size_t lds = (size_t)16 * nt * (16 * nt + 1) * sizeof(double);
-                raise_lds_limit((const void*)kernel, lds);
-                hipLaunchKernelGGL(kernel, dim3((unsigned)s.nsub), dim3(64 * nw), lds, st, s.scatter.d_m.get(),
-                                   s.scatter.d_val_off.get(), s.d_blocks.get(), s.d_fallback.get());
-                check_launch("k_spd_inverse_mf");
-            };
-            if (dim <= 16)
-                run(&k_spd_inverse_mf<1, 1>, 1, 1);
-            else if (dim <= 32)
-                run(&k_spd_inverse_mf<2, 1>, 2, 1);
-            else
-                run(&k_spd_inverse_mf<4, 4>, 4, 4);
-        } else {
-            hipLaunchKernelGGL(k_spd_inverse<6>, dim3((unsigned)s.nsub), dim3(EIG_THREADS), 0, st, s.scatter.d_m.get(),
-                               s.scatter.d_val_off.get(), s.d_blocks.get(), s.d_fallback.get());
-            check_launch("k_spd_inverse");
-        }
+        auto run = [&](auto kernel, int nt, int nw) {
+            const size_t lds = (size_t)16 * nt * (16 * nt + 1) * sizeof(double);
+            raise_lds_limit((const void*)kernel, lds);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)s.nsub), dim3(64 * nw), lds, st, s.scatter.d_m.get(),
+                               s.scatter.d_val_off.get(), s.scatter.d_slot_off.get(), s.d_off.get(), s.d_nodes.get(),
+                               s.d_jslot.get(), m.pattern.d_rowptr.get(), J, s.d_blocks.get(), s.d_fallback.get());
+            check_launch("k_spd_inverse_mf");
+        };
+        if (dim <= 16)
+            run(&k_spd_inverse_mf<VJ, 1, 1>, 1, 1);
+        else if (dim <= 32)
+            run(&k_spd_inverse_mf<VJ, 2, 1>, 2, 1);
+        else if (dim <= 64)
+            run(&k_spd_inverse_mf<VJ, 4, 4>, 4, 4);
+        else
+            run(&k_spd_inverse_mf<VJ, 6, 8>, 6, 8);
         const int dp = (dim + 3) & ~3;
         const int ld_pc = dp + 1;
         const size_t lds_pc = (size_t)2 * dp * ld_pc * sizeof(double);  // 149 KB at dim 96
