@@ -145,133 +145,34 @@ __global__ __launch_bounds__(64) void k_element_forces(int64_t ne, const int32_t
 
 // ------------------------------------------------------------------ element tangents
 // assemble_generalized_element_stiffness (fenris/src/assembly.rs:747-797) with the SNH
-// contraction (fenris/src/solid/materials.rs:349-376, :690-743). One 256-lane work-group per
-// element; lanes = quadrature points build dP/dF and the scaled gradients in LDS, then every
-// lane accumulates a fixed set of K_e entries (lower block triangle, mirrored on write).
-// Output: row-major (3N)^2 block per element in the staging buffer.
-constexpr int STIFF_THREADS = 256;
-constexpr int STIFF_QC = 16;
-
-template <int ET, class T, int MAT>
-__global__ __launch_bounds__(STIFF_THREADS) void k_element_stiffness(
-    int64_t ne, const int32_t* __restrict__ conn, const double* __restrict__ verts, const int32_t* __restrict__ qoff,
-    const double* __restrict__ qw, const double* __restrict__ qxi, T thr, T mu, T lambda,
-    const double* __restrict__ u, T* __restrict__ ke, int* err) {
-    constexpr int N = ElemTraits<ET>::N, GN = ElemTraits<ET>::GN, M3 = 3 * N;
-    constexpr int PAIRS = N * (N + 1) / 2;
-    constexpr int ENTRIES = 9 * PAIRS;
-    constexpr int PER = (ENTRIES + STIFF_THREADS - 1) / STIFF_THREADS;
-    const int64_t e = blockIdx.x;
-    const int t = threadIdx.x;
-    __shared__ int s_node[N];
-    __shared__ T s_u[3 * N];
-    __shared__ T s_X[3 * GN];
-    __shared__ T s_C[STIFF_QC][81];
-    __shared__ T s_a[STIFF_QC][M3];
-    __shared__ unsigned char s_pI[PAIRS], s_pJ[PAIRS];
-    if (t < N) s_node[t] = conn[(int64_t)t * ne + e];
-    if (t == 0) {
-        int p = 0;
-        for (int J = 0; J < N; ++J)
-            for (int I = J; I < N; ++I) {
-                s_pI[p] = (unsigned char)I;
-                s_pJ[p] = (unsigned char)J;
-                ++p;
-            }
-    }
-    __syncthreads();
-    for (int k = t; k < 3 * N; k += STIFF_THREADS) s_u[k] = T(u[3 * (int64_t)s_node[k / 3] + k % 3]);
-    for (int k = t; k < 3 * GN; k += STIFF_THREADS) s_X[k] = T(verts[3 * (int64_t)s_node[k / 3] + k % 3]);
-    __syncthreads();
-    T acc[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) acc[j] = T(0);
-    const int q0 = qoff[e], q1 = qoff[e + 1];
-    for (int qb = q0; qb < q1; qb += STIFF_QC) {
-        const int cnt = min(STIFF_QC, q1 - qb);
-        if (t < cnt) {
-            const int q = qb + t;
-            const T xi[3] = {T(qxi[3 * q]), T(qxi[3 * q + 1]), T(qxi[3 * q + 2])};
-            T J[9], Jinv[9];
-            ref_jacobian<ET>(s_X, xi, J);
-            const T detJ = det3(J);
-            bool ok = inv3(J, Jinv);
-            T psi[4];
-            tet4_psi(xi, psi);
-            T ug[9] = {T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0), T(0)};  // u_grad(a, b) = sum_I G(a, I) u(b, I)
-            if (ok) {
-                for (int I = 0; I < N; ++I) {
-                    T Gr[3];
-                    grad_node<ET>(I, xi, psi, Gr);
-                    T G[3];
-                    // G = J^-T G_ref : G(a) = sum_c Jinv(c, a) G_ref(c)
-                    for (int a = 0; a < 3; ++a) G[a] = Jinv[0 + 3 * a] * Gr[0] + Jinv[1 + 3 * a] * Gr[1] + Jinv[2 + 3 * a] * Gr[2];
-                    for (int b = 0; b < 3; ++b)
-                        for (int a = 0; a < 3; ++a) ug[a + 3 * b] += G[a] * s_u[3 * I + b];
-                    for (int a = 0; a < 3; ++a) s_a[t][3 * I + a] = G[a];
-                }
-                const T sq = sqrt(T(qw[q]) * fabs(detJ));
-                for (int k = 0; k < M3; ++k) s_a[t][k] *= sq;
-                T F[9];
-                for (int a = 0; a < 3; ++a)
-                    for (int b = 0; b < 3; ++b) F[b + 3 * a] = ug[a + 3 * b];
-                F[0] += T(1);
-                F[4] += T(1);
-                F[8] += T(1);
-                ok = material_dpdf(MAT, thr, mu, lambda, F, s_C[t]);
-            }
-            if (!ok) {
-                atomicOr(err, KERR_SINGULAR);
-                for (int k = 0; k < 81; ++k) s_C[t][k] = T(0);
-                for (int k = 0; k < M3; ++k) s_a[t][k] = T(0);
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int ent = t + STIFF_THREADS * j;
-            if (ent < ENTRIES) {
-                const int p = ent / 9, ij = ent % 9;
-                const int i = ij % 3, jj = ij / 3;
-                const int I = s_pI[p], Jn = s_pJ[p];
-                for (int k2 = 0; k2 < cnt; ++k2) {
-                    const T* C = s_C[k2];
-                    const T* aI = s_a[k2] + 3 * I;
-                    const T* aJ = s_a[k2] + 3 * Jn;
-                    T res = T(0);
-                    for (int l = 0; l < 3; ++l)
-                        for (int k = 0; k < 3; ++k) res += C[(3 * k + i) + 9 * (3 * l + jj)] * aI[k] * aJ[l];
-                    acc[j] += res;
-                }
-            }
-        }
-        __syncthreads();
-    }
-    T* out = ke + e * (int64_t)M3 * M3;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int ent = t + STIFF_THREADS * j;
-        if (ent < ENTRIES) {
-            const int p = ent / 9, ij = ent % 9;
-            const int i = ij % 3, jj = ij / 3;
-            const int I = s_pI[p], Jn = s_pJ[p];
-            out[(3 * I + i) * M3 + 3 * Jn + jj] = acc[j];
-            if (I != Jn) out[(3 * Jn + jj) * M3 + 3 * I + i] = acc[j];
-        }
-    }
-}
-
-// FP64 element tangents on the matrix cores. With G~_q = sqrt(w_q |det J_q|) G_q (3 x N spatial
+// contraction (fenris/src/solid/materials.rs:349-376, :690-743), on the matrix cores. Output: row-major (3N)^2
+// block per element in the staging buffer. With G~_q = sqrt(w_q |det J_q|) G_q (3 x N spatial
 // gradients) and C_q = dP/dF (column-major 9 x 9, entry (3k + i, 3l + j)), the block
 //     K[(I, i), (J, j)] = sum_q sum_{k, l} G~_q(k, I) C_q(3k + i, 3l + j) G~_q(l, J)
 // is, for each component pair (i, j), the product K^{ij} = A B with A(I, kk) = G~_q(k, I) and
 // B(kk, J) = U^{ij}_q(k, J) = sum_l C_q(3k + i, 3l + j) G~_q(l, J) over kk = 3q + k. The six pairs
 // i <= j suffice (C has the major symmetry, so K^{ji} = (K^{ij})^T). Nodes are padded to 16 or 32,
 // so a pair is one or four 16 x 16 tiles, accumulated in registers across the quadrature chunks.
-// Lane layout of v_mfma_f64_16x16x4 (lane l): A operand A(l % 16, l / 16), B operand
-// B(l / 16, l % 16), result item v = D(4 v + l / 16, l % 16). Each entry of K_e is written exactly
+// Lane layout of v_mfma_f64_16x16x4 and v_mfma_f32_16x16x4 (lane l): A operand A(l % 16, l / 16), B operand
+// B(l / 16, l % 16), result item v = D(4 v + l / 16, l % 16) in FP64, D(4 (l / 16) + v, l % 16) in FP32. Each
+// entry of K_e is written exactly
 // once (diagonal pairs from their lower triangle), so K_e is exactly symmetric.
 typedef double mf_double4 __attribute__((ext_vector_type(4)));
+typedef float mf_float4 __attribute__((ext_vector_type(4)));
+template <class T>
+struct MfTile;
+template <>
+struct MfTile<double> {
+    typedef mf_double4 Acc;
+    static __device__ Acc mul(double a, double b, Acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+    static __device__ int row(int v, int l) { return 4 * v + (l >> 4); }
+};
+template <>
+struct MfTile<float> {
+    typedef mf_float4 Acc;
+    static __device__ Acc mul(float a, float b, Acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+    static __device__ int row(int v, int l) { return 4 * (l >> 4) + v; }
+};
 
 // One element per 128-lane work-group (two wavefronts; many work-groups per CU, so the SIMDs
 // interleave the phases of different elements). Quadrature points go in chunks of TW_QC:
@@ -285,13 +186,27 @@ typedef double mf_double4 __attribute__((ext_vector_type(4)));
 //    (i, j) = (w, w..2) for w = 0 and (1, 1), (1, 2), (2, 2) for w = 1, with the B operand
 //    U^{ij}(kk, col) = sum_m C_q(3k + i, 3m + j) G~(3q + m, col) formed in registers at each k-step
 //    (no U staging in LDS); a diagonal pair skips its tile above the diagonal.
+// FP32 tangents of the 24-cell Hex20 cylinder take 60 us, with vector FMAs over K_e's entries 82 us, at
+// 1.1 to 3 times its error against FP64 (2.9e-7 of the norm on 20 cells, now 0.9e-7).
 constexpr int TW_QC = 8, TW_THREADS = 128, TW_SUB = TW_THREADS / TW_QC;
 
-template <int ET, int MAT>
-__global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_element_stiffness_tw(
+// Waves per SIMD that the registers are allotted for: as many as the accumulators (12 tiles per wavefront in the
+// elements above 16 nodes) and the per-point phase leave without much spilling. Tet10, FP64, 10,368 elements:
+// 55 us with four, 63 with two.
+template <int ET, class T, int MAT>
+constexpr int tw_waves() {
+    if (ElemTraits<ET>::N > 16) return sizeof(T) == 8 || MAT != MAT_SNH ? 2 : 3;
+    if (MAT != MAT_SNH || ET == HEX8) return sizeof(T) == 8 ? 2 : 3;
+    return 4;
+}
+
+template <int ET, class T, int MAT>
+__global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(
+    tw_waves<ET, T, MAT>()))) void k_element_stiffness_tw(
     int64_t ne, const int32_t* __restrict__ conn, const double* __restrict__ verts, const int32_t* __restrict__ qoff,
-    const double* __restrict__ qw, const double* __restrict__ qxi, double thr, double mu, double lambda,
-    const double* __restrict__ u, double* __restrict__ ke, int* err) {
+    const double* __restrict__ qw, const double* __restrict__ qxi, T thr, T mu, T lambda,
+    const double* __restrict__ u, T* __restrict__ ke, int* err) {
+    typedef typename MfTile<T>::Acc Acc;
     constexpr int N = ElemTraits<ET>::N, GN = ElemTraits<ET>::GN, M3 = 3 * N;
     constexpr int NP = N > 16 ? 32 : 16, NT = NP / 16, JW = 3 * NT * NT;  // jobs per wavefront
     constexpr int KS = (3 * TW_QC) / 4;                                    // k-steps of a full chunk
@@ -301,12 +216,14 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
     __shared__ int s_node[N];
     __shared__ double s_u[3 * N];
     __shared__ double s_X[3 * GN];
-    __shared__ double s_C[TW_QC][81];
-    __shared__ double s_G[3 * TW_QC * NP];
+    __shared__ T s_C[TW_QC][81];
+    __shared__ T s_G[3 * TW_QC * NP];
     const int pq = t / TW_SUB, sub = t % TW_SUB;
     const int q0 = qoff[e], q1 = qoff[e + 1];
     if (t < N) s_node[t] = conn[(int64_t)t * ne + e];
     __syncthreads();
+    // Geometry and gradients in FP64 also for FP32 tangents (rounded where they enter s_G and F): an element's shape
+    // is then not lost in its distance from the origin
     for (int k = t; k < 3 * N; k += TW_THREADS) s_u[k] = u[3 * (int64_t)s_node[k / 3] + k % 3];
     for (int k = t; k < 3 * GN; k += TW_THREADS) s_X[k] = verts[3 * (int64_t)s_node[k / 3] + k % 3];
     // the lane's point of the first chunk (rule position and weight), loaded with the element's data
@@ -319,13 +236,13 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
         pxi[2] = qxi[3 * q + 2];
         pw = qw[q];
     }
-    mf_double4 acc[JW];
+    Acc acc[JW];
     // One chunk of up to TW_QC points. The first chunk is its own instance: its products start from
     // zero, so the accumulators hold nothing during its per-point phase (fewer live registers there).
     auto chunk = [&](int qc, auto first_tag) {
         constexpr bool FIRST = decltype(first_tag)::value;
         const int cnt = min(TW_QC, q1 - qc);
-        for (int k = t; k < 3 * TW_QC * NP; k += TW_THREADS) s_G[k] = 0.0;
+        for (int k = t; k < 3 * TW_QC * NP; k += TW_THREADS) s_G[k] = T(0);
         __syncthreads();
         // ---- per-point phase: TW_SUB lanes per quadrature point
         const bool act = pq < cnt;
@@ -358,7 +275,7 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
                     for (int a = 0; a < 3; ++a) G[a] = Jinv[0 + 3 * a] * Gr[0] + Jinv[1 + 3 * a] * Gr[1] + Jinv[2 + 3 * a] * Gr[2];
                     for (int b = 0; b < 3; ++b)
                         for (int a = 0; a < 3; ++a) ug[a + 3 * b] += G[a] * s_u[3 * I + b];
-                    for (int a = 0; a < 3; ++a) s_G[(3 * pq + a) * NP + I] = G[a] * sq;
+                    for (int a = 0; a < 3; ++a) s_G[(3 * pq + a) * NP + I] = T(G[a] * sq);
                 }
             }
         }
@@ -366,27 +283,24 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
         for (int k = 0; k < 9; ++k)
 #pragma unroll
             for (int off = 1; off < TW_SUB; off <<= 1) ug[k] += __shfl_xor(ug[k], off, 64);
-        double* C = s_C[pq];
+        T* C = s_C[pq];
         if (ok) {
-            double F[9];
+            T F[9];
             for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) F[b + 3 * a] = ug[a + 3 * b];
-            F[0] += 1.0;
-            F[4] += 1.0;
-            F[8] += 1.0;
+                for (int b = 0; b < 3; ++b) F[b + 3 * a] = T(ug[a + 3 * b] + (a == b ? 1.0 : 0.0));
             if constexpr (MAT == MAT_SNH) {
-                const double alpha = 1.0 + mu / lambda * 0.75;
-                double I_C = 0.0;
+                const T alpha = T(1) + mu / lambda * T(0.75);
+                T I_C = T(0);
                 for (int k = 0; k < 9; ++k) I_C += F[k] * F[k];
-                const double Jf = det3(F);
-                if (Jf == 0.0) {
+                const T Jf = det3(F);
+                if (Jf == T(0)) {
                     ok = false;
                 } else {
-                    double g[9];
+                    T g[9];
                     cof3(F, g);
-                    const double beta = I_C + 1.0;
-                    const double diag = mu * (1.0 - 1.0 / beta), cf = mu * 2.0 / (beta * beta);
-                    const double scale = lambda * (Jf - alpha);
+                    const T beta = I_C + T(1);
+                    const T diag = mu * (T(1) - T(1) / beta), cf = mu * T(2) / (beta * beta);
+                    const T scale = lambda * (Jf - alpha);
                     // the 81 entries of dP/dF as nine 3 x 3 blocks, one per lane of the point
                     if (sub < 9) snh_dpdf_block(sub % 3, sub / 3, F, g, diag, cf, lambda, scale, C);
                 }
@@ -399,13 +313,13 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
         }
         if (act && !ok) {  // singular element Jacobian or deformation gradient: the point adds nothing
             if (sub == 0) atomicOr(err, KERR_SINGULAR);
-            for (int idx = sub; idx < 81; idx += TW_SUB) C[idx] = 0.0;
-            for (int k = sub; k < 3 * NP; k += TW_SUB) s_G[3 * pq * NP + k] = 0.0;
+            for (int idx = sub; idx < 81; idx += TW_SUB) C[idx] = T(0);
+            for (int k = sub; k < 3 * NP; k += TW_SUB) s_G[3 * pq * NP + k] = T(0);
         }
         __syncthreads();
         // ---- product phase: rows kk of the chunk (3 per point); rows >= 3 cnt are zero in s_G
         const int ksteps = (3 * cnt + 3) / 4;
-        double a[NT][KS];
+        T a[NT][KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
@@ -415,31 +329,38 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
             const int p = 3 * w + pp;  // pairs (0,0) (0,1) (0,2) | (1,1) (1,2) (2,2)
             const int i = p < 3 ? 0 : (p < 5 ? 1 : 2);
             const int j = p < 3 ? p : (p < 5 ? p - 2 : 2);
+            Acc* sum = acc + pp * NT * NT;
+            Acc part[NT * NT];  // FP32: the chunk's own sums, added to the others' at its end (shorter chains of roundings)
+            constexpr bool PART = sizeof(T) == 4 && !FIRST;
+            if constexpr (PART) sum = part;
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
                 if (ks == 0 || ks < ksteps) {  // a chunk has at least one point: k-step 0 always runs
                     const int kk = 4 * ks + (l >> 4), qq = kk / 3, k = kk % 3;
                     const bool live = qq < cnt;
-                    const double* Cq = s_C[live ? qq : 0];
-                    const double c0 = Cq[(3 * k + i) + 9 * j], c1 = Cq[(3 * k + i) + 9 * (3 + j)],
+                    const T* Cq = s_C[live ? qq : 0];
+                    const T c0 = Cq[(3 * k + i) + 9 * j], c1 = Cq[(3 * k + i) + 9 * (3 + j)],
                                  c2 = Cq[(3 * k + i) + 9 * (6 + j)];
 #pragma unroll
                     for (int tj = 0; tj < NT; ++tj) {
                         const int col = 16 * tj + (l & 15);
-                        double b = 0.0;
+                        T b = T(0);
                         if (live)
                             b = c0 * s_G[(3 * qq) * NP + col] + c1 * s_G[(3 * qq + 1) * NP + col] +
                                 c2 * s_G[(3 * qq + 2) * NP + col];
 #pragma unroll
                         for (int ti = 0; ti < NT; ++ti) {
                             if (i == j && ti < tj) continue;  // a diagonal pair's tile above its diagonal is never stored
-                            mf_double4& A = acc[(pp * NT + ti) * NT + tj];
-                            A = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                                a[ti][ks], b, (FIRST && ks == 0) ? mf_double4{0.0, 0.0, 0.0, 0.0} : A, 0, 0, 0);
+                            Acc& A = sum[ti * NT + tj];
+                            A = MfTile<T>::mul(a[ti][ks], b, ((FIRST || PART) && ks == 0) ? Acc{T(0), T(0), T(0), T(0)} : A);
                         }
                     }
                 }
             }
+            if constexpr (PART)
+#pragma unroll
+                for (int x = 0; x < NT * NT; ++x)
+                    if (i != j || x / NT >= x % NT) acc[pp * NT * NT + x] += part[x];
         }
         __syncthreads();
     };
@@ -448,9 +369,9 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
         for (int qc = q0 + TW_QC; qc < q1; qc += TW_QC) chunk(qc, std::false_type{});
     } else {
 #pragma unroll
-        for (int j = 0; j < JW; ++j) acc[j] = mf_double4{0.0, 0.0, 0.0, 0.0};
+        for (int j = 0; j < JW; ++j) acc[j] = Acc{T(0), T(0), T(0), T(0)};
     }
-    double* out = ke + e * (int64_t)M3 * M3;
+    T* out = ke + e * (int64_t)M3 * M3;
 #pragma unroll
     for (int jb = 0; jb < JW; ++jb) {
         const int pp = jb / (NT * NT), tile = jb % (NT * NT);
@@ -461,7 +382,7 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
         if (i == j && ti < tj) continue;  // not computed: every entry of it lies above the diagonal
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int I = 16 * ti + (4 * v + (l >> 4)), Jn = 16 * tj + (l & 15);
+            const int I = 16 * ti + MfTile<T>::row(v, l), Jn = 16 * tj + (l & 15);
             if (I < N && Jn < N && (i != j || I >= Jn)) {
                 out[(3 * I + i) * M3 + 3 * Jn + j] = acc[jb][v];
                 out[(3 * Jn + j) * M3 + 3 * I + i] = acc[jb][v];
@@ -801,25 +722,22 @@ void launch_element_forces(Model& m, double mu_r, double lambda_r, const double*
 
 void launch_element_stiffness(Model& m, double mu_r, double lambda_r, const double* u, bool fp32) {
     if (m.ne == 0) return;
+    auto run = [&](auto* ke) {
+        typedef std::remove_pointer_t<decltype(ke)> T;
+        HOEFEM_MATERIAL_DISPATCH(
+            m.material,
+            HOEFEM_DISPATCH(m.type, launch_timed(prof_slot(m), k_element_stiffness_tw<ET, T, MK>, dim3((unsigned)m.ne),
+                                                 dim3(TW_THREADS), 0, m.stream, m.ne, (const int32_t*)m.d_conn.get(),
+                                                 (const double*)m.d_vertices.get(), (const int32_t*)m.q_stiff.off.get(),
+                                                 (const double*)m.q_stiff.w.get(), (const double*)m.q_stiff.xi.get(),
+                                                 (T)m.inversion_threshold, (T)mu_r, (T)lambda_r, u, ke, m.d_err.get())));
+    };
     if (fp32) {
         m.d_ke32.ensure((size_t)m.ne * 9 * m.n * m.n);
-        HOEFEM_MATERIAL_DISPATCH(
-            m.material,
-            HOEFEM_DISPATCH(m.type,
-                            k_element_stiffness<ET, float, MK><<<dim3((unsigned)m.ne), dim3(STIFF_THREADS), 0, m.stream>>>(
-                                m.ne, m.d_conn.get(), m.d_vertices.get(), m.q_stiff.off.get(), m.q_stiff.w.get(),
-                                m.q_stiff.xi.get(), (float)m.inversion_threshold, (float)mu_r, (float)lambda_r, u,
-                                m.d_ke32.get(), m.d_err.get())));
+        run(m.d_ke32.get());
     } else {
         m.d_ke.ensure((size_t)m.ne * 9 * m.n * m.n);
-        HOEFEM_MATERIAL_DISPATCH(
-            m.material,
-            HOEFEM_DISPATCH(m.type,
-                            launch_timed(prof_slot(m), k_element_stiffness_tw<ET, MK>, dim3((unsigned)m.ne),
-                                         dim3(TW_THREADS), 0, m.stream, m.ne, (const int32_t*)m.d_conn.get(),
-                                         (const double*)m.d_vertices.get(), (const int32_t*)m.q_stiff.off.get(),
-                                         (const double*)m.q_stiff.w.get(), (const double*)m.q_stiff.xi.get(),
-                                         m.inversion_threshold, mu_r, lambda_r, u, m.d_ke.get(), m.d_err.get())));
+        run(m.d_ke.get());
     }
     check_launch("k_element_stiffness");
 }
