@@ -556,8 +556,11 @@ __global__ __launch_bounds__(GRID_THREADS) __attribute__((amdgpu_waves_per_eu(2,
 // ------------------------------------------------------------------ plan
 // W: a phase's exchange grows from 2.9 us at 8 work-groups to 5.1 us at 256 while its products shrink with
 // 1/W (about 0.13 us per block of a thread), so small systems take few work-groups: enough for
-// GRID_BLOCKS_PER_THREAD blocks per thread, at least 8, at most the CUs.
-constexpr int GRID_BLOCKS_PER_THREAD = 6;
+// GRID_BLOCKS_PER_THREAD blocks per thread, at least 8. Past GRID_WIDE work-groups the two balance over a wide
+// range of W, and a system takes no more than what still keeps its blocks on the chip
+// (GRID_BLOCKS_ON_CHIP per thread): alone it is as fast (48 to 74 thousand DOFs: -4 to +2.5 %), and two of a
+// batch fit the CUs side by side (eight scenes of 2 to 30 thousand DOFs: 139 -> 100 ms per batch step).
+constexpr int GRID_BLOCKS_PER_THREAD = 6, GRID_BLOCKS_ON_CHIP = 12, GRID_WIDE = 128;
 constexpr int GRID_MAX_SLOTS = 32;                 // bits of a thread's row-end mask
 constexpr size_t GRID_MAX_LDS = 143 * 1024;  // beside 16.3 KiB of fixed arrays
 constexpr int GRID_MAX_NODES = GRID_THREADS / 3;   // per work-group
@@ -573,7 +576,8 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
     for (int64_t v = 0; v < nn; ++v) total += ka(v) + kp(v);
     const int wmax = std::min(cus, GRID_MAX_WG);
     if (nn > (int64_t)wmax * GRID_MAX_NODES || total > (int64_t)wmax * GRID_THREADS * GRID_MAX_SLOTS) return;
-    int64_t w = (total + (int64_t)GRID_THREADS * GRID_BLOCKS_PER_THREAD - 1) / ((int64_t)GRID_THREADS * GRID_BLOCKS_PER_THREAD);
+    auto share = [&](int64_t blocks) { return (total + GRID_THREADS * blocks - 1) / (GRID_THREADS * blocks); };
+    int64_t w = std::max(share(GRID_BLOCKS_ON_CHIP), std::min<int64_t>(share(GRID_BLOCKS_PER_THREAD), GRID_WIDE));
     w = std::max<int64_t>(w, (nn + GRID_MAX_NODES - 1) / GRID_MAX_NODES);
     w = std::min<int64_t>(std::max<int64_t>((w + 7) / 8 * 8, 8), wmax);
     w = std::min(w, nn);
