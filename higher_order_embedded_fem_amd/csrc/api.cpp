@@ -1378,7 +1378,8 @@ hoefem_status hoefem_schwarz_autotune(hoefem_schwarz* s, int32_t* lanes_per_node
 // Jacobian kernel, lanes per node of the preconditioner kernel) and keeps the fastest. The
 // trial system is J = M (symmetric positive definite) with the Schwarz operator of M and
 // tolerance 0, so every trial runs exactly the same number of full iterations. J and P are
-// overwritten; the next step assembles them again.
+// overwritten; the next step assembles them again. The trials run the two-kernel iteration, the one whose
+// kernels have lanes per node (the resident grid has none, and serves the systems it fits whatever is chosen).
 static void sim_autotune_cg(Sim& s, int* ga_out, int* gb_out, double* candidate_us) {
     Model& m = *s.model;
     const int64_t n = 3 * m.nv, nnz = m.pattern.nnz();
@@ -1390,6 +1391,12 @@ static void sim_autotune_cg(Sim& s, int* ga_out, int* gb_out, double* candidate_
         if (s.schwarz) schwarz_update(*s.schwarz, s.d_J.get());
     }
     launch_fill(m, s.d_F.get(), n, 1.0);
+    struct TwoKernels {
+        CgWork& w;
+        const bool before = w.use_grid;
+        explicit TwoKernels(CgWork& work) : w(work) { w.use_grid = false; }
+        ~TwoKernels() { w.use_grid = before; }
+    } two_kernels(s.cg);
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
