@@ -1,9 +1,9 @@
 """Many independent scenes advanced together on one GPU (hoefem_batch_step).
 
-The scenes' Newton loops run in lockstep from one host thread: each round issues every scene's
-residual evaluations, Jacobian assemblies or line-search trials before one synchronization, and
-the round's linear solves run as one batched Schwarz-PCG whose launches cover all scenes, each
-scene stopping on the device when it converges; iteration batches are captured HIP graphs. Each
+One host thread drives every scene's Newton loop, no scene waiting for another: residual evaluations,
+Jacobian assemblies and line-search trials go to the scene's stream, and the linear solves that are
+ready share launches (resident grids side by side, or batched two-kernel iterations for the systems
+that do not fit), each scene stopping on the device when it converges. Each
 scene keeps its own model and tile shapes (lanes per node row of J and of P, picked by the
 library's autotuner); the models are spread round robin over a few streams so the per-scene
 assembly kernels of different scenes overlap. Every scene's result equals what stepping it alone

@@ -217,8 +217,9 @@ hoefem_status hoefem_pcg(hoefem_model* model, const double* A_values, hoefem_sch
 
 /* hoefem_pcg without allocation. No counterpart in the reference: for callers that cannot
  * allocate device or pinned memory during a solve (serving loops, harnesses that forbid it, code
- * that runs under stream capture nearby). Same kernels, arguments and results as hoefem_pcg; the
- * work buffers live in a fixed per-GPU array of 18.9 MB held until the process ends, so the model
+ * that runs under stream capture nearby). Same kernels, arguments and results as hoefem_pcg: a system
+ * that fits the resident grid uses the buffers its model and preconditioner allotted when they were
+ * created, the others a fixed per-GPU array of 18.9 MB held until the process ends. The model
  * may have at most 262144 DOFs (larger models: HOEFEM_ERROR_INVALID_ARGUMENT) and the model must use
  * device pointers. Runs on the model's stream and synchronizes it. Calls that overlap in time on
  * one GPU share that array and race; serialize them. FP64 operators only. */
@@ -243,7 +244,7 @@ hoefem_status hoefem_sim_autotune(hoefem_sim* sim, int32_t* lanes_matrix, int32_
 /* Kernel timing (no counterpart in the reference, which times phases with coarse_prof scopes,
  * simulation_toolbox/src/fem/newton_cg.rs:685-764): when enabled, every launch of the CG
  * system-matrix kernel (fused direction update + SpMV + p.Ap) is bracketed by HIP events on
- * the model stream. "full" launches performed a CG iteration; the remaining launches found
+ * the model stream (solves then run the two-kernel iteration, not the resident grid). "full" launches performed a CG iteration; the remaining launches found
  * the solve already finished and returned immediately. */
 hoefem_status hoefem_profile_enable(hoefem_model* model, int32_t enable);
 hoefem_status hoefem_profile_read(hoefem_model* model, int64_t* full_launches, double* full_ms,
@@ -336,11 +337,10 @@ hoefem_status hoefem_sim_set_dirichlet_values(hoefem_sim* sim, const double* u_v
 /* ------------------------------------------------------------------ batched scenes
  * No counterpart in the reference, which steps one scene per process (integrate_model_with_substeps,
  * simulation_toolbox/src/fem/newton_cg.rs:146-228). A batch steps independent sims (each its own
- * model, material and boundary conditions) together: their Newton loops run in lockstep, their
- * residual evaluations, assemblies and line-search trials are issued before one synchronization per
- * round, and each round's linear solves run as one batched PCG whose scenes stop on the device as
- * they converge. Every scene's u and v equal what hoefem_sim_step gives it, bit for bit (a scene
- * whose single-step attempt fails continues alone with hoefem_sim_step's substepping). The sims
+ * model, material and boundary conditions) together: one host thread drives every
+ * scene's Newton loop, no scene waiting for another, and the linear solves that are ready share
+ * launches, each stopping on the device as it converges. Every scene's u and v equal what
+ * hoefem_sim_step gives it, bit for bit (a scene whose single-step attempt fails continues alone with hoefem_sim_step's substepping). The sims
  * must outlive the batch, take device pointers, have no learned correction attached and share one
  * precision mode (FP64, or mixed_precision 1); their models may use different streams. */
 typedef struct hoefem_batch hoefem_batch;
