@@ -186,9 +186,16 @@ struct MfTile<float> {
 //    (i, j) = (w, w..2) for w = 0 and (1, 1), (1, 2), (2, 2) for w = 1, with the B operand
 //    U^{ij}(kk, col) = sum_m C_q(3k + i, 3m + j) G~(3q + m, col) formed in registers at each k-step
 //    (no U staging in LDS); a diagonal pair skips its tile above the diagonal.
-// FP32 tangents of the 24-cell Hex20 cylinder take 60 us, with vector FMAs over K_e's entries 82 us, at
+// FP32 tangents of the 24-cell Hex20 cylinder take 49 us, with vector FMAs over K_e's entries 82 us, at
 // 1.1 to 3 times its error against FP64 (2.9e-7 of the norm on 20 cells, now 0.9e-7).
 constexpr int TW_QC = 8, TW_THREADS = 128, TW_SUB = TW_THREADS / TW_QC;
+
+// orders a wavefront's LDS accesses before and after it (the hardware executes them in order)
+__device__ inline void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // Waves per SIMD that the registers are allotted for: as many as the accumulators (12 tiles per wavefront in the
 // elements above 16 nodes) and the per-point phase leave without much spilling. Tet10, FP64, 10,368 elements:
@@ -372,6 +379,13 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(
         for (int j = 0; j < JW; ++j) acc[j] = Acc{T(0), T(0), T(0), T(0)};
     }
     T* out = ke + e * (int64_t)M3 * M3;
+    // FP32: a tile's transpose goes through LDS (s_C, no longer read), so that both copies are stored along rows of K_e
+    // (24-cell Hex20 cylinder 49 us; 60 us stored column by column, a memory request per entry). In FP64 the
+    // products hide the requests and the trip costs more than it gives (36-cell Hex27: 546 against 536 us).
+    constexpr bool BY_ROWS = sizeof(T) == 4;
+    constexpr int LT = 17;
+    static_assert(2 * 16 * LT <= TW_QC * 81, "a tile per wavefront");
+    T* tr = &s_C[0][0] + w * 16 * LT;
 #pragma unroll
     for (int jb = 0; jb < JW; ++jb) {
         const int pp = jb / (NT * NT), tile = jb % (NT * NT);
@@ -382,12 +396,23 @@ __global__ __launch_bounds__(TW_THREADS) __attribute__((amdgpu_waves_per_eu(
         if (i == j && ti < tj) continue;  // not computed: every entry of it lies above the diagonal
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int I = 16 * ti + MfTile<T>::row(v, l), Jn = 16 * tj + (l & 15);
+            const int r = MfTile<T>::row(v, l), c = l & 15;
+            const int I = 16 * ti + r, Jn = 16 * tj + c;
+            if constexpr (BY_ROWS) tr[r * LT + c] = acc[jb][v];
             if (I < N && Jn < N && (i != j || I >= Jn)) {
                 out[(3 * I + i) * M3 + 3 * Jn + j] = acc[jb][v];
-                out[(3 * Jn + j) * M3 + 3 * I + i] = acc[jb][v];
+                if constexpr (!BY_ROWS) out[(3 * Jn + j) * M3 + 3 * I + i] = acc[jb][v];
             }
         }
+        if constexpr (!BY_ROWS) continue;
+        wave_lds_fence();
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = l & 15, c = 4 * v + (l >> 4);
+            const int I = 16 * ti + r, Jn = 16 * tj + c;
+            if (I < N && Jn < N && (i != j || I >= Jn)) out[(3 * Jn + j) * M3 + 3 * I + i] = tr[r * LT + c];
+        }
+        wave_lds_fence();
     }
 }
 
