@@ -712,7 +712,7 @@ static void batch_step(Batch& B, const double* dt, double* const* u, double* con
         const int64_t ndof = 3 * s.model->nv;
         int c = 0;
         while (c < BATCH_POOLS - 1 && ndof >= BATCH_POOL_DOFS[c]) ++c;
-        if ((s.schwarz ? s.schwarz->grid : s.model->grid).W) c = BATCH_POOLS;  // the resident grid's
+        if ((s.schwarz ? s.schwarz->grid : s.model->grid).serves(s.model->pattern)) c = BATCH_POOLS;  // the resident grid's
         pool_of[i] = c;
         pool_size[c] += 1;
     }

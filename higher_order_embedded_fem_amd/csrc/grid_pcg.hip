@@ -568,6 +568,7 @@ constexpr int GRID_SPARE = 8;                      // spare partial sums (row_su
 
 void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStream_t s) {
     W = 0;
+    matrix = J.id;
     const int64_t nn = J.num_nodes;
     if (nn == 0 || cus < 8) return;
     auto ka = [&](int64_t v) { return J.nptr[v + 1] - J.nptr[v]; };

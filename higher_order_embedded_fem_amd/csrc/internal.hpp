@@ -101,7 +101,10 @@ struct __align__(16) NodeEntry {
     int32_t node, first, count, rowoff;
 };
 
+uint64_t next_pattern_id();  // never the same twice in a process
+
 struct NodePattern {
+    uint64_t id = next_pattern_id();
     int64_t num_nodes = 0;
     std::vector<int32_t> nptr, ncol;  // node-level neighbour lists, sorted
     std::vector<int32_t> rowptr, col; // DOF-level CSR
@@ -206,6 +209,7 @@ struct GridResult {              // pinned: written by the kernel
 // How a matrix pattern (and its preconditioner's) is split over the grid, with the buffers of a solve.
 // W == 0: the system does not fit and takes the two-kernel path.
 struct GridPlan {
+    uint64_t matrix = 0;  // id of the matrix pattern it splits
     int W = 0, max_slots = 0, nlds = 0, blk_off = 0;
     uint32_t phase = 0;
     int64_t ndof = 0;
@@ -219,6 +223,8 @@ struct GridPlan {
     DevBuf<GridState> d_state;
     std::unique_ptr<PinnedBuf<GridResult>> host;
     void build(const NodePattern& J, const NodePattern* P, int cus, hipStream_t s);
+    // the plan is for this matrix pattern (a preconditioner may come from another model's) and fits the chip
+    bool serves(const NodePattern& J) const { return W > 0 && matrix == J.id; }
     void reset(hipStream_t s);  // after a failed launch
 };
 int grid_device_cus();

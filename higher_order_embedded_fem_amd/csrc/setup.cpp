@@ -1,6 +1,7 @@
 // Host-side setup of the hoefem library: node-level CSR patterns, first-fit coloring and
 // the color-ordered block incidence used by the atomic-free gather kernels.
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <numeric>
@@ -95,6 +96,11 @@ void NodePattern::upload(hipStream_t s) {
         if (diag_only[v]) entries.push_back(NodeEntry{(int32_t)v, 0, 0, rowptr[3 * v]});
     n_diag = (int64_t)entries.size() - n_block;
     d_entries.upload(entries, s);
+}
+
+uint64_t next_pattern_id() {
+    static std::atomic<uint64_t> next{1};
+    return next.fetch_add(1, std::memory_order_relaxed);
 }
 
 // The set of node pairs of every node set, expanded to 3x3 blocks, sorted by row and column:

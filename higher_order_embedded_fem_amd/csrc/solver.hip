@@ -1173,11 +1173,18 @@ static void cg_launch_all(Model& m, CgWork& w, const Csr3<VT>& A, const Csr3<VT>
     }
 }
 
+// A preconditioner made on another model serves any matrix over as many nodes
+static void check_preconditioner(const NodePattern& A, const Schwarz* P) {
+    if (P && P->P.num_nodes != A.num_nodes)
+        throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "the preconditioner's model has another number of nodes");
+}
+
 template <class VT>
 static hoefem_status pcg_solve_t(Model& m, CgWork& w, const VT* Avals, const VT* Pvals, Schwarz* Pre, const double* b,
                                  double* x, double tol, int64_t max_iter, int64_t* iterations, CgHarvest* h = nullptr,
                                  const LearnedView* lv = nullptr) {
     const NodePattern& pat = m.pattern;
+    check_preconditioner(pat, Pre);
     const int64_t nn = pat.num_nodes;
     const int GA = spmv_group_size(pat);
     const int GB = Pre ? spmv_group_size(Pre->P) : 8;
@@ -1197,10 +1204,11 @@ static hoefem_status pcg_solve_t(Model& m, CgWork& w, const VT* Avals, const VT*
     if (FLEX && JAC) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "the learned correction needs the Schwarz preconditioner");
     if (FLEX && (lv->na < 1 || lv->na > CG_MAX_BLOCKS))
         throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "number of aggregates out of range");
-    // the resident grid takes every plain solve that fits it; per-iteration hooks (kernel timing, snapshots)
-    // and the flexible variant keep the two kernels
+    // the resident grid takes every plain solve that fits it; per-iteration hooks (kernel timing, snapshots),
+    // the flexible variant and a preconditioner of another model, whose plan splits that model's matrix, keep
+    // the two kernels
     GridPlan& grid = Pre ? Pre->grid : m.grid;
-    if (grid.W && !FLEX && !h && !m.prof && w.use_grid &&
+    if (grid.serves(pat) && !FLEX && !h && !m.prof && w.use_grid &&
         grid_solve<VT>(grid, m, Avals, Pre, Pre ? nullptr : w.diag_inv.get(), b, x, tol, max_iter, iterations, &st))
         return st;
 #define CG_CASE(ga, gb, j, f)                                                                            \
@@ -1332,6 +1340,7 @@ hoefem_status pcg_solve_noalloc(Model& m, const double* Avals, Schwarz* Pre, con
                                                        std::to_string(NOALLOC_MAX_DOFS) + " DOFs (model has " +
                                                        std::to_string(pat.ndof()) + ")");
     if (Pre && Pre->fp32) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "FP32 preconditioner with an FP64 operator");
+    check_preconditioner(pat, Pre);
     if (pat.num_nodes == 0) return HOEFEM_OK;
     double* base = scratch_address();
     const int GA = spmv_group_size(pat);
@@ -1346,7 +1355,7 @@ hoefem_status pcg_solve_noalloc(Model& m, const double* Avals, Schwarz* Pre, con
     }
     GridPlan& grid = Pre ? Pre->grid : m.grid;
     hoefem_status st = HOEFEM_OK;
-    if (grid.W && grid_solve<double>(grid, m, Avals, Pre, Pre ? nullptr : base + NA_DIAG, b, x, tol, max_iter, iterations, &st))
+    if (grid.serves(pat) && grid_solve<double>(grid, m, Avals, Pre, Pre ? nullptr : base + NA_DIAG, b, x, tol, max_iter, iterations, &st))
         return st;
 #define NA_CASE(ga, gb, j) \
     if (GA == ga && GB == gb && (Pre == nullptr) == j) return cg_launch_noalloc<ga, gb, j>(m, base, A, Pm, b, x, tol, max_iter, iterations);

@@ -210,7 +210,8 @@ hoefem_status hoefem_schwarz_apply(hoefem_schwarz* s, const double* x, double* y
 
 /* ConjugateGradient::solve_with_guess (fenris/src/cg.rs:377-482) with the relative residual
  * criterion (:85-124). A has the model pattern (device values); the preconditioner is the
- * Schwarz operator, or the Jacobi diagonal of A when schwarz == NULL. b, x: device.
+ * Schwarz operator (of this model or of another with as many nodes; with another number:
+ * HOEFEM_ERROR_INVALID_ARGUMENT), or the Jacobi diagonal of A when schwarz == NULL. b, x: device.
  * Returns HOEFEM_ERROR_CG_* for the SolveErrorKind cases; *iterations is always written. */
 hoefem_status hoefem_pcg(hoefem_model* model, const double* A_values, hoefem_schwarz* schwarz, const double* b,
                          double* x, double tolerance, int64_t max_iterations, int64_t* iterations);

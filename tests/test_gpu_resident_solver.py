@@ -1,0 +1,85 @@
+"""Which systems the resident-grid PCG may take, and what becomes of the others."""
+
+import ctypes as C
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle as O
+from higher_order_embedded_fem_amd import _lib, scenes
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def dev(x):
+    return torch.as_tensor(np.ascontiguousarray(x), dtype=torch.float64, device="cuda")
+
+
+def matrix(sc, stiff=1e-5):
+    om = O.Model(sc)
+    mu, lam = scenes.lame_from_young_poisson(sc.young, sc.poisson)
+    rp, col = om.pattern()
+    K = om.stiffness_add(mu, lam, np.zeros(sc.ndof), np.zeros(om.nnz))
+    return rp, col, O.dirichlet_csr(rp, col, (0.0 + stiff * K) + 1.0 * om.mass(sc.density), sc.dirichlet_nodes)
+
+
+def system(sc, seed):
+    """The scene's matrix M + 1e-5 K on the device, a solution and its right-hand side."""
+    rp, col, J = matrix(sc)
+    x = np.random.default_rng(seed).standard_normal(sc.ndof)
+    y = J * x[col]
+    return dev(J), x, dev(np.add.reduceat(np.concatenate([y, [0.0]]), rp[:-1]))
+
+
+def thinned(sc):
+    """The scene without every other element that its nodes can spare: the same nodes, fewer couplings."""
+    count = np.bincount(sc.connectivity.ravel(), minlength=sc.num_vertices)
+    keep = np.ones(sc.num_elements, bool)
+    for e in range(0, sc.num_elements, 2):
+        if (count[sc.connectivity[e]] > 1).all():
+            count[sc.connectivity[e]] -= 1
+            keep[e] = False
+    conn = np.ascontiguousarray(sc.connectivity[keep])
+    off = np.arange(0, conn.size + 1, conn.shape[1], dtype=np.int64)
+    return dataclasses.replace(sc, connectivity=conn, num_interior=len(conn), subdomain_offsets=off,
+                               subdomain_nodes=conn.ravel().astype(np.int32),
+                               untreated_nodes=np.zeros(0, np.int32))
+
+
+# Both directions: rows shorter and longer than the preconditioner's model has them. The solve's residual of 1e-13
+# times the mass-dominated matrix's condition (Jacobi-scaled at most about 1e4) bounds the error by 1e-9.
+@pytest.mark.parametrize("cells,element", [(3, scenes.TET10), (9, scenes.TET4)])
+@pytest.mark.parametrize("own_thinned", [False, True])
+@pytest.mark.parametrize("entry", ["hoefem_pcg", "hoefem_pcg_noalloc"])
+def test_preconditioner_of_another_model_on_the_same_nodes(cells, element, own_thinned, entry):
+    from higher_order_embedded_fem_amd import fem
+
+    full = scenes.cube_scene(cells, element)
+    part = thinned(full)
+    assert part.num_elements < 0.8 * full.num_elements
+    own, other = (part, full) if own_thinned else (full, part)
+    Jd, x_true, b = system(own, cells)
+    gm, gother = fem.ElasticityModel(own), fem.ElasticityModel(other)
+    pre = fem.SchwarzPreconditioner.from_scene(gother, other)
+    pre.update(dev(matrix(other)[2]))
+    solve = getattr(_lib.load(), entry)
+    x, its = torch.zeros_like(b), C.c_int64()
+    assert solve(gm.h, Jd.data_ptr(), pre.h, b.data_ptr(), x.data_ptr(), 1e-13, 20000, C.byref(its)) == 0
+    assert np.linalg.norm(x.cpu().numpy() - x_true) <= 1e-9 * np.linalg.norm(x_true)
+
+
+@pytest.mark.parametrize("entry", ["hoefem_pcg", "hoefem_pcg_noalloc"])
+def test_preconditioner_of_another_size_is_refused(entry):
+    from higher_order_embedded_fem_amd import fem
+
+    small, large = scenes.cube_scene(2, scenes.TET10), scenes.cube_scene(3, scenes.TET10)
+    Jd, _, b = system(large, 1)
+    gm, gsmall = fem.ElasticityModel(large), fem.ElasticityModel(small)
+    pre = fem.SchwarzPreconditioner.from_scene(gsmall, small)
+    L = _lib.load()
+    x, its = torch.zeros_like(b), C.c_int64()
+    assert getattr(L, entry)(gm.h, Jd.data_ptr(), pre.h, b.data_ptr(), x.data_ptr(), 1e-8, 10, C.byref(its)) == 1
+    assert b"nodes" in L.hoefem_last_error()
