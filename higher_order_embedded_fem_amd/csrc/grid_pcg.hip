@@ -565,6 +565,7 @@ constexpr int GRID_MAX_SLOTS = 32;                 // bits of a thread's row-end
 constexpr size_t GRID_MAX_LDS = 143 * 1024;  // beside 16.3 KiB of fixed arrays
 constexpr int GRID_MAX_NODES = GRID_THREADS / 3;   // per work-group
 constexpr int GRID_SPARE = 8;                      // spare partial sums (row_sum)
+constexpr int64_t GRID_STATE_WORDS = (sizeof(GridState) + 255) / 256 * 32;
 
 void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStream_t s) {
     W = 0;
@@ -707,9 +708,9 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
     }
     std::vector<int32_t> halo;
     std::vector<uint16_t> col, rp;
-    size_t ws = 0;
     lds_bytes = 0;
     max_slots = 0;
+    ws = 0;
     for (int64_t b = 0; b < w; ++b) {
         GridWg& g = wg[b];
         const Part& o = part[b];
@@ -739,14 +740,53 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
     d_col.upload(col, s);
     d_rp.upload(rp, s);
     d_start.upload(start, s);
-    d_ws.ensure(ws);
-    d_save.ensure((size_t)3 * 3 * nn);
-    d_state.ensure(1);
-    host.reset(new PinnedBuf<GridResult>(1, hipHostMallocCoherent));
-    *host->p = GridResult{};
     ndof = 3 * nn;
     W = (int)w;
-    reset(s);
+    if (exchange() + saved() + GRID_STATE_WORDS + (int64_t)ws > GRID_SCRATCH) d_spill.ensure(ws);
+}
+
+int64_t GridPlan::exchange() const { return (int64_t)8 * GRID_COPIES * W + 4 * ndof; }
+
+void GridWork::ensure(const GridPlan& g) {
+    if (W_ != g.W || ndof_ != g.ndof) {
+        d_slots_.ensure((size_t)g.exchange());
+        d_save_.ensure((size_t)g.saved());
+        W_ = g.W;
+        ndof_ = g.ndof;
+        cleared = false;
+    }
+    d_ws_.ensure(g.ws);
+    d_state_.ensure(1);
+    if (!host_) host_.reset(new PinnedBuf<GridResult>(1, hipHostMallocCoherent));
+    slots = d_slots_.get();
+    save = d_save_.get();
+    ws = d_ws_.get();
+    state = d_state_.get();
+    result = host_->p;
+}
+
+GridBuffers grid_scratch_buffers(const GridPlan& g, double* scratch, GridResult* result) {
+    GridBuffers w;
+    w.slots = reinterpret_cast<unsigned long long*>(scratch);
+    w.save = scratch + g.exchange();
+    w.state = reinterpret_cast<GridState*>(w.save + g.saved());
+    w.ws = g.d_spill.n ? g.d_spill.get() : w.save + g.saved() + GRID_STATE_WORDS;
+    w.result = result;
+    return w;
+}
+
+__global__ void k_grid_clear(int64_t n, unsigned long long* __restrict__ p) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = GRID_EMPTY;
+}
+
+void grid_clear(const GridPlan& g, GridBuffers& w, hipStream_t s) {
+    if (w.cleared) return;
+    const int64_t n = g.exchange();
+    k_grid_clear<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(n, w.slots);
+    check_launch("k_grid_clear");
+    w.phase = 0;
+    w.cleared = true;
 }
 
 // ------------------------------------------------------------------ admission
@@ -814,8 +854,8 @@ void GridSlots::release() {
 
 // ------------------------------------------------------------------ launches
 template <class VT>
-GridSeg<VT> grid_segment(const GridPlan& g, Model& m, const VT* A, const Schwarz* P, const double* dinv,
-                         const double* b, double* x, double tol, int64_t max_iter) {
+GridSeg<VT> grid_segment(const GridPlan& g, const GridBuffers& w, Model& m, const VT* A, const Schwarz* P,
+                         const double* dinv, const double* b, double* x, double tol, int64_t max_iter) {
     GridSeg<VT> S{};
     S.wg = g.d_wg.get();
     S.halo = g.d_halo.get();
@@ -838,24 +878,24 @@ GridSeg<VT> grid_segment(const GridPlan& g, Model& m, const VT* A, const Schwarz
     }
     S.b = b;
     S.x = x;
-    S.vec = reinterpret_cast<double*>(g.d_slots.get() + (size_t)8 * GRID_COPIES * g.W);
-    S.save = g.d_save.get();
+    S.vec = reinterpret_cast<double*>(w.slots + (size_t)8 * GRID_COPIES * g.W);
+    S.save = w.save;
     S.ndof = g.ndof;
-    S.ws = reinterpret_cast<VT*>(g.d_ws.get());
-    S.slots = g.d_slots.get();
-    S.state = g.d_state.get();
-    S.host = g.host->p;
+    S.ws = reinterpret_cast<VT*>(w.ws);
+    S.slots = w.slots;
+    S.state = w.state;
+    S.host = w.result;
     S.W = g.W;
-    S.phase = g.phase;
+    S.phase = w.phase;
     S.nlds = g.nlds;
     S.blk_off = g.blk_off;
     S.tol = tol;
     S.max_iter = max_iter;
     return S;
 }
-template GridSeg<double> grid_segment<double>(const GridPlan&, Model&, const double*, const Schwarz*, const double*,
+template GridSeg<double> grid_segment<double>(const GridPlan&, const GridBuffers&, Model&, const double*, const Schwarz*, const double*,
                                               const double*, double*, double, int64_t);
-template GridSeg<float> grid_segment<float>(const GridPlan&, Model&, const float*, const Schwarz*, const double*,
+template GridSeg<float> grid_segment<float>(const GridPlan&, const GridBuffers&, Model&, const float*, const Schwarz*, const double*,
                                             const double*, double*, double, int64_t);
 
 template <class VT>
@@ -874,14 +914,15 @@ template void grid_launch<double, GRID_SEGS>(const GridSegs<double, GRID_SEGS>&,
 template void grid_launch<float, GRID_SEGS>(const GridSegs<float, GRID_SEGS>&, int, size_t, hipStream_t);
 
 template <class VT>
-bool grid_solve(GridPlan& g, Model& m, const VT* A, const Schwarz* P, const double* dinv, const double* b, double* x,
-                double tol, int64_t max_iter, int64_t* iterations, hoefem_status* status) {
+bool grid_solve(const GridPlan& g, GridBuffers& w, Model& m, const VT* A, const Schwarz* P, const double* dinv,
+                const double* b, double* x, double tol, int64_t max_iter, int64_t* iterations, hoefem_status* status) {
     GridSegs<VT, 1> all;
     GridSeg<VT>& S = all.seg[0];
-    S = grid_segment<VT>(g, m, A, P, dinv, b, x, tol, max_iter);
+    grid_clear(g, w, m.stream);
+    S = grid_segment<VT>(g, w, m, A, P, dinv, b, x, tol, max_iter);
     S.chunk = GRID_CHUNK;
     while (true) {
-        volatile GridResult* h = g.host->p;
+        volatile GridResult* h = w.result;
         h->status = GRID_RUNNING;
         h->failed = 0;
         {
@@ -891,22 +932,22 @@ bool grid_solve(GridPlan& g, Model& m, const VT* A, const Schwarz* P, const doub
             HIP_CHECK(hipStreamSynchronize(m.stream));
         }
         if (h->failed) {
-            g.reset(m.stream);
+            w.cleared = false;
             return false;
         }
-        g.phase = S.phase = h->phase;
+        w.phase = S.phase = h->phase;
         *iterations = h->iters;
         if (h->status != GRID_RUNNING) break;
         S.resume = 1;
     }
-    const int st = g.host->p->status;
+    const int st = w.result->status;
     *status = st == GRID_CONVERGED || st == GRID_ZERO_RHS ? HOEFEM_OK : (hoefem_status)st;
     return true;
 }
-template bool grid_solve<double>(GridPlan&, Model&, const double*, const Schwarz*, const double*, const double*,
-                                 double*, double, int64_t, int64_t*, hoefem_status*);
-template bool grid_solve<float>(GridPlan&, Model&, const float*, const Schwarz*, const double*, const double*,
-                                double*, double, int64_t, int64_t*, hoefem_status*);
+template bool grid_solve<double>(const GridPlan&, GridBuffers&, Model&, const double*, const Schwarz*,
+                                 const double*, const double*, double*, double, int64_t, int64_t*, hoefem_status*);
+template bool grid_solve<float>(const GridPlan&, GridBuffers&, Model&, const float*, const Schwarz*,
+                                const double*, const double*, double*, double, int64_t, int64_t*, hoefem_status*);
 
 // ------------------------------------------------------------------ many systems
 GridBatch::~GridBatch() {
@@ -927,7 +968,8 @@ template <class VT>
 struct GridPoolT final : CgPool {
     struct Item {
         CgBatchSystem q;
-        GridPlan* g;
+        const GridPlan* g;
+        GridWork* w;
         GridSeg<VT> seg;
     };
     GridBatch& B;
@@ -948,11 +990,12 @@ struct GridPoolT final : CgPool {
             if (!running[l].empty()) (void)hipStreamSynchronize(B.lanes[l].s);
     }
     int join(const CgBatchSystem& q) override {
-        Item it{q, q.P ? &q.P->grid : &q.m->grid, {}};
+        Item it{q, q.P ? &q.P->grid : &q.m->grid, &q.w->grid, {}};
+        it.w->ensure(*it.g);
         it.q.iterations = 0;
         it.q.status = HOEFEM_OK;
-        it.seg = grid_segment<VT>(*it.g, *q.m, (const VT*)q.A, q.P, q.P ? nullptr : q.w->diag_inv.get(), q.b, q.x, q.tol,
-                                  q.max_iter);
+        it.seg = grid_segment<VT>(*it.g, *it.w, *q.m, (const VT*)q.A, q.P, q.P ? nullptr : q.w->diag_inv.get(), q.b, q.x,
+                                  q.tol, q.max_iter);
         it.seg.chunk = GRID_BATCH_CHUNK;
         items.push_back(it);
         waiting.push_back((int)items.size() - 1);
@@ -969,9 +1012,9 @@ struct GridPoolT final : CgPool {
         std::vector<int> again;
         for (int id : running[lane]) {
             Item& it = items[id];
-            volatile GridResult* h = it.g->host->p;
+            volatile GridResult* h = it.w->result;
             if (h->failed) {  // solved from the start by the two kernels
-                it.g->reset(B.lanes[lane].s);
+                it.w->cleared = false;
                 HIP_CHECK(hipMemsetAsync(it.q.x, 0, sizeof(double) * it.g->ndof, it.q.m->stream));
                 it.q.w->use_grid = false;
                 it.q.status = pcg_solve(*it.q.m, *it.q.w, (const VT*)it.q.A, it.q.P, it.q.b, it.q.x, it.q.tol,
@@ -981,7 +1024,7 @@ struct GridPoolT final : CgPool {
                 ended.push_back(id);
                 continue;
             }
-            it.g->phase = it.seg.phase = h->phase;
+            it.w->phase = h->phase;
             if (h->status == GRID_RUNNING) {
                 it.seg.resume = 1;
                 again.push_back(id);
@@ -1015,11 +1058,12 @@ struct GridPoolT final : CgPool {
             const hipStream_t s = B.lanes[l].s;
             for (int k = 0; k < n; ++k) {
                 Item& it = items[waiting[k]];
-                volatile GridResult* h = it.g->host->p;
+                volatile GridResult* h = it.w->result;
                 h->status = GRID_RUNNING;
                 h->failed = 0;
                 if (!it.seg.resume) HIP_CHECK(hipMemsetAsync(it.q.x, 0, sizeof(double) * it.g->ndof, s));
-                it.seg.phase = it.g->phase;
+                grid_clear(*it.g, *it.w, s);
+                it.seg.phase = it.w->phase;
                 all.seg[k] = it.seg;
                 lds = std::max(lds, it.g->lds_bytes);
                 running[l].push_back(waiting[k]);
@@ -1035,19 +1079,6 @@ struct GridPoolT final : CgPool {
 std::unique_ptr<CgPool> make_grid_pool(GridBatch& B, bool fp32) {
     if (fp32) return std::unique_ptr<CgPool>(new GridPoolT<float>(B));
     return std::unique_ptr<CgPool>(new GridPoolT<double>(B));
-}
-
-__global__ void k_grid_clear(int64_t n, unsigned long long* __restrict__ p) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = GRID_EMPTY;
-}
-
-void GridPlan::reset(hipStream_t s) {
-    const int64_t n = (int64_t)8 * GRID_COPIES * W + 4 * ndof;
-    d_slots.ensure((size_t)n);
-    k_grid_clear<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(n, d_slots.get());
-    check_launch("k_grid_clear");
-    phase = 0;
 }
 
 }  // namespace hoefem

@@ -65,13 +65,19 @@ private:
 int grid_free_cus();  // CUs of the current device not held
 
 template <class VT>
-GridSeg<VT> grid_segment(const GridPlan& g, Model& m, const VT* A, const Schwarz* P, const double* dinv,
-                         const double* b, double* x, double tol, int64_t max_iter);
+GridSeg<VT> grid_segment(const GridPlan& g, const GridBuffers& w, Model& m, const VT* A, const Schwarz* P,
+                         const double* dinv, const double* b, double* x, double tol, int64_t max_iter);
+// One launch; the systems' buffers must be clear (grid_clear) before it on the same stream
 template <class VT, int K>
 void grid_launch(const GridSegs<VT, K>& all, int wgs, size_t lds, hipStream_t s);
+void grid_clear(const GridPlan& g, GridBuffers& w, hipStream_t s);
 // Solves A x = b on the model stream; false: the grid could not run (x is a valid guess for another solver)
 template <class VT>
-bool grid_solve(GridPlan& g, Model& m, const VT* A, const Schwarz* P, const double* dinv, const double* b, double* x,
-                double tol, int64_t max_iter, int64_t* iterations, hoefem_status* status);
+bool grid_solve(const GridPlan& g, GridBuffers& w, Model& m, const VT* A, const Schwarz* P, const double* dinv,
+                const double* b, double* x, double tol, int64_t max_iter, int64_t* iterations, hoefem_status* status);
+
+// Buffers of allocation-free solves in a scratch of GRID_SCRATCH doubles
+constexpr int64_t GRID_SCRATCH = 8 * 262144;
+GridBuffers grid_scratch_buffers(const GridPlan& g, double* scratch, GridResult* result);
 
 }  // namespace hoefem

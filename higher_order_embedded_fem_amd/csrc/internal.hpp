@@ -206,26 +206,43 @@ struct GridResult {              // pinned: written by the kernel
     uint32_t phase, pad;
     int64_t iters;
 };
-// How a matrix pattern (and its preconditioner's) is split over the grid, with the buffers of a solve.
-// W == 0: the system does not fit and takes the two-kernel path.
+// How a matrix pattern (and its preconditioner's) is split over the grid. Not written after it is built, so solves
+// that run beside each other may share it. W == 0: the system does not fit and takes the two-kernel path.
 struct GridPlan {
     uint64_t matrix = 0;  // id of the matrix pattern it splits
     int W = 0, max_slots = 0, nlds = 0, blk_off = 0;
-    uint32_t phase = 0;
     int64_t ndof = 0;
-    size_t lds_bytes = 0;
+    size_t lds_bytes = 0, ws = 0;  // ws: doubles for the blocks past the registers and the LDS
     DevBuf<GridWg> d_wg;
     DevBuf<int32_t> d_halo;
     DevBuf<uint16_t> d_col, d_rp;
     DevBuf<GridStart> d_start;
-    DevBuf<double> d_ws, d_save;
-    DevBuf<unsigned long long> d_slots;  // partial sums, then the exchanged vectors (four sets each)
-    DevBuf<GridState> d_state;
-    std::unique_ptr<PinnedBuf<GridResult>> host;
+    DevBuf<double> d_spill;  // those blocks in allocation-free solves, where that path's scratch is too small
     void build(const NodePattern& J, const NodePattern* P, int cus, hipStream_t s);
     // the plan is for this matrix pattern (a preconditioner may come from another model's) and fits the chip
     bool serves(const NodePattern& J) const { return W > 0 && matrix == J.id; }
-    void reset(hipStream_t s);  // after a failed launch
+    int64_t exchange() const;                        // 64-bit words of partial sums and exchanged vectors (four sets each)
+    int64_t saved() const { return 3 * ndof; }       // doubles kept between launches
+};
+// The buffers of one solve at a time
+struct GridBuffers {
+    unsigned long long* slots = nullptr;  // partial sums, then the exchanged vectors
+    double *save = nullptr, *ws = nullptr;
+    GridState* state = nullptr;
+    GridResult* result = nullptr;
+    uint32_t phase = 0;    // exchanges done so far
+    bool cleared = false;  // slots hold what phase says; else the next launch clears them first
+};
+struct GridWork : GridBuffers {
+    void ensure(const GridPlan& g);
+
+private:
+    int W_ = 0;
+    int64_t ndof_ = 0;
+    DevBuf<unsigned long long> d_slots_;
+    DevBuf<double> d_save_, d_ws_;
+    DevBuf<GridState> d_state_;
+    std::unique_ptr<PinnedBuf<GridResult>> host_;
 };
 int grid_device_cus();
 
@@ -262,7 +279,8 @@ struct Model {
     DevBuf<int32_t> d_elem_m;   // per element: nodes (n), for the batched element-matrix kernels
     DevBuf<int64_t> d_elem_off; // per element: offset of its (3n)^2 block in d_ke
     DevBuf<int> d_elem_need;    // per element: its matrix needs the eigen path (projection)
-    PinnedBuf<int> h_err{1};
+    PinnedBuf<int> h_err{8 + sizeof(GridResult) / sizeof(int)};  // [0]: d_err's copy; from [8]: see grid_result
+    GridResult* grid_result() const { return reinterpret_cast<GridResult*>(h_err.p + 8); }  // of allocation-free solves
     // kernel timing of the CG system-matrix kernel (HIP events on the model stream)
     bool prof = false;
     int prof_tag = -1;           // PROF_* kind of the next launches of the tagged launchers, -1: none
@@ -331,6 +349,7 @@ struct CgWork {
     std::vector<const void*> batch_key;
     bool use_graphs = true;
     bool use_grid = true;  // the resident grid where the system fits it (grid_pcg.hip)
+    GridWork grid;
     PinnedBuf<CgScalars> h_scalars{3};  // final readback (slot 2)
     PinnedBuf<int> h_status{1, hipHostMallocCoherent};  // the solve's status, written by the kernel that ends it
     hipEvent_t ev[2] = {nullptr, nullptr};

@@ -1207,10 +1207,12 @@ static hoefem_status pcg_solve_t(Model& m, CgWork& w, const VT* Avals, const VT*
     // the resident grid takes every plain solve that fits it; per-iteration hooks (kernel timing, snapshots),
     // the flexible variant and a preconditioner of another model, whose plan splits that model's matrix, keep
     // the two kernels
-    GridPlan& grid = Pre ? Pre->grid : m.grid;
-    if (grid.serves(pat) && !FLEX && !h && !m.prof && w.use_grid &&
-        grid_solve<VT>(grid, m, Avals, Pre, Pre ? nullptr : w.diag_inv.get(), b, x, tol, max_iter, iterations, &st))
-        return st;
+    const GridPlan& grid = Pre ? Pre->grid : m.grid;
+    if (grid.serves(pat) && !FLEX && !h && !m.prof && w.use_grid) {
+        w.grid.ensure(grid);
+        if (grid_solve<VT>(grid, w.grid, m, Avals, Pre, Pre ? nullptr : w.diag_inv.get(), b, x, tol, max_iter, iterations, &st))
+            return st;
+    }
 #define CG_CASE(ga, gb, j, f)                                                                            \
     if (GA == ga && GB == gb && JAC == j && FLEX == f) {                                                 \
         cg_launch_all<ga, gb, j, f, VT>(m, w, A, Pm, b, x, tol, max_iter, iterations, &st, h, lv);        \
@@ -1246,6 +1248,7 @@ constexpr int64_t NA_VEC0 = NA_PART_B + 3 * CG_MAX_BLOCKS;
 constexpr int64_t NA_DIAG = NA_VEC0 + 4 * NOALLOC_VEC;
 constexpr int64_t NA_TOTAL = NA_DIAG + NOALLOC_MAX_DOFS;  // 9 * 262144 + 5248 doubles = 18.9 MB
 static_assert(sizeof(CgScalars) <= 32 * sizeof(double), "iteration state does not fit its region");
+static_assert(4 * NOALLOC_VEC == GRID_SCRATCH, "the resident grid's buffers take the CG vectors' place");
 static_assert(NA_PART_PRE % 32 == 0 && NA_VEC0 % 32 == 0 && NOALLOC_VEC % 32 == 0, "region alignment");
 
 static __device__ __align__(256) double scratch[NA_TOTAL];
@@ -1353,10 +1356,13 @@ hoefem_status pcg_solve_noalloc(Model& m, const double* Avals, Schwarz* Pre, con
         check_launch("k_jacobi_diag");
         if (read_and_clear_err(m) & KERR_ZERO_DIAG) throw Error(HOEFEM_ERROR_SINGULAR, "Diagonal matrix is not invertible.");
     }
-    GridPlan& grid = Pre ? Pre->grid : m.grid;
-    hoefem_status st = HOEFEM_OK;
-    if (grid.serves(pat) && grid_solve<double>(grid, m, Avals, Pre, Pre ? nullptr : base + NA_DIAG, b, x, tol, max_iter, iterations, &st))
-        return st;
+    const GridPlan& grid = Pre ? Pre->grid : m.grid;
+    if (grid.serves(pat)) {
+        GridBuffers w = grid_scratch_buffers(grid, base + NA_VEC0, m.grid_result());
+        hoefem_status st = HOEFEM_OK;
+        if (grid_solve<double>(grid, w, m, Avals, Pre, Pre ? nullptr : base + NA_DIAG, b, x, tol, max_iter, iterations, &st))
+            return st;
+    }
 #define NA_CASE(ga, gb, j) \
     if (GA == ga && GB == gb && (Pre == nullptr) == j) return cg_launch_noalloc<ga, gb, j>(m, base, A, Pm, b, x, tol, max_iter, iterations);
     NA_CASE(8, 8, true) NA_CASE(16, 8, true) NA_CASE(32, 8, true)

@@ -218,9 +218,9 @@ hoefem_status hoefem_pcg(hoefem_model* model, const double* A_values, hoefem_sch
 
 /* hoefem_pcg without allocation. No counterpart in the reference: for callers that cannot
  * allocate device or pinned memory during a solve (serving loops, harnesses that forbid it, code
- * that runs under stream capture nearby). Same kernels, arguments and results as hoefem_pcg: a system
- * that fits the resident grid uses the buffers its model and preconditioner allotted when they were
- * created, the others a fixed per-GPU array of 18.9 MB held until the process ends. The model
+ * that runs under stream capture nearby). Same kernels, arguments and results as hoefem_pcg; the
+ * work buffers live in a fixed per-GPU array of 18.9 MB held until the process ends (and, for the few systems
+ * whose resident grid needs more, in a buffer allotted with the model and the preconditioner). The model
  * may have at most 262144 DOFs (larger models: HOEFEM_ERROR_INVALID_ARGUMENT) and the model must use
  * device pointers. Runs on the model's stream and synchronizes it. Calls that overlap in time on
  * one GPU share that array and race; serialize them. FP64 operators only. */

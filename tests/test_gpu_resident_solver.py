@@ -83,3 +83,33 @@ def test_preconditioner_of_another_size_is_refused(entry):
     x, its = torch.zeros_like(b), C.c_int64()
     assert getattr(L, entry)(gm.h, Jd.data_ptr(), pre.h, b.data_ptr(), x.data_ptr(), 1e-8, 10, C.byref(its)) == 1
     assert b"nodes" in L.hoefem_last_error()
+
+
+@pytest.mark.parametrize("schwarz", [False, True])
+def test_sims_of_one_model_in_one_batch(schwarz):
+    """Sims that share a model are in flight together: each ends where it ends alone, bit for bit."""
+    from higher_order_embedded_fem_amd import fem
+
+    sc = scenes.cube_scene(4, scenes.TET10)
+    gm = fem.ElasticityModel(sc)
+    sims = [fem.NewtonCgIntegrator(gm, sc, schwarz=schwarz, newton_tolerance_factor=1e-6, cg_max_iter=5000)
+            for _ in range(4)]
+    rng = np.random.default_rng(7)
+    v0 = 0.2 * rng.standard_normal((len(sims), sc.ndof))
+    v0.reshape(len(sims), -1, 3)[:, sc.dirichlet_nodes] = 0.0
+    state = [(torch.zeros(sc.ndof, dtype=torch.float64, device="cuda"), dev(v)) for v in v0]
+    alone = []
+    for sim, (u, v) in zip(sims, state):
+        ua, va = u.clone(), v.clone()
+        for i in range(2):
+            sim.step(i * sc.dt, sc.dt, ua, va)
+        alone.append((ua, va))
+    L, n = _lib.load(), len(sims)
+    h = C.c_void_p()
+    _lib.check(L.hoefem_batch_create((C.c_void_p * n)(*[s.h.value for s in sims]), n, C.byref(h)))
+    us, vs = (C.c_void_p * n)(*[u.data_ptr() for u, _ in state]), (C.c_void_p * n)(*[v.data_ptr() for _, v in state])
+    for _ in range(2):
+        _lib.check(L.hoefem_batch_step(h, (C.c_double * n)(*[sc.dt] * n), us, vs, None, None, None))
+    L.hoefem_batch_destroy(h)
+    for (u, v), (ua, va) in zip(state, alone):
+        assert torch.equal(u, ua) and torch.equal(v, va)
