@@ -39,7 +39,6 @@
 // falls back to the two-kernel path.
 #include <algorithm>
 #include <cmath>
-#include <condition_variable>
 #include <map>
 #include <mutex>
 #include <system_error>
@@ -790,66 +789,51 @@ void grid_clear(const GridPlan& g, GridBuffers& w, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------ admission
-// CUs of each device taken by resident grids in flight: a launch is admitted when its work-groups (one per
-// CU at most) fit beside those already admitted, so admitted grids are all resident and make progress.
+// A launch is admitted when its work-groups (one per CU at most) fit beside those of the process's launches in
+// flight on the device, so admitted grids are all resident and make progress.
 namespace {
-struct Slots {
-    std::mutex mu;
-    std::condition_variable cv;
-    std::map<int, std::pair<int, int>> dev;  // device -> (CUs, free)
-    std::pair<int, int>& of(int d) {
-        auto it = dev.find(d);
-        if (it == dev.end()) {
-            int n = 0;
-            HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, d));
-            it = dev.emplace(d, std::make_pair(n, n)).first;
-        }
-        return it->second;
+CuLine& device_line() {
+    static std::mutex mu;
+    static std::map<int, CuLine> lines;
+    int d = 0;
+    HIP_CHECK(hipGetDevice(&d));
+    std::lock_guard<std::mutex> lock(mu);
+    auto it = lines.find(d);
+    if (it == lines.end()) {
+        int n = 0;
+        HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, d));
+        it = lines.try_emplace(d, n).first;
     }
-};
-Slots& slots() {
-    static Slots s;
-    return s;
+    return it->second;
 }
 }  // namespace
 
-int grid_device_cus() {
-    int d = 0;
-    HIP_CHECK(hipGetDevice(&d));
-    std::lock_guard<std::mutex> lock(slots().mu);
-    return slots().of(d).first;
+int grid_device_cus() { return device_line().cus(); }
+
+bool GridSlots::acquire(int wgs, bool wait) {
+    if (!place_) {
+        release();
+        line_ = &device_line();
+        if (wgs > line_->cus()) return false;
+        place_ = line_->enter();
+    }
+    if (!line_->take(place_, wgs, wait)) return false;
+    place_ = 0;
+    n_ = wgs;
+    return true;
 }
 
-int grid_free_cus() {
-    int d = 0;
-    HIP_CHECK(hipGetDevice(&d));
-    std::lock_guard<std::mutex> lock(slots().mu);
-    return slots().of(d).second;
-}
-
-bool GridSlots::acquire(int n, bool wait) {
-    release();
-    HIP_CHECK(hipGetDevice(&dev_));
-    std::unique_lock<std::mutex> lock(slots().mu);
-    auto& c = slots().of(dev_);
-    if (n > c.first) return false;
-    if (wait)
-        slots().cv.wait(lock, [&] { return c.second >= n; });
-    else if (c.second < n)
-        return false;
-    c.second -= n;
-    n_ = n;
+bool GridSlots::grow(int wgs) {
+    if (!line_->take_more(wgs - n_)) return false;
+    n_ = wgs;
     return true;
 }
 
 void GridSlots::release() {
-    if (!n_) return;
-    {
-        std::lock_guard<std::mutex> lock(slots().mu);
-        slots().dev[dev_].second += n_;
-    }
+    if (place_) line_->leave(place_);
+    if (n_) line_->give(n_);
+    place_ = 0;
     n_ = 0;
-    slots().cv.notify_all();
 }
 
 // ------------------------------------------------------------------ launches
@@ -1045,14 +1029,16 @@ struct GridPoolT final : CgPool {
                 HIP_CHECK(e);
                 ended_launch(l, ended);
             }
-        for (int l = 0; l < GRID_LANES && !waiting.empty(); ++l) {
-            if (!running[l].empty()) continue;
+        while (!waiting.empty()) {
+            int l = -1;  // an idle lane, the one with a place in the line first
+            for (int i = 0; i < GRID_LANES; ++i)
+                if (running[i].empty() && (l < 0 || slots[i].waiting())) l = i;
+            if (l < 0) break;
             // as many waiting systems as fit, at least the first
-            int wgs = 0, n = 0;
-            const int cus = grid_free_cus();
-            while (n < (int)waiting.size() && n < GRID_SEGS && wgs + items[waiting[n]].g->W <= cus)
+            int wgs = items[waiting[0]].g->W, n = 1;
+            if (!slots[l].acquire(wgs, false)) break;
+            while (n < (int)waiting.size() && n < GRID_SEGS && slots[l].grow(wgs + items[waiting[n]].g->W))
                 wgs += items[waiting[n++]].g->W;
-            if (n == 0 || !slots[l].acquire(wgs, false)) break;
             GridSegs<VT, GRID_SEGS> all{};
             size_t lds = 0;
             const hipStream_t s = B.lanes[l].s;

@@ -1,6 +1,7 @@
 // The resident-grid PCG (grid_pcg.hip): plan of a system, its launch descriptor and entry points.
 #pragma once
 
+#include "cu_line.hpp"
 #include "internal.hpp"
 
 namespace hoefem {
@@ -48,21 +49,24 @@ struct GridSegs {
 };
 static_assert(sizeof(GridSegs<double, GRID_SEGS>) <= 4096, "kernel arguments");
 
-// CUs held for resident grids in flight on the current device
+// CUs held for a launch of resident grids on the current device
 class GridSlots {
 public:
     GridSlots() = default;
     GridSlots(const GridSlots&) = delete;
     GridSlots& operator=(const GridSlots&) = delete;
     ~GridSlots() { release(); }
-    bool acquire(int n, bool wait);  // false: not free (wait: never will be)
+    // false: not yet its turn, its place in the line kept (wait: the device never has so many)
+    bool acquire(int wgs, bool wait);
+    bool grow(int wgs);  // to wgs in all; false: not free, or others wait
+    bool waiting() const { return place_ != 0; }
     void release();
 
 private:
-    int n_ = 0, dev_ = 0;
+    CuLine* line_ = nullptr;
+    uint64_t place_ = 0;
+    int n_ = 0;
 };
-
-int grid_free_cus();  // CUs of the current device not held
 
 template <class VT>
 GridSeg<VT> grid_segment(const GridPlan& g, const GridBuffers& w, Model& m, const VT* A, const Schwarz* P,

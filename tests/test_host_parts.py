@@ -1,0 +1,76 @@
+"""Host parts of the library that need no GPU, compiled by themselves and run."""
+
+import os
+import subprocess
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "higher_order_embedded_fem_amd", "csrc")
+
+
+def run(tmp_path, source):
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    src.write_text(source)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-pthread", "-I", CSRC, "-o", str(exe), str(src)], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+CHECK = """
+#include <cstdio>
+#define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\\n", __LINE__, #x); return 1; } } while (0)
+"""
+
+
+def test_resident_grids_are_admitted_in_order(tmp_path):
+    """A launch that needs the whole device is not passed by later small ones, whether it waits or polls."""
+    run(tmp_path, CHECK + """
+#include <thread>
+#include "cu_line.hpp"
+using hoefem::CuLine;
+int main() {
+    CuLine L(16);
+    const uint64_t a = L.enter();
+    CHECK(L.take(a, 8, false));
+    // one that waits in another thread
+    const uint64_t wide = L.enter();
+    std::thread t([&] { L.take(wide, 16, true); });
+    const uint64_t small = L.enter();
+    CHECK(!L.take(small, 4, false));  // 8 are free, but the wide one was first
+    CHECK(!L.take_more(4));
+    L.give(8);
+    t.join();
+    CHECK(!L.take(small, 4, false));  // all taken
+    L.give(16);
+    CHECK(L.take(small, 4, false));
+    CHECK(L.take_more(12));
+    CHECK(!L.take_more(1));
+    L.give(16);
+    // one that polls, and gives up
+    const uint64_t b = L.enter();
+    CHECK(L.take(b, 4, false));
+    const uint64_t poll = L.enter();
+    CHECK(!L.take(poll, 16, false));
+    const uint64_t next = L.enter();
+    CHECK(!L.take(next, 1, false));
+    L.leave(poll);
+    CHECK(L.take(next, 12, false));
+    L.give(16);
+    // small ones by turns from two threads while a wide one waits: it gets through
+    auto churn = [&] {
+        for (int i = 0; i < 20000; ++i) {
+            const uint64_t p = L.enter();
+            L.take(p, 6, true);
+            L.give(6);
+        }
+    };
+    std::thread c1(churn), c2(churn);
+    for (int i = 0; i < 100; ++i) {
+        const uint64_t p = L.enter();
+        L.take(p, 16, true);
+        L.give(16);
+    }
+    c1.join();
+    c2.join();
+    return 0;
+}
+""")
