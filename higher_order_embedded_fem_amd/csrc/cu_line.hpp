@@ -14,6 +14,13 @@ namespace hoefem {
 // beside threads that step small scenes).
 class CuLine {
 public:
+    // The work-groups of a launch are dealt to the XCDs in turn, the first to the same one each time, and one that
+    // finds its XCD full waits there although others have room. A launch is therefore charged the same number of
+    // CUs on every XCD, the most that any of them gets: launches of 82, 82 and 90 work-groups (254) would put 34 on
+    // an XCD of 32 CUs.
+    static constexpr int XCDS = 8;
+    static int charge(int wgs) { return (wgs + XCDS - 1) / XCDS * XCDS; }
+
     explicit CuLine(int cus) : cus_(cus), free_(cus) {}
     int cus() const { return cus_; }
 

@@ -802,7 +802,7 @@ CuLine& device_line() {
     if (it == lines.end()) {
         int n = 0;
         HIP_CHECK(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, d));
-        it = lines.try_emplace(d, n).first;
+        it = lines.try_emplace(d, n / CuLine::XCDS * CuLine::XCDS).first;
     }
     return it->second;
 }
@@ -811,21 +811,23 @@ CuLine& device_line() {
 int grid_device_cus() { return device_line().cus(); }
 
 bool GridSlots::acquire(int wgs, bool wait) {
+    const int n = CuLine::charge(wgs);
     if (!place_) {
         release();
         line_ = &device_line();
-        if (wgs > line_->cus()) return false;
+        if (n > line_->cus()) return false;
         place_ = line_->enter();
     }
-    if (!line_->take(place_, wgs, wait)) return false;
+    if (!line_->take(place_, n, wait)) return false;
     place_ = 0;
-    n_ = wgs;
+    n_ = n;
     return true;
 }
 
 bool GridSlots::grow(int wgs) {
-    if (!line_->take_more(wgs - n_)) return false;
-    n_ = wgs;
+    const int n = CuLine::charge(wgs);
+    if (n > n_ && !line_->take_more(n - n_)) return false;
+    n_ = n;
     return true;
 }
 

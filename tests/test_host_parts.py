@@ -74,3 +74,36 @@ int main() {
     return 0;
 }
 """)
+
+
+def test_admitted_grids_fit_every_xcd(tmp_path):
+    """Every launch's work-groups go to the XCDs in turn from the first one: whatever is admitted together, no
+    XCD gets more work-groups than it has CUs."""
+    run(tmp_path, CHECK + """
+#include <random>
+#include <vector>
+#include "cu_line.hpp"
+using hoefem::CuLine;
+int main() {
+    std::mt19937 rng(1);
+    for (int round = 0; round < 20000; ++round) {
+        CuLine L(256);
+        int xcd[8] = {};
+        int sum = 0;
+        for (int k = 0; k < 6; ++k) {
+            const int wgs = round == 0 ? (k < 2 ? 82 : 90) : 1 + (int)(rng() % (round % 2 ? 256 : 100));
+            const uint64_t p = L.enter();
+            if (!L.take(p, CuLine::charge(wgs), false)) {
+                L.leave(p);
+                continue;
+            }
+            sum += wgs;
+            for (int w = 0; w < wgs; ++w) ++xcd[w % 8];
+        }
+        CHECK(sum > 0 && sum <= 256);
+        for (int x : xcd) CHECK(x <= 32);
+    }
+    CHECK(CuLine::charge(256) == 256 && CuLine::charge(1) == 8);
+    return 0;
+}
+""")
