@@ -1391,12 +1391,6 @@ static void sim_autotune_cg(Sim& s, int* ga_out, int* gb_out, double* candidate_
         if (s.schwarz) schwarz_update(*s.schwarz, s.d_J.get());
     }
     launch_fill(m, s.d_F.get(), n, 1.0);
-    struct TwoKernels {
-        CgWork& w;
-        const bool before = w.use_grid;
-        explicit TwoKernels(CgWork& work) : w(work) { w.use_grid = false; }
-        ~TwoKernels() { w.use_grid = before; }
-    } two_kernels(s.cg);
     hipEvent_t e0, e1;
     HIP_CHECK(hipEventCreate(&e0));
     HIP_CHECK(hipEventCreate(&e1));
@@ -1406,9 +1400,10 @@ static void sim_autotune_cg(Sim& s, int* ga_out, int* gb_out, double* candidate_
     auto run = [&](int64_t iters) {
         launch_fill(m, s.d_sol.get(), n, 0.0);
         if (s.mixed)
-            (void)pcg_solve(m, s.cg, s.d_J32.get(), s.schwarz.get(), s.d_F.get(), s.d_sol.get(), 0.0, iters, &it);
+            (void)pcg_solve(m, s.cg, s.d_J32.get(), s.schwarz.get(), s.d_F.get(), s.d_sol.get(), 0.0, iters, &it,
+                            true);
         else
-            (void)pcg_solve(m, s.cg, s.d_J.get(), s.schwarz.get(), s.d_F.get(), s.d_sol.get(), 0.0, iters, &it);
+            (void)pcg_solve(m, s.cg, s.d_J.get(), s.schwarz.get(), s.d_F.get(), s.d_sol.get(), 0.0, iters, &it, true);
     };
     // AUTOTUNE_ROUNDS rounds over all pairs, each pair's best 96-iteration solve kept: a drift of the
     // GPU's speed during tuning then reaches every pair instead of favouring the ones measured last

@@ -1002,10 +1002,8 @@ struct GridPoolT final : CgPool {
             if (h->failed) {  // solved from the start by the two kernels
                 it.w->cleared = false;
                 HIP_CHECK(hipMemsetAsync(it.q.x, 0, sizeof(double) * it.g->ndof, it.q.m->stream));
-                it.q.w->use_grid = false;
                 it.q.status = pcg_solve(*it.q.m, *it.q.w, (const VT*)it.q.A, it.q.P, it.q.b, it.q.x, it.q.tol,
-                                        it.q.max_iter, &it.q.iterations);
-                it.q.w->use_grid = true;
+                                        it.q.max_iter, &it.q.iterations, true);
                 HIP_CHECK(hipStreamSynchronize(it.q.m->stream));
                 ended.push_back(id);
                 continue;

@@ -348,7 +348,6 @@ struct CgWork {
     hipGraphExec_t batch_exec = nullptr;
     std::vector<const void*> batch_key;
     bool use_graphs = true;
-    bool use_grid = true;  // the resident grid where the system fits it (grid_pcg.hip)
     GridWork grid;
     PinnedBuf<CgScalars> h_scalars{3};  // final readback (slot 2)
     PinnedBuf<int> h_status{1, hipHostMallocCoherent};  // the solve's status, written by the kernel that ends it
@@ -410,16 +409,17 @@ void schwarz_update(Schwarz& s, const float* J);
 void schwarz_apply(Schwarz& s, const double* x, double* y);
 
 // ------------------------------------------------------------------ CG (solver.hip)
-// Solves A x = b. A has the model pattern; preconditioner = Schwarz or Jacobi(diag(A)).
+// Solves A x = b. A has the model pattern; preconditioner = Schwarz or Jacobi(diag(A)). two_kernels: not by the
+// resident grid (grid_pcg.hip), whether or not the system fits it.
 hoefem_status pcg_solve(Model& m, CgWork& w, const double* A, Schwarz* P, const double* b, double* x, double tol,
-                        int64_t max_iter, int64_t* iterations);
+                        int64_t max_iter, int64_t* iterations, bool two_kernels = false);
 // pcg_solve (FP64) with every work buffer in a fixed per-device scratch array: no allocation;
 // models of at most 262144 DOFs; calls overlapping in time on one GPU race
 hoefem_status pcg_solve_noalloc(Model& m, const double* A, Schwarz* P, const double* b, double* x, double tol,
                                 int64_t max_iter, int64_t* iterations);
 // mixed precision: FP32 system matrix and FP32 Schwarz operator (P->fp32 must be set), FP64 vectors / dots
 hoefem_status pcg_solve(Model& m, CgWork& w, const float* A, Schwarz* P, const double* b, double* x, double tol,
-                        int64_t max_iter, int64_t* iterations);
+                        int64_t max_iter, int64_t* iterations, bool two_kernels = false);
 
 // One system of a batched solve: the arguments of pcg_solve (A of value type double, or float
 // with an FP32 Schwarz operator) and its results.

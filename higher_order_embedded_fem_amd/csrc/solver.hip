@@ -1181,8 +1181,8 @@ static void check_preconditioner(const NodePattern& A, const Schwarz* P) {
 
 template <class VT>
 static hoefem_status pcg_solve_t(Model& m, CgWork& w, const VT* Avals, const VT* Pvals, Schwarz* Pre, const double* b,
-                                 double* x, double tol, int64_t max_iter, int64_t* iterations, CgHarvest* h = nullptr,
-                                 const LearnedView* lv = nullptr) {
+                                 double* x, double tol, int64_t max_iter, int64_t* iterations, bool two_kernels,
+                                 CgHarvest* h = nullptr, const LearnedView* lv = nullptr) {
     const NodePattern& pat = m.pattern;
     check_preconditioner(pat, Pre);
     const int64_t nn = pat.num_nodes;
@@ -1208,7 +1208,7 @@ static hoefem_status pcg_solve_t(Model& m, CgWork& w, const VT* Avals, const VT*
     // the flexible variant and a preconditioner of another model, whose plan splits that model's matrix, keep
     // the two kernels
     const GridPlan& grid = Pre ? Pre->grid : m.grid;
-    if (grid.serves(pat) && !FLEX && !h && !m.prof && w.use_grid) {
+    if (grid.serves(pat) && !two_kernels && !m.prof) {
         w.grid.ensure(grid);
         if (grid_solve<VT>(grid, w.grid, m, Avals, Pre, Pre ? nullptr : w.diag_inv.get(), b, x, tol, max_iter, iterations, &st))
             return st;
@@ -1374,39 +1374,39 @@ hoefem_status pcg_solve_noalloc(Model& m, const double* Avals, Schwarz* Pre, con
 }
 
 hoefem_status pcg_solve(Model& m, CgWork& w, const double* A, Schwarz* P, const double* b, double* x, double tol,
-                        int64_t max_iter, int64_t* iterations) {
+                        int64_t max_iter, int64_t* iterations, bool two_kernels) {
     if (P && P->fp32) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "FP32 preconditioner with an FP64 operator");
-    return pcg_solve_t<double>(m, w, A, P ? P->d_vals.get() : nullptr, P, b, x, tol, max_iter, iterations);
+    return pcg_solve_t<double>(m, w, A, P ? P->d_vals.get() : nullptr, P, b, x, tol, max_iter, iterations, two_kernels);
 }
 
 hoefem_status pcg_solve(Model& m, CgWork& w, const float* A, Schwarz* P, const double* b, double* x, double tol,
-                        int64_t max_iter, int64_t* iterations) {
+                        int64_t max_iter, int64_t* iterations, bool two_kernels) {
     if (P && !P->fp32) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "FP64 preconditioner with an FP32 operator");
-    return pcg_solve_t<float>(m, w, A, P ? P->d_vals32.get() : nullptr, P, b, x, tol, max_iter, iterations);
+    return pcg_solve_t<float>(m, w, A, P ? P->d_vals32.get() : nullptr, P, b, x, tol, max_iter, iterations, two_kernels);
 }
 
 hoefem_status pcg_solve_harvest(Model& m, CgWork& w, const double* A, Schwarz* P, const double* b, double* x,
                                 double tol, int64_t max_iter, int64_t* iterations, CgHarvest* h) {
     if (P && P->fp32) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "FP32 preconditioner with an FP64 operator");
-    return pcg_solve_t<double>(m, w, A, P ? P->d_vals.get() : nullptr, P, b, x, tol, max_iter, iterations, h);
+    return pcg_solve_t<double>(m, w, A, P ? P->d_vals.get() : nullptr, P, b, x, tol, max_iter, iterations, true, h);
 }
 
 hoefem_status pcg_solve_harvest(Model& m, CgWork& w, const float* A, Schwarz* P, const double* b, double* x,
                                 double tol, int64_t max_iter, int64_t* iterations, CgHarvest* h) {
     if (P && !P->fp32) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "FP64 preconditioner with an FP32 operator");
-    return pcg_solve_t<float>(m, w, A, P ? P->d_vals32.get() : nullptr, P, b, x, tol, max_iter, iterations, h);
+    return pcg_solve_t<float>(m, w, A, P ? P->d_vals32.get() : nullptr, P, b, x, tol, max_iter, iterations, true, h);
 }
 
 hoefem_status pcg_solve_learned(Model& m, CgWork& w, const double* A, Schwarz* P, const LearnedView& lv,
                                 const double* b, double* x, double tol, int64_t max_iter, int64_t* iterations) {
     if (!P || P->fp32) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "learned solve needs the FP64 Schwarz operator");
-    return pcg_solve_t<double>(m, w, A, P->d_vals.get(), P, b, x, tol, max_iter, iterations, nullptr, &lv);
+    return pcg_solve_t<double>(m, w, A, P->d_vals.get(), P, b, x, tol, max_iter, iterations, true, nullptr, &lv);
 }
 
 hoefem_status pcg_solve_learned(Model& m, CgWork& w, const float* A, Schwarz* P, const LearnedView& lv,
                                 const double* b, double* x, double tol, int64_t max_iter, int64_t* iterations) {
     if (!P || !P->fp32) throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "learned solve needs the FP32 Schwarz operator");
-    return pcg_solve_t<float>(m, w, A, P->d_vals32.get(), P, b, x, tol, max_iter, iterations, nullptr, &lv);
+    return pcg_solve_t<float>(m, w, A, P->d_vals32.get(), P, b, x, tol, max_iter, iterations, true, nullptr, &lv);
 }
 
 // ================================================================== batched PCG
