@@ -50,6 +50,8 @@ EXPORTED = [
     "hoefem_model_autotune",
     "hoefem_schwarz_autotune",
     "hoefem_sim_autotune",
+    "hoefem_resident_solver_set",
+    "hoefem_resident_solver_stats",
     "hoefem_profile_enable",
     "hoefem_profile_read",
     "hoefem_profile_kernel",
@@ -252,6 +254,8 @@ def load(path: str = LIB_PATH):
     L.hoefem_model_autotune.argtypes = [vp, C.POINTER(i32), vp]
     L.hoefem_schwarz_autotune.argtypes = [vp, C.POINTER(i32), vp]
     L.hoefem_sim_autotune.argtypes = [vp, C.POINTER(i32), C.POINTER(i32), vp]
+    L.hoefem_resident_solver_set.argtypes = [vp, i32, i32]
+    L.hoefem_resident_solver_stats.argtypes = [vp, C.POINTER(i64), C.POINTER(i64)]
     L.hoefem_profile_enable.argtypes = [vp, i32]
     L.hoefem_profile_read.argtypes = [vp, C.POINTER(i64), C.POINTER(f64), C.POINTER(i64), C.POINTER(f64)]
     L.hoefem_profile_kernel.argtypes = [vp, i32, C.POINTER(i64), C.POINTER(f64)]

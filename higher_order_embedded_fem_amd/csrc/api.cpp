@@ -705,21 +705,26 @@ static void batch_step(Batch& B, const double* dt, double* const* u, double* con
         B.ev.push_back(e);
     }
     const bool fp32 = B.sims[0]->fp32_jacobian();
-    std::vector<int> pool_of(ns);
-    int pool_size[BATCH_POOLS + 1] = {};
+    // pools by size, the resident grid's last, each made for its first system
+    std::vector<int> size_of(ns);
+    int pool_size[BATCH_POOLS] = {};
     for (size_t i = 0; i < ns; ++i) {
-        const Sim& s = *B.sims[i];
-        const int64_t ndof = 3 * s.model->nv;
-        int c = 0;
-        while (c < BATCH_POOLS - 1 && ndof >= BATCH_POOL_DOFS[c]) ++c;
-        if ((s.schwarz ? s.schwarz->grid : s.model->grid).serves(s.model->pattern)) c = BATCH_POOLS;  // the resident grid's
-        pool_of[i] = c;
-        pool_size[c] += 1;
+        const int64_t ndof = 3 * B.sims[i]->model->nv;
+        while (size_of[i] < BATCH_POOLS - 1 && ndof >= BATCH_POOL_DOFS[size_of[i]]) ++size_of[i];
+        pool_size[size_of[i]] += 1;
     }
     std::unique_ptr<CgPool> pools[BATCH_POOLS + 1];
-    for (int c = 0; c < BATCH_POOLS; ++c)
-        if (pool_size[c]) pools[c] = make_cg_pool(B.cg[c], fp32, pool_size[c]);
-    if (pool_size[BATCH_POOLS]) pools[BATCH_POOLS] = make_grid_pool(B.grid, fp32);
+    auto pool_for = [&](size_t i) {  // of the scene's next solve, which may follow a failed one
+        Sim& s = *B.sims[i];
+        int c = BATCH_POOLS;
+        if (!s.model->use_grid || !(s.schwarz ? s.schwarz->grid : s.model->grid).serves(s.model->pattern) ||
+            s.cg.grid.rest.resting()) {
+            c = size_of[i];
+            s.cg.grid.rest.pass();
+        }
+        if (!pools[c]) pools[c] = c < BATCH_POOLS ? make_cg_pool(B.cg[c], fp32, pool_size[c]) : make_grid_pool(B.grid, fp32);
+        return c;
+    };
     std::vector<BatchScene> q(ns);
     const auto t0 = std::chrono::steady_clock::now();
     auto elapsed_ms = [&]() {
@@ -844,7 +849,7 @@ static void batch_step(Batch& B, const double* dt, double* const* u, double* con
                     sys.x = s.d_sol.get();
                     sys.tol = s.d.cg_tolerance;
                     sys.max_iter = s.d.cg_max_iter;
-                    const int pc = pool_of[i];
+                    const int pc = pool_for(i);
                     b.cg_id = pools[pc]->join(sys);
                     if ((int)owner[pc].size() <= b.cg_id) owner[pc].resize(b.cg_id + 1, -1);
                     owner[pc][b.cg_id] = (int)i;
@@ -1453,6 +1458,22 @@ hoefem_status hoefem_sim_autotune(hoefem_sim* sim, int32_t* lanes_matrix, int32_
         sim_autotune_cg(sim->s, &ga, &gb, candidate_us);
         if (lanes_matrix) *lanes_matrix = ga;
         if (lanes_preconditioner) *lanes_preconditioner = gb;
+    });
+}
+
+hoefem_status hoefem_resident_solver_set(hoefem_model* model, int32_t enable, int32_t poll_limit) {
+    return guarded([&] {
+        Model& m = M_(model);
+        m.use_grid = enable != 0;
+        m.grid_polls = poll_limit;
+    });
+}
+
+hoefem_status hoefem_resident_solver_stats(hoefem_model* model, int64_t* solves, int64_t* failures) {
+    return guarded([&] {
+        const Model& m = M_(model);
+        if (solves) *solves = m.grid_solves;
+        if (failures) *failures = m.grid_failures;
     });
 }
 

@@ -35,7 +35,7 @@
 //
 // Residency. The work-groups wait for each other, so all of a launch's must be resident: launches are
 // admitted against the device's number of CUs (GridSlots below), one work-group per CU. Every wait is
-// bounded (GRID_POLL_LIMIT); a launch that cannot make progress ends with an error status and the caller
+// bounded (GRID_POLL_LIMIT polls); a launch that cannot make progress ends with an error status and the caller
 // falls back to the two-kernel path.
 #include <algorithm>
 #include <cmath>
@@ -356,8 +356,8 @@ __global__ __launch_bounds__(GRID_THREADS) __attribute__((amdgpu_waves_per_eu(2,
             for (int w = 0; w < GRID_WAVES; ++w) s += s_w[w][wid];
             if (lane < GRID_COPIES) agent_store((double*)&sl[lane * W + b], s);
             sl += (b % GRID_COPIES) * W;
-            double got[GRID_MAX_WG / 64];
-            for (int i = 0; missing && i < GRID_POLL_LIMIT; ++i) {
+            double got[GRID_MAX_WG / 64] = {};
+            for (int i = 0; missing && i < S.polls; ++i) {
                 missing = false;
 #pragma unroll
                 for (int q = 0; q < GRID_MAX_WG / 64; ++q) {
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(GRID_THREADS) __attribute__((amdgpu_waves_per_eu(2,
             }
         }
         missing = true;
-        for (int i = 0; missing && i < GRID_POLL_LIMIT; ++i) {
+        for (int i = 0; missing && i < S.polls; ++i) {
             missing = false;
 #pragma unroll
             for (int h = 0; h < H; ++h) {
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(GRID_THREADS) __attribute__((amdgpu_waves_per_eu(2,
         const double* vec = S.vec + (int64_t)((phase - 1) & 3u) * S.ndof;
         for (int j = t + H * GRID_THREADS; j < n; j += GRID_THREADS) {
             double q = agent_load(vec + off[j]);
-            for (int i = 0; is_empty(q) && i < GRID_POLL_LIMIT; ++i) q = agent_load(vec + off[j]);
+            for (int i = 0; is_empty(q) && i < S.polls; ++i) q = agent_load(vec + off[j]);
             if (is_empty(q)) s_bad = 1;
             dst[j] = fn(dst[j], q);
         }
@@ -873,6 +873,7 @@ GridSeg<VT> grid_segment(const GridPlan& g, const GridBuffers& w, Model& m, cons
     S.host = w.result;
     S.W = g.W;
     S.phase = w.phase;
+    S.polls = m.grid_polls < 0 ? GRID_POLL_LIMIT : m.grid_polls;
     S.nlds = g.nlds;
     S.blk_off = g.blk_off;
     S.tol = tol;
@@ -900,8 +901,13 @@ template void grid_launch<double, GRID_SEGS>(const GridSegs<double, GRID_SEGS>&,
 template void grid_launch<float, GRID_SEGS>(const GridSegs<float, GRID_SEGS>&, int, size_t, hipStream_t);
 
 template <class VT>
-bool grid_solve(const GridPlan& g, GridBuffers& w, Model& m, const VT* A, const Schwarz* P, const double* dinv,
-                const double* b, double* x, double tol, int64_t max_iter, int64_t* iterations, hoefem_status* status) {
+bool grid_solve(const GridPlan& g, GridBuffers& w, GridRest& rest, Model& m, const VT* A, const Schwarz* P,
+                const double* dinv, const double* b, double* x, double tol, int64_t max_iter, int64_t* iterations,
+                hoefem_status* status) {
+    if (rest.resting()) {
+        rest.pass();
+        return false;
+    }
     GridSegs<VT, 1> all;
     GridSeg<VT>& S = all.seg[0];
     grid_clear(g, w, m.stream);
@@ -919,6 +925,8 @@ bool grid_solve(const GridPlan& g, GridBuffers& w, Model& m, const VT* A, const 
         }
         if (h->failed) {
             w.cleared = false;
+            rest.ended(false);
+            m.grid_failures += 1;
             return false;
         }
         w.phase = S.phase = h->phase;
@@ -926,13 +934,15 @@ bool grid_solve(const GridPlan& g, GridBuffers& w, Model& m, const VT* A, const 
         if (h->status != GRID_RUNNING) break;
         S.resume = 1;
     }
+    rest.ended(true);
+    m.grid_solves += 1;
     const int st = w.result->status;
     *status = st == GRID_CONVERGED || st == GRID_ZERO_RHS ? HOEFEM_OK : (hoefem_status)st;
     return true;
 }
-template bool grid_solve<double>(const GridPlan&, GridBuffers&, Model&, const double*, const Schwarz*,
+template bool grid_solve<double>(const GridPlan&, GridBuffers&, GridRest&, Model&, const double*, const Schwarz*,
                                  const double*, const double*, double*, double, int64_t, int64_t*, hoefem_status*);
-template bool grid_solve<float>(const GridPlan&, GridBuffers&, Model&, const float*, const Schwarz*,
+template bool grid_solve<float>(const GridPlan&, GridBuffers&, GridRest&, Model&, const float*, const Schwarz*,
                                 const double*, const double*, double*, double, int64_t, int64_t*, hoefem_status*);
 
 // ------------------------------------------------------------------ many systems
@@ -1001,6 +1011,8 @@ struct GridPoolT final : CgPool {
             volatile GridResult* h = it.w->result;
             if (h->failed) {  // solved from the start by the two kernels
                 it.w->cleared = false;
+                it.w->rest.ended(false);
+                it.q.m->grid_failures += 1;
                 HIP_CHECK(hipMemsetAsync(it.q.x, 0, sizeof(double) * it.g->ndof, it.q.m->stream));
                 it.q.status = pcg_solve(*it.q.m, *it.q.w, (const VT*)it.q.A, it.q.P, it.q.b, it.q.x, it.q.tol,
                                         it.q.max_iter, &it.q.iterations, true);
@@ -1014,6 +1026,8 @@ struct GridPoolT final : CgPool {
                 again.push_back(id);
                 continue;
             }
+            it.w->rest.ended(true);
+            it.q.m->grid_solves += 1;
             it.q.iterations = h->iters;
             it.q.status = h->status == GRID_CONVERGED || h->status == GRID_ZERO_RHS ? HOEFEM_OK : (hoefem_status)h->status;
             ended.push_back(id);

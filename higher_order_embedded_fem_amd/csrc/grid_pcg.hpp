@@ -37,6 +37,7 @@ struct GridSeg {
     int W;            // work-groups
     uint32_t phase;   // exchanges done so far (the sets in use)
     int resume;
+    int polls;        // of a value before the launch is given up
     int nlds, blk_off;  // blocks of a thread in LDS, and their offset there (doubles)
     int64_t chunk, max_iter;
     double tol;
@@ -75,9 +76,10 @@ GridSeg<VT> grid_segment(const GridPlan& g, const GridBuffers& w, Model& m, cons
 template <class VT, int K>
 void grid_launch(const GridSegs<VT, K>& all, int wgs, size_t lds, hipStream_t s);
 void grid_clear(const GridPlan& g, GridBuffers& w, hipStream_t s);
-// Solves A x = b on the model stream; false: the grid could not run (x is a valid guess for another solver)
+// Solves A x = b on the model stream; false: the grid rests (rest) or could not run (x is a valid guess for
+// another solver)
 template <class VT>
-bool grid_solve(const GridPlan& g, GridBuffers& w, Model& m, const VT* A, const Schwarz* P, const double* dinv,
+bool grid_solve(const GridPlan& g, GridBuffers& w, GridRest& rest, Model& m, const VT* A, const Schwarz* P, const double* dinv,
                 const double* b, double* x, double tol, int64_t max_iter, int64_t* iterations, hoefem_status* status);
 
 // Buffers of allocation-free solves in a scratch of GRID_SCRATCH doubles

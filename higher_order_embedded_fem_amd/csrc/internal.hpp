@@ -233,7 +233,21 @@ struct GridBuffers {
     uint32_t phase = 0;    // exchanges done so far
     bool cleared = false;  // slots hold what phase says; else the next launch clears them first
 };
+// What is kept of launches that failed. A grid whose work-groups do not all become resident, because another
+// process's launches hold CUs of the device, takes about 2 s to give up: after a failure the next solves run the
+// two kernels, twice as many after every further one, until a launch ends well.
+struct GridRest {
+    static constexpr int FIRST = 64, MOST = 1 << 16;
+    int left = 0, last = 0;
+    bool resting() const { return left > 0; }
+    void pass() { left -= left > 0 ? 1 : 0; }  // a solve by the two kernels
+    void ended(bool well) {
+        last = well ? 0 : last == 0 ? FIRST : last < MOST ? 2 * last : MOST;
+        left = last;
+    }
+};
 struct GridWork : GridBuffers {
+    GridRest rest;
     void ensure(const GridPlan& g);
 
 private:
@@ -263,6 +277,10 @@ struct Model {
     NodePattern pattern;
     BlockScatter scatter;                         // element blocks -> pattern, color order
     GridPlan grid;                                // resident-grid solves with the Jacobi preconditioner
+    bool use_grid = true;                         // hoefem_resident_solver_set
+    int grid_polls = -1;
+    int64_t grid_solves = 0, grid_failures = 0;   // hoefem_resident_solver_stats
+    GridRest noalloc_rest;                        // of allocation-free solves
     double mass_reg = 0.0;
     int material = 0;                 // dev::MAT_* (elastic model wrapping Stable Neo-Hookean)
     double inversion_threshold = 0.0; // InvertibleMaterial threshold

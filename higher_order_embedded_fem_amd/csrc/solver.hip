@@ -1208,9 +1208,10 @@ static hoefem_status pcg_solve_t(Model& m, CgWork& w, const VT* Avals, const VT*
     // the flexible variant and a preconditioner of another model, whose plan splits that model's matrix, keep
     // the two kernels
     const GridPlan& grid = Pre ? Pre->grid : m.grid;
-    if (grid.serves(pat) && !two_kernels && !m.prof) {
+    if (grid.serves(pat) && m.use_grid && !two_kernels && !m.prof) {
         w.grid.ensure(grid);
-        if (grid_solve<VT>(grid, w.grid, m, Avals, Pre, Pre ? nullptr : w.diag_inv.get(), b, x, tol, max_iter, iterations, &st))
+        if (grid_solve<VT>(grid, w.grid, w.grid.rest, m, Avals, Pre, Pre ? nullptr : w.diag_inv.get(), b, x, tol, max_iter,
+                           iterations, &st))
             return st;
     }
 #define CG_CASE(ga, gb, j, f)                                                                            \
@@ -1357,10 +1358,11 @@ hoefem_status pcg_solve_noalloc(Model& m, const double* Avals, Schwarz* Pre, con
         if (read_and_clear_err(m) & KERR_ZERO_DIAG) throw Error(HOEFEM_ERROR_SINGULAR, "Diagonal matrix is not invertible.");
     }
     const GridPlan& grid = Pre ? Pre->grid : m.grid;
-    if (grid.serves(pat)) {
+    if (grid.serves(pat) && m.use_grid) {
         GridBuffers w = grid_scratch_buffers(grid, base + NA_VEC0, m.grid_result());
         hoefem_status st = HOEFEM_OK;
-        if (grid_solve<double>(grid, w, m, Avals, Pre, Pre ? nullptr : base + NA_DIAG, b, x, tol, max_iter, iterations, &st))
+        if (grid_solve<double>(grid, w, m.noalloc_rest, m, Avals, Pre, Pre ? nullptr : base + NA_DIAG, b, x, tol, max_iter,
+                               iterations, &st))
             return st;
     }
 #define NA_CASE(ga, gb, j) \

@@ -187,6 +187,16 @@ class ElasticityModel:
         (True) or device tensors (False, the default)."""
         check(_lib.load().hoefem_model_set_pointer_mode(self.h, 1 if host else 0))
 
+    def set_resident_solver(self, enable: bool = True, poll_limit: int = -1):
+        """Whether solves that fit the resident grid run on it (hoefem_resident_solver_set)."""
+        check(_lib.load().hoefem_resident_solver_set(self.h, int(enable), poll_limit))
+
+    def resident_solver_stats(self):
+        """Solves that the resident grid has ended, and launches that gave up."""
+        solves, failures = C.c_int64(), C.c_int64()
+        check(_lib.load().hoefem_resident_solver_stats(self.h, C.byref(solves), C.byref(failures)))
+        return solves.value, failures.value
+
     def set_material(self, material: StableNeoHookeanMaterial):
         """The elastic model used by this model's assembly and by simulations built on it."""
         check(_lib.load().hoefem_model_set_material(self.h, material.kind, material.threshold))

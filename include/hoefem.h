@@ -242,6 +242,18 @@ hoefem_status hoefem_schwarz_autotune(hoefem_schwarz* s, int32_t* lanes_per_node
 hoefem_status hoefem_sim_autotune(hoefem_sim* sim, int32_t* lanes_matrix, int32_t* lanes_preconditioner,
                                   double* candidate_us);
 
+/* The resident grid (no counterpart in the reference): solves of systems up to about 43,000 nodes run as one
+ * launch whose work-groups stay on the chip and wait for each other's values. The launches of one process are
+ * admitted so that all their work-groups are resident; launches of another process on the same GPU are not
+ * counted. A launch that cannot make progress gives up after about 2 s of polling, its solve runs the two-kernel
+ * iteration from there, and so do the next 64 solves of the same sim (or thread, for hoefem_pcg; or model, for
+ * hoefem_pcg_noalloc), twice as many after every further failure in a row.
+ * enable == 0: every solve of the model runs the two-kernel iteration. poll_limit: polls of a value before a
+ * launch gives up, negative for the default; with 0 every launch ends at once, unfinished. */
+hoefem_status hoefem_resident_solver_set(hoefem_model* model, int32_t enable, int32_t poll_limit);
+/* Solves of the model that the resident grid has ended, and launches that gave up, since it was created. */
+hoefem_status hoefem_resident_solver_stats(hoefem_model* model, int64_t* solves, int64_t* failures);
+
 /* Kernel timing (no counterpart in the reference, which times phases with coarse_prof scopes,
  * simulation_toolbox/src/fem/newton_cg.rs:685-764): when enabled, every launch of the CG
  * system-matrix kernel (fused direction update + SpMV + p.Ap) is bracketed by HIP events on

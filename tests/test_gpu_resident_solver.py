@@ -113,3 +113,74 @@ def test_sims_of_one_model_in_one_batch(schwarz):
     L.hoefem_batch_destroy(h)
     for (u, v), (ua, va) in zip(state, alone):
         assert torch.equal(u, ua) and torch.equal(v, va)
+
+
+# With a poll limit of 0 every launch ends at once, unfinished, as one does whose work-groups cannot all become
+# resident. Its solve is the two-kernel iteration's, bit for bit, and so are the 64 after it.
+@pytest.mark.parametrize("schwarz", [True, False])
+@pytest.mark.parametrize("entry", ["hoefem_pcg", "hoefem_pcg_noalloc"])
+def test_launch_that_gives_up(entry, schwarz):
+    from higher_order_embedded_fem_amd import fem
+
+    sc = scenes.cube_scene(5, scenes.TET10)
+    Jd, x_true, b = system(sc, 3)
+    L = _lib.load()
+    results = {}
+    for way in ("kernels", "gives_up"):
+        gm = fem.ElasticityModel(sc)
+        pre = None
+        if schwarz:
+            pre = fem.SchwarzPreconditioner.from_scene(gm, sc)
+            pre.update(Jd)
+
+        def solve():
+            x, its = torch.zeros_like(b), C.c_int64()
+            assert getattr(L, entry)(gm.h, Jd.data_ptr(), pre.h if pre else None, b.data_ptr(), x.data_ptr(), 1e-13,
+                                     20000, C.byref(its)) == 0
+            assert np.linalg.norm(x.cpu().numpy() - x_true) <= 1e-9 * np.linalg.norm(x_true)
+            return its.value, x
+
+        gm.set_resident_solver(enable=way != "kernels", poll_limit=0)
+        results[way] = solve()
+        if way == "kernels":
+            assert gm.resident_solver_stats() == (0, 0)
+            continue
+        assert results[way][0] == results["kernels"][0] and torch.equal(results[way][1], results["kernels"][1])
+        assert gm.resident_solver_stats() == (0, 1)
+        gm.set_resident_solver(poll_limit=-1)
+        for _ in range(64):
+            solve()
+        assert gm.resident_solver_stats() == (0, 1)
+        solve()
+        assert gm.resident_solver_stats() == (1, 1)
+        gm.set_resident_solver(poll_limit=0)  # the count starts again at the first failure after a good launch
+        solve()
+        gm.set_resident_solver(poll_limit=-1)
+        for _ in range(65):
+            solve()
+        assert gm.resident_solver_stats() == (2, 2)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_batch_launch_that_gives_up(precision):
+    """Scenes whose launch gives up in the middle of a step, and those that rest after it, end where the two-kernel
+    iteration takes them; a scene beside them keeps the resident grid."""
+    from higher_order_embedded_fem_amd import batch
+
+    scs = [scenes.cube_scene(c, scenes.TET10) for c in (3, 4, 5)]
+    kw = dict(newton_tolerance_factor=1e-6, mixed_precision=precision, autotune=False)
+    ref, st = batch.BatchedStepper(scs, **kw), batch.BatchedStepper(scs, **kw)
+    for k in (0, 1):
+        ref.models[k].set_resident_solver(enable=False)
+        st.models[k].set_resident_solver(poll_limit=0)
+    for _ in range(3):
+        a, b = ref.step(), st.step()
+        assert a["status"] == b["status"] == [0, 0, 0]
+        assert [s["cg_iterations"] for s in a["stats"]] == [s["cg_iterations"] for s in b["stats"]]
+    torch.cuda.synchronize()
+    for k in range(3):
+        assert torch.equal(ref.u[k], st.u[k]) and torch.equal(ref.v[k], st.v[k])
+    for k in (0, 1):
+        assert ref.models[k].resident_solver_stats() == (0, 0) and st.models[k].resident_solver_stats() == (0, 1)
+    solves = st.models[2].resident_solver_stats()
+    assert solves == ref.models[2].resident_solver_stats() and solves[0] >= 3 and solves[1] == 0
