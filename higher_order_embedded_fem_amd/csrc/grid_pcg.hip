@@ -41,11 +41,10 @@
 #include <cmath>
 #include <map>
 #include <mutex>
-#include <system_error>
-#include <thread>
 #include <type_traits>
 
 #include "grid_pcg.hpp"
+#include "host_threads.hpp"
 
 namespace hoefem {
 
@@ -694,17 +693,9 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
             }
         }
     };
-    {  // large patterns on a few host threads
-        const int nt = total < 100000 ? 1 : (int)std::min<int64_t>(std::max(1u, std::thread::hardware_concurrency()), 8);
-        std::vector<std::thread> th;
-        try {
-            for (int i = 1; i < nt; ++i) th.emplace_back(work, i, nt);
-        } catch (const std::system_error&) {  // fewer threads than asked for: their shares here
-            for (int i = (int)th.size() + 1; i < nt; ++i) work(i, nt);
-        }
-        work(0, nt);
-        for (std::thread& t : th) t.join();
-    }
+    // large patterns on a few host threads
+    const int nt = total < 100000 ? 1 : thread_count(total, 1);
+    run_on_threads(nt, [&](int i) { work(i, nt); });
     std::vector<int32_t> halo;
     std::vector<uint16_t> col, rp;
     lds_bytes = 0;

@@ -107,3 +107,31 @@ int main() {
     return 0;
 }
 """)
+
+
+def test_an_exception_in_a_worker_thread_reaches_the_caller(tmp_path):
+    run(tmp_path, CHECK + """
+#include <atomic>
+#include <new>
+#include <stdexcept>
+#include "host_threads.hpp"
+int main() {
+    for (int n : {1, 2, 5, 8})
+        for (int bad = -1; bad < n; ++bad) {  // the caller's own share is 0
+            std::atomic<int> ran{0};
+            bool caught = false;
+            try {
+                hoefem::run_on_threads(n, [&](int i) {
+                    ++ran;
+                    if (i == bad) throw std::bad_alloc();
+                });
+            } catch (const std::bad_alloc&) {
+                caught = true;
+            }
+            CHECK(ran == n);
+            CHECK(caught == (bad >= 0));
+        }
+    CHECK(hoefem::thread_count(0, 10) == 1 && hoefem::thread_count(1 << 30, 1) >= 1);
+    return 0;
+}
+""")
