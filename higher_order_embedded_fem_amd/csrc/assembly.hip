@@ -782,12 +782,11 @@ template <class TB, class TV>
 void launch_block_gather(const NodePattern& pat, const BlockScatter& sc, const TB* blocks, TV* values, int mode,
                          double c, const double* M, bool zero_first, hipStream_t s, const double* D2, double cd,
                          double cm, KernelProf* prof) {
-    const int64_t nblk = (int64_t)sc.dest.size();
+    const int64_t nblk = sc.ndest;
     if (nblk == 0) return;
     auto run = [&](auto kernel) {
         launch_timed(prof, kernel, dim3((unsigned)((3 * nblk + BS_THREADS - 1) / BS_THREADS)), dim3(BS_THREADS), 0, s, nblk,
-                     (const BlockScatter::Dest*)sc.d_dest.get(), (const int32_t*)sc.d_term_ptr.get(),
-                     (const uint32_t*)sc.d_term.get(), (const int32_t*)sc.d_term_row.get(), sc.row_stride, blocks,
+                     sc.d_dest, sc.d_term_ptr, sc.d_term, sc.d_term_row, sc.row_stride, blocks,
                      values, mode, c, M, zero_first ? 1 : 0, D2, cd, cm);
     };
     if (sc.row_stride)

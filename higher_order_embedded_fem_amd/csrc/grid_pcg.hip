@@ -39,6 +39,7 @@
 // falls back to the two-kernel path.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -572,8 +573,9 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
     if (nn == 0 || cus < 8) return;
     auto ka = [&](int64_t v) { return J.nptr[v + 1] - J.nptr[v]; };
     auto kp = [&](int64_t v) { return !P || P->diag_only[v] ? 0 : P->nptr[v + 1] - P->nptr[v]; };
-    int64_t total = 0;
-    for (int64_t v = 0; v < nn; ++v) total += ka(v) + kp(v);
+    std::vector<int64_t> psum(nn + 1, 0);  // P's blocks before each node; A's are J.nptr
+    for (int64_t v = 0; v < nn; ++v) psum[v + 1] = psum[v] + kp(v);
+    const int64_t total = J.nptr[nn] + psum[nn];
     const int wmax = std::min(cus, GRID_MAX_WG);
     if (nn > (int64_t)wmax * GRID_MAX_NODES || total > (int64_t)wmax * GRID_THREADS * GRID_MAX_SLOTS) return;
     auto share = [&](int64_t blocks) { return (total + GRID_THREADS * blocks - 1) / (GRID_THREADS * blocks); };
@@ -582,28 +584,29 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
     w = std::min<int64_t>(std::max<int64_t>((w + 7) / 8 * 8, 8), wmax);
     w = std::min(w, nn);
     // Contiguous node ranges: the fewest blocks per thread that w ranges allow, then the evenest ranges (blocks,
-    // and a few blocks' worth per node) with that many. Both by filling range after range up to a cap.
+    // and a few blocks' worth per node) with that many. Both by filling range after range up to a cap, a range's end
+    // by bisection.
     std::vector<int64_t> cut;
     auto fill = [&](int64_t slots, int64_t cap) -> bool {
         cut.assign(1, 0);
-        int64_t a = 0, p = 0;
-        for (int64_t v = 0; v < nn; ++v) {
-            const int64_t a1 = a + ka(v), p1 = p + kp(v), n1 = v + 1 - cut.back();
-            const bool full = n1 > GRID_MAX_NODES || a1 + p1 + 4 * n1 > cap ||
-                              (a1 + GRID_THREADS - 1) / GRID_THREADS + (p1 + GRID_THREADS - 1) / GRID_THREADS > slots;
-            if (full && n1 > 1) {
-                if ((int64_t)cut.size() == w) return false;
-                cut.push_back(v);
-                a = ka(v);
-                p = kp(v);
-            } else if (full) {
-                return false;  // a node by itself is too much
-            } else {
-                a = a1;
-                p = p1;
+        auto fits = [&](int64_t c, int64_t v) {  // the nodes [c, v) in one range
+            const int64_t a = J.nptr[v] - J.nptr[c], p = psum[v] - psum[c];
+            return a + p + 4 * (v - c) <= cap &&
+                   (a + GRID_THREADS - 1) / GRID_THREADS + (p + GRID_THREADS - 1) / GRID_THREADS <= slots;
+        };
+        if (!fits(0, 1)) return false;
+        for (int64_t c = 0; c < nn; c = cut.back()) {
+            if ((int64_t)cut.size() > w) return false;
+            int64_t lo = c + 1, hi = std::min(nn, c + GRID_MAX_NODES);  // a node by itself is a range in any case
+            while (lo < hi) {
+                const int64_t mid = (lo + hi + 1) / 2;
+                if (fits(c, mid))
+                    lo = mid;
+                else
+                    hi = mid - 1;
             }
+            cut.push_back(lo);
         }
-        cut.push_back(nn);
         return true;
     };
     int64_t slots = std::max<int64_t>(1, total / (w * GRID_THREADS));
@@ -696,8 +699,7 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
     // large patterns on a few host threads
     const int nt = total < 100000 ? 1 : thread_count(total, 1);
     run_on_threads(nt, [&](int i) { work(i, nt); });
-    std::vector<int32_t> halo;
-    std::vector<uint16_t> col, rp;
+    size_t nhalo = 0, ncol = 0, nrp = 0;
     lds_bytes = 0;
     max_slots = 0;
     ws = 0;
@@ -706,12 +708,12 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
         const Part& o = part[b];
         max_slots = std::max(max_slots, g.sA + g.sP);
         if (!o.fits || max_slots > GRID_MAX_SLOTS) return;
-        g.halo_off = (int64_t)halo.size();
-        g.rp_off = (int64_t)rp.size();
-        g.col_off = (int64_t)col.size();
-        halo.insert(halo.end(), o.halo.begin(), o.halo.end());
-        rp.insert(rp.end(), o.rp.begin(), o.rp.end());
-        col.insert(col.end(), o.col.begin(), o.col.end());
+        g.halo_off = (int64_t)nhalo;
+        g.rp_off = (int64_t)nrp;
+        g.col_off = (int64_t)ncol;
+        nhalo += o.halo.size();
+        nrp += o.rp.size();
+        ncol += o.col.size();
         lds_bytes = std::max(lds_bytes, sizeof(double) * (size_t)(3 * (2 * g.nown + g.nhA + g.nhP) + 3 * (o.parts + GRID_SPARE)));
     }
     if (lds_bytes > GRID_MAX_LDS) return;
@@ -725,11 +727,25 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
         g.ws_off = (int64_t)ws;
         ws += (size_t)std::max(0, g.sA + g.sP - GRID_REG_F64 - nlds) * 9 * GRID_THREADS;
     }
-    d_wg.upload(wg, s);
-    d_halo.upload(halo, s);
-    d_col.upload(col, s);
-    d_rp.upload(rp, s);
-    d_start.upload(start, s);
+    // one upload of everything (an allocation and a copy each would be half a small model's setup)
+    const size_t at_start = wg.size() * sizeof(GridWg), at_halo = at_start + start.size() * sizeof(GridStart);
+    const size_t at_col = at_halo + nhalo * sizeof(int32_t), at_rp = at_col + ncol * sizeof(uint16_t);
+    const size_t bytes = at_rp + nrp * sizeof(uint16_t);
+    std::unique_ptr<char[]> all(new char[bytes]);
+    std::memcpy(all.get(), wg.data(), at_start);
+    std::memcpy(all.get() + at_start, start.data(), at_halo - at_start);
+    for (int64_t b = 0; b < w; ++b) {
+        const Part& o = part[b];
+        std::copy(o.halo.begin(), o.halo.end(), reinterpret_cast<int32_t*>(all.get() + at_halo) + wg[b].halo_off);
+        std::copy(o.col.begin(), o.col.end(), reinterpret_cast<uint16_t*>(all.get() + at_col) + wg[b].col_off);
+        std::copy(o.rp.begin(), o.rp.end(), reinterpret_cast<uint16_t*>(all.get() + at_rp) + wg[b].rp_off);
+    }
+    d_all.upload(all.get(), bytes, s);
+    d_wg = reinterpret_cast<const GridWg*>(d_all.get());
+    d_start = reinterpret_cast<const GridStart*>(d_all.get() + at_start);
+    d_halo = reinterpret_cast<const int32_t*>(d_all.get() + at_halo);
+    d_col = reinterpret_cast<const uint16_t*>(d_all.get() + at_col);
+    d_rp = reinterpret_cast<const uint16_t*>(d_all.get() + at_rp);
     ndof = 3 * nn;
     W = (int)w;
     if (exchange() + saved() + GRID_STATE_WORDS + (int64_t)ws > GRID_SCRATCH) d_spill.ensure(ws);
@@ -834,11 +850,11 @@ template <class VT>
 GridSeg<VT> grid_segment(const GridPlan& g, const GridBuffers& w, Model& m, const VT* A, const Schwarz* P,
                          const double* dinv, const double* b, double* x, double tol, int64_t max_iter) {
     GridSeg<VT> S{};
-    S.wg = g.d_wg.get();
-    S.halo = g.d_halo.get();
-    S.col = g.d_col.get();
-    S.rp = g.d_rp.get();
-    S.start = g.d_start.get();
+    S.wg = g.d_wg;
+    S.halo = g.d_halo;
+    S.col = g.d_col;
+    S.rp = g.d_rp;
+    S.start = g.d_start;
     S.jnptr = m.pattern.d_nptr.get();
     S.jrowptr = m.pattern.d_rowptr.get();
     S.A = A;

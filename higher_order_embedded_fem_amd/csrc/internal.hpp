@@ -120,6 +120,8 @@ struct NodePattern {
     int64_t nnz() const { return (int64_t)col.size(); }
     int64_t ndof() const { return 3 * num_nodes; }
     int32_t find(int32_t a, int32_t b) const;  // local index of b in nbr(a), or -1
+    // slot[i m + j] = find(node i, node j) for the m nodes of a set
+    void find_pairs(const int32_t* set, int m, int32_t* slot) const;
     void upload(hipStream_t s);
 };
 
@@ -134,6 +136,7 @@ std::vector<std::vector<int32_t>> greedy_coloring(int64_t nsets, const int64_t* 
 
 // Color-ordered incidence of dense blocks ("element matrices") into a node pattern; shared
 // by the stiffness / mass assembly and the Schwarz preconditioner assembly.
+constexpr int64_t SETUP_ENTRIES = 1 << 15;  // block entries worth a host thread (about 1 ms of one)
 struct BlockScatter {
     int64_t nblocks = 0;
     int max_m = 0;
@@ -150,13 +153,13 @@ struct BlockScatter {
     struct Dest {
         int32_t pos, row;  // first value, distance of the rows (0: a diagonal-only node's entry, not written)
     };
-    std::vector<Dest> dest;
-    std::vector<int32_t> term_ptr, term_row;
-    std::vector<uint32_t> term;
+    int64_t ndest = 0;
     int row_stride = 0;
-    DevBuf<Dest> d_dest;
-    DevBuf<int32_t> d_term_ptr, d_term_row;
-    DevBuf<uint32_t> d_term;
+    std::vector<int32_t> lists;  // dest (two words each), term_ptr, term, term_row
+    DevBuf<int32_t> d_lists;
+    const Dest* d_dest = nullptr;
+    const int32_t *d_term_ptr = nullptr, *d_term_row = nullptr;
+    const uint32_t* d_term = nullptr;
     DevBuf<int32_t> d_m, d_inc_ptr, d_inc_blk, d_inc_loc;
     DevBuf<int64_t> d_val_off, d_slot_off;
     void build(const NodePattern& pat, int64_t nblocks, const int64_t* off, const int32_t* nodes,
@@ -213,10 +216,11 @@ struct GridPlan {
     int W = 0, max_slots = 0, nlds = 0, blk_off = 0;
     int64_t ndof = 0;
     size_t lds_bytes = 0, ws = 0;  // ws: doubles for the blocks past the registers and the LDS
-    DevBuf<GridWg> d_wg;
-    DevBuf<int32_t> d_halo;
-    DevBuf<uint16_t> d_col, d_rp;
-    DevBuf<GridStart> d_start;
+    DevBuf<char> d_all;   // the arrays below
+    const GridWg* d_wg = nullptr;
+    const GridStart* d_start = nullptr;
+    const int32_t* d_halo = nullptr;
+    const uint16_t *d_col = nullptr, *d_rp = nullptr;
     DevBuf<double> d_spill;  // those blocks in allocation-free solves, where that path's scratch is too small
     void build(const NodePattern& J, const NodePattern* P, int cus, hipStream_t s);
     // the plan is for this matrix pattern (a preconditioner may come from another model's) and fits the chip

@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "host_threads.hpp"
 #include "internal.hpp"
 
 namespace hoefem {
@@ -42,11 +43,15 @@ void schwarz_setup(Schwarz& s, Model& m, int64_t nsub, const int64_t* off, const
     s.large.clear();
     std::vector<int64_t> panel_off;
     int64_t panel_total = 0;
+    const int nt = thread_count((int64_t)s.jslot.size(), SETUP_ENTRIES);
+    run_on_threads(nt, [&](int t) {
+        for (int64_t b = t * nsub / nt; b < (t + 1) * nsub / nt; ++b) {
+            m.pattern.find_pairs(s.nodes.data() + s.off[b], (int)(s.off[b + 1] - s.off[b]),
+                                 s.jslot.data() + s.scatter.slot_off[b]);
+        }
+    });
     for (int64_t b = 0; b < nsub; ++b) {
-        const int32_t* g = s.nodes.data() + s.off[b];
         const int mb = (int)(s.off[b + 1] - s.off[b]);
-        for (int a = 0; a < mb; ++a)
-            for (int c = 0; c < mb; ++c) s.jslot[s.scatter.slot_off[b] + (int64_t)a * mb + c] = m.pattern.find(g[a], g[c]);
         if (3 * mb > SCHWARZ_SMALL_DIM) {
             s.large.push_back((int32_t)b);
             s.large_max_dim = std::max(s.large_max_dim, 3 * mb);

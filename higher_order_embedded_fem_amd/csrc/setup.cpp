@@ -6,6 +6,7 @@
 #include <mutex>
 #include <numeric>
 
+#include "host_threads.hpp"
 #include "internal.hpp"
 
 namespace hoefem {
@@ -78,6 +79,22 @@ int32_t NodePattern::find(int32_t a, int32_t b) const {
     const int32_t* it = std::lower_bound(lo, hi, b);
     if (it == hi || *it != b) return -1;
     return (int32_t)(it - lo);
+}
+
+void NodePattern::find_pairs(const int32_t* set, int m, int32_t* slot) const {
+    std::vector<std::pair<int32_t, int32_t>> sorted(m);  // node, place in the set
+    for (int j = 0; j < m; ++j) sorted[j] = {set[j], j};
+    std::sort(sorted.begin(), sorted.end());
+    for (int i = 0; i < m; ++i) {  // the set's nodes and the row's neighbours are both in order
+        const int32_t *nb = ncol.data() + nptr[set[i]], *end = ncol.data() + nptr[set[i] + 1], *p = nb;
+        for (const auto& [node, j] : sorted) {
+            if (end - p > 16)
+                p = std::lower_bound(p, end, node);
+            else
+                while (p < end && *p < node) ++p;
+            slot[(int64_t)i * m + j] = p < end && *p == node ? (int32_t)(p - nb) : -1;
+        }
+    }
 }
 
 void NodePattern::upload(hipStream_t s) {
@@ -287,15 +304,15 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
         slot_off[b + 1] = slot_off[b] + (int64_t)m[b] * m[b];
     }
     slot.resize(slot_off[nb]);
-    for (int64_t b = 0; b < nb; ++b) {
-        const int32_t* g = nodes + off[b];
-        for (int a = 0; a < m[b]; ++a)
-            for (int c = 0; c < m[b]; ++c) {
-                const int32_t k = pat.find(g[a], g[c]);
-                if (k < 0) throw Error(HOEFEM_ERROR_PATTERN, "block entry missing from CSR pattern");
-                slot[slot_off[b] + (int64_t)a * m[b] + c] = k;
-            }
-    }
+    const int nt = thread_count(slot_off[nb], SETUP_ENTRIES);
+    run_on_threads(nt, [&](int t) {
+        for (int64_t b = t * nb / nt; b < (t + 1) * nb / nt; ++b) {
+            int32_t* sl = slot.data() + slot_off[b];
+            pat.find_pairs(nodes + off[b], m[b], sl);
+            if (std::find(sl, sl + (int64_t)m[b] * m[b], -1) != sl + (int64_t)m[b] * m[b])
+                throw Error(HOEFEM_ERROR_PATTERN, "block entry missing from CSR pattern");
+        }
+    });
     inc_ptr.assign(pat.num_nodes + 1, 0);
     for (int l = 0; l < ncolor_lists; ++l)
         for (const auto& color : color_lists[l])
@@ -323,45 +340,60 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
     const int64_t nblk = pat.ncol.size(), nterms = slot_off[nb];
     if (nterms > INT32_MAX || val_off[nb] / 3 > UINT32_MAX)
         throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "too many element block entries");
-    dest.resize(nblk);
-    term_ptr.assign(nblk + 1, 0);
-    term.resize(nterms);
-    term_row.resize(row_stride ? 0 : nterms);
-    std::vector<int32_t> at;
-    for (int64_t v = 0; v < pat.num_nodes; ++v) {
-        const int32_t b0 = pat.nptr[v], k = pat.nptr[v + 1] - b0;
-        for (int j = 0; j < k; ++j)
-            dest[b0 + j] = pat.diag_only[v] ? Dest{0, 0} : Dest{pat.rowptr[3 * v] + 3 * j, 3 * k};
-        int32_t* count = term_ptr.data() + b0 + 1;
-        for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
-            const int32_t b = inc_blk[it], mb = m[b];
-            const int32_t* sl = slot.data() + slot_off[b] + (int64_t)inc_loc[it] * mb;
-            for (int c = 0; c < mb; ++c) count[sl[c]]++;
-        }
-        at.resize(k);
-        for (int j = 0; j < k; ++j) {
-            at[j] = term_ptr[b0 + j];
-            term_ptr[b0 + j + 1] += term_ptr[b0 + j];
-        }
-        for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
-            const int32_t b = inc_blk[it], mb = m[b], a = inc_loc[it];
-            const int32_t* sl = slot.data() + slot_off[b] + (int64_t)a * mb;
-            const uint32_t base = (uint32_t)(val_off[b] / 3 + (int64_t)(3 * a) * mb);  // of row 3 a, over 3
-            for (int c = 0; c < mb; ++c) {
-                const int32_t q = at[sl[c]]++;
-                term[q] = base + c;
-                if (!row_stride) term_row[q] = 3 * mb;
+    ndest = nblk;
+    lists.resize(3 * nblk + 1 + nterms * (row_stride ? 1 : 2));
+    Dest* dest = reinterpret_cast<Dest*>(lists.data());
+    int32_t* term_ptr = lists.data() + 2 * nblk;
+    uint32_t* term = reinterpret_cast<uint32_t*>(term_ptr + nblk + 1);
+    int32_t* term_row = term_ptr + nblk + 1 + nterms;  // of blocks of several sizes
+    term_ptr[0] = 0;
+    const int64_t nn = pat.num_nodes;
+    std::vector<int32_t> first(nn + 1, 0);  // terms of the nodes before
+    for (int64_t v = 0; v < nn; ++v) {
+        first[v + 1] = first[v];
+        for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) first[v + 1] += m[inc_blk[it]];
+    }
+    run_on_threads(nt, [&](int t) {
+        std::vector<int32_t> at;
+        for (int64_t v = t * nn / nt; v < (t + 1) * nn / nt; ++v) {
+            const int32_t b0 = pat.nptr[v], k = pat.nptr[v + 1] - b0;
+            for (int j = 0; j < k; ++j)
+                dest[b0 + j] = pat.diag_only[v] ? Dest{0, 0} : Dest{pat.rowptr[3 * v] + 3 * j, 3 * k};
+            at.assign(k, 0);
+            for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
+                const int32_t b = inc_blk[it], mb = m[b];
+                const int32_t* sl = slot.data() + slot_off[b] + (int64_t)inc_loc[it] * mb;
+                for (int c = 0; c < mb; ++c) at[sl[c]]++;
+            }
+            int32_t end = first[v];
+            for (int j = 0; j < k; ++j) {
+                const int32_t count = at[j];
+                at[j] = end;
+                end += count;
+                term_ptr[b0 + j + 1] = end;
+            }
+            for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
+                const int32_t b = inc_blk[it], mb = m[b], a = inc_loc[it];
+                const int32_t* sl = slot.data() + slot_off[b] + (int64_t)a * mb;
+                const uint32_t base = (uint32_t)(val_off[b] / 3 + (int64_t)(3 * a) * mb);  // of row 3 a, over 3
+                for (int c = 0; c < mb; ++c) {
+                    const int32_t q = at[sl[c]]++;
+                    term[q] = base + c;
+                    if (!row_stride) term_row[q] = 3 * mb;
+                }
             }
         }
-    }
+    });
 }
 
 void BlockScatter::upload(hipStream_t s) {
     d_m.upload(m, s);
-    d_dest.upload(dest, s);
-    d_term_ptr.upload(term_ptr, s);
-    d_term.upload(term, s);
-    if (!row_stride) d_term_row.upload(term_row, s);
+    d_lists.upload(lists, s);
+    std::vector<int32_t>().swap(lists);
+    d_dest = reinterpret_cast<const Dest*>(d_lists.get());
+    d_term_ptr = d_lists.get() + 2 * ndest;
+    d_term = reinterpret_cast<const uint32_t*>(d_term_ptr + ndest + 1);
+    d_term_row = d_term_ptr + ndest + 1 + slot_off[nblocks];
     d_inc_ptr.upload(inc_ptr, s);
     d_inc_blk.upload(inc_blk, s);
     d_inc_loc.upload(inc_loc, s);
