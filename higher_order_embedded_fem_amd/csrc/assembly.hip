@@ -7,6 +7,7 @@
 // node's row block.
 #include <type_traits>
 #include <algorithm>
+#include <mutex>
 
 #include "fem_device.hpp"
 #include "gather_device.hpp"
@@ -918,18 +919,51 @@ void material_energy(double mu, double lambda, int64_t nq, const double* F, doub
     HIP_CHECK(hipDeviceSynchronize());
 }
 
+// An error word in host memory that a kernel writes, one per thread: a thread that ends leaves it to the next one
+// (at most KEPT are kept). Taken and given back for each call it cost 1.4 us of 71.
+class HostWord {
+public:
+    HostWord() {
+        std::lock_guard<std::mutex> lock(pool().mu);
+        if (!pool().free.empty()) {
+            word_ = std::move(pool().free.back());
+            pool().free.pop_back();
+        } else {
+            word_.reset(new PinnedBuf<int>(1, hipHostMallocCoherent));
+        }
+    }
+    ~HostWord() {
+        std::lock_guard<std::mutex> lock(pool().mu);
+        if (pool().free.size() < KEPT) pool().free.push_back(std::move(word_));
+    }
+    HostWord(const HostWord&) = delete;
+    HostWord& operator=(const HostWord&) = delete;
+    int* get() const { return word_->p; }
+
+private:
+    static constexpr size_t KEPT = 16;
+    struct Pool {
+        std::mutex mu;
+        std::vector<std::unique_ptr<PinnedBuf<int>>> free;
+        Pool() { free.reserve(KEPT); }
+    };
+    static Pool& pool() {
+        static Pool* p = new Pool;  // outlives the process's static objects, among them the HIP runtime's
+        return *p;
+    }
+    std::unique_ptr<PinnedBuf<int>> word_;
+};
+
 void material_eval(int mat, double thr, double mu_r, double lambda_r, int64_t nq, const double* F, double* P,
                    double* dPdF) {
-    // the error word, written by the kernel into host memory: one per thread, for the life of the process
-    static thread_local PinnedBuf<int>* err = nullptr;
-    if (!err) err = new PinnedBuf<int>(1, hipHostMallocCoherent);
-    volatile int* h = err->p;
+    static thread_local HostWord err;
+    volatile int* h = err.get();
     *h = 0;
     if (nq > 0) {
         const unsigned g = (unsigned)((nq + MT_PTS - 1) / MT_PTS);
         const uint32_t lds = (uint32_t)(sizeof(double) * MT_PTS * (dPdF ? 81 : 9));
         HOEFEM_MATERIAL_DISPATCH(mat, hipLaunchKernelGGL(k_material<MK>, dim3(g), dim3(MT_PTS), lds, nullptr, thr, mu_r,
-                                                         lambda_r, nq, F, P, dPdF, err->p));
+                                                         lambda_r, nq, F, P, dPdF, err.get()));
         check_launch("k_material");
     }
     HIP_CHECK(hipStreamSynchronize(nullptr));

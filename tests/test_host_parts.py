@@ -2,8 +2,11 @@
 
 import os
 import subprocess
+import sys
 
-CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "higher_order_embedded_fem_amd", "csrc")
+HERE = os.path.dirname(os.path.abspath(__file__))
+PACKAGE = os.path.join(os.path.dirname(HERE), "higher_order_embedded_fem_amd")
+CSRC = os.path.join(PACKAGE, "csrc")
 
 
 def run(tmp_path, source):
@@ -135,3 +138,34 @@ int main() {
     return 0;
 }
 """)
+
+
+def test_material_calls_of_short_lived_threads_leave_nothing_behind(tmp_path):
+    """Threads one after the other use the same few pinned error words, and of many at a time a bounded number is kept
+    (a thread may still be about to give its word back when join returns)."""
+    stub = tmp_path / "libstub.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(stub), os.path.join(HERE, "hip_stub.c")], check=True)
+    script = f"""
+import ctypes as C, threading, time
+S = C.CDLL({str(stub)!r}, mode=C.RTLD_GLOBAL)  # found before the HIP library's symbols
+L = C.CDLL({os.path.join(PACKAGE, "libhoefem.so")!r})
+L.hoefem_material_eval.argtypes = [C.c_double, C.c_double, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]
+buf = (C.c_double * 90)()
+def call(times=1):
+    for _ in range(times):
+        assert L.hoefem_material_eval(1.0, 1.0, 1, C.addressof(buf), C.addressof(buf), None) == 0
+before = S.stub_pinned_now()
+for _ in range(50):
+    t = threading.Thread(target=call)
+    t.start()
+    t.join()
+    time.sleep(0.002)
+assert S.stub_pinned_total() - before <= 16, S.stub_pinned_total()
+ts = [threading.Thread(target=call, args=(200,)) for _ in range(40)]
+for t in ts: t.start()
+for t in ts: t.join()
+time.sleep(0.2)
+assert S.stub_pinned_now() - before <= 16, S.stub_pinned_now()
+"""
+    r = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
