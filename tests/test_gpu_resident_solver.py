@@ -184,3 +184,49 @@ def test_batch_launch_that_gives_up(precision):
         assert ref.models[k].resident_solver_stats() == (0, 0) and st.models[k].resident_solver_stats() == (0, 1)
     solves = st.models[2].resident_solver_stats()
     assert solves == ref.models[2].resident_solver_stats() and solves[0] >= 3 and solves[1] == 0
+
+
+def two_jacobi_steps(rp, col, J, diag, b):
+    """x after two iterations of Jacobi-preconditioned CG from zero, in FP64."""
+    x, r = np.zeros_like(b), b.copy()
+    z = r / diag
+    p, ztr = z.copy(), z @ r
+    for _ in range(2):
+        ap = np.add.reduceat(np.append(J * p[col], 0.0), rp[:-1])
+        alpha = ztr / (p @ ap)
+        x += alpha * p
+        r -= alpha * ap
+        z = r / diag
+        ztr, old = z @ r, ztr
+        p = z + ztr / old * p
+    return x
+
+
+# The second iterate holds the rounding of one product of the FP32 operator. Both iterations round its operands alike;
+# the resident grid rounds once per 3x3 block and row, the two kernels once per block and then along their lanes' sums.
+@pytest.mark.parametrize("cells,element", [(5, scenes.TET10), (12, scenes.TET10), (15, scenes.TET10), (24, scenes.TET4)])
+def test_fp32_products_are_no_less_accurate_than_the_two_kernels(cells, element):
+    from higher_order_embedded_fem_amd import fem
+
+    sc = scenes.cube_scene(cells, element)
+    gm = fem.ElasticityModel(sc)
+    sim = fem.NewtonCgIntegrator(gm, sc, schwarz=False, cg_tolerance=1e-15, cg_max_iter=2, mixed_precision=3)
+    zero = torch.zeros(sc.ndof, dtype=torch.float64, device="cuda")
+    sim.set_state(0.0, zero, zero)
+    sim.init_solve_jacobian_combination(-sc.dt * sc.dt, None)
+    b = np.random.default_rng(cells).standard_normal(sc.ndof)
+    b.reshape(-1, 3)[sc.dirichlet_nodes] = 0.0
+    error = {}
+    for enable in (False, True):
+        gm.set_resident_solver(enable=enable)
+        sol = torch.zeros_like(zero)
+        assert sim.solve_jacobian_combination(sol, dev(b)) == 2
+        if not error:
+            rp, col = gm.pattern()
+            J = sim.jacobian().cpu().numpy()  # the FP32 values
+            rows = np.repeat(np.arange(sc.ndof), np.diff(rp))
+            exact = two_jacobi_steps(rp, col, J, J[rows == col], b)
+        error[enable] = np.linalg.norm(sol.cpu().numpy() - exact) / np.linalg.norm(exact)
+    assert gm.resident_solver_stats() == (1, 0)
+    print(f"two kernels {error[False]:.2e}, resident grid {error[True]:.2e}")
+    assert error[True] <= error[False] < 1e-6
