@@ -194,7 +194,7 @@ def _kernel_kib(rows):
             cga.setdefault(int(m.group(1)), []).append(v)
         elif "k_element_stiffness_tw" in name:
             out["tangent"].append(v)
-        elif "k_block_sum" in name and ("k_element_stiffness" in prev):
+        elif ("k_block_sum" in name or "k_block_gather_pf" in name) and "k_element_stiffness" in prev:
             out["jgather"].append(v)
         elif "k_element_forces" in name:
             out["forces"].append(v)

@@ -527,6 +527,108 @@ __global__ __launch_bounds__(BS_THREADS) void k_block_sum(
     values[o2] = combine(s2, o2, m2);
 }
 
+// The same sum with a wavefront per pattern node: it walks the node's incident blocks in color order and adds
+// their three rows, which are contiguous, into the node's rows in LDS. Where the staging is read from memory and an
+// element's rows are as long as Hex20's, whole rows need fewer bytes than the lists' 24-byte pieces and their
+// places (BlockScatter::by_rows): J = M + dt^2 K of the Hex20 cylinder of 31 cells 103 us and 327 MB, by lists 112 and
+// 364; of 36 cells 164 and 178 us, of 24 cells 58 and 56. Bound by those bytes.
+// The incident blocks' metadata is held one incidence per lane (moved by shuffles instead of loaded per block) and
+// each block's row values and slots are loaded one block ahead, so a node row's blocks cost one memory latency
+// between them instead of three. For at most 64 incidences, blocks of at most 28 nodes (3 rows x 3m <= 256 values,
+// four per lane) and rows that fit the LDS.
+constexpr int GP_VALS = 4;
+template <class TB, class TV>
+__global__ __launch_bounds__(64) void k_block_gather_pf(
+    const int32_t* __restrict__ nptr, const int32_t* __restrict__ rowptr, const uint8_t* __restrict__ diag_only,
+    const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_blk, const int32_t* __restrict__ inc_loc,
+    const int32_t* __restrict__ msz, const int64_t* __restrict__ val_off, const int64_t* __restrict__ slot_off,
+    const int32_t* __restrict__ slot, const TB* __restrict__ blocks, TV* __restrict__ values, int mode,
+    double c, const double* __restrict__ M, int zero_first, const double* __restrict__ D2, double cd, double cm) {
+    extern __shared__ double s_rb[];
+    const int64_t v = blockIdx.x;
+    const int t = threadIdx.x;
+    if (diag_only[v]) return;
+    const int k = nptr[v + 1] - nptr[v];
+    if (k == 0) return;
+    const int rw = 3 * k, R = 3 * rw;
+    const int64_t r0 = rowptr[3 * v];
+    const int i0 = inc_ptr[v], ninc = inc_ptr[v + 1] - i0;
+    // lane j holds incidence j (at most 64, checked by the launch)
+    int a_l = 0, mb_l = 0;
+    int64_t vo_l = 0, so_l = 0;
+    if (t < ninc) {
+        const int b = inc_blk[i0 + t];
+        a_l = inc_loc[i0 + t];
+        mb_l = msz[b];
+        vo_l = val_off[b];
+        so_l = slot_off[b];
+    }
+    for (int idx = t; idx < R; idx += 64) s_rb[idx] = (zero_first || mode == 1) ? 0.0 : (double)values[r0 + idx];
+    // incidence j's row values and slots: every lane loads (a lane past the block's 3 x 3m values
+    // re-reads its first one and does not use it), so the loads in flight are counted statically and
+    // adding one incidence waits only for its own loads
+    auto fetch = [&](int j, double* vv, int* ss, int& bwj) {
+        const int a = __shfl(a_l, j, 64), mb = __shfl(mb_l, j, 64);
+        const int64_t vo = __shfl(vo_l, j, 64), so = __shfl(so_l, j, 64);
+        const int bw = 3 * mb;
+        bwj = bw;
+        const TB* base = blocks + vo + (int64_t)(3 * a) * bw;
+        const int32_t* sl = slot + so + (int64_t)a * mb;
+#pragma unroll
+        for (int q = 0; q < GP_VALS; ++q) {
+            const int idx = t + 64 * q;
+            const int id = idx < 3 * bw ? idx : 0;
+            vv[q] = (double)base[id];
+            ss[q] = sl[(id % bw) / 3];
+        }
+    };
+    // two incidence buffers used in turn (no register copy between them, which would wait for the
+    // loads): the next incidence's loads are in flight while this one's values are added
+    double av[GP_VALS] = {0.0, 0.0, 0.0, 0.0}, bv[GP_VALS] = {0.0, 0.0, 0.0, 0.0};
+    int as[GP_VALS] = {0, 0, 0, 0}, bs[GP_VALS] = {0, 0, 0, 0};
+    int abw = 0, bbw = 0;
+    auto add = [&](const double* vv, const int* ss, int bw) {
+#pragma unroll
+        for (int q = 0; q < GP_VALS; ++q) {
+            const int idx = t + 64 * q;
+            if (idx < 3 * bw) {
+                const int i = idx / bw, cc = idx % bw;
+                s_rb[i * rw + 3 * ss[q] + cc % 3] += vv[q];
+            }
+        }
+    };
+    // The work-group is one wavefront, whose LDS accesses take effect in program order: the row's sums
+    // need no s_barrier, only a compiler barrier that keeps the LDS accesses of consecutive incidences
+    // in order (an s_barrier's fence would also wait for the loads of the incidence ahead). The fetches
+    // are unconditional inside the block (the last incidence again past the end), so every path reaches
+    // the loop with the same loads in flight and each addition waits only for its own incidence.
+    if (ninc > 0) {
+        fetch(0, av, as, abw);
+        __builtin_amdgcn_wave_barrier();
+        for (int j = 0; j < ninc; j += 2) {
+            fetch(min(j + 1, ninc - 1), bv, bs, bbw);
+            add(av, as, abw);
+            __builtin_amdgcn_wave_barrier();
+            fetch(min(j + 2, ninc - 1), av, as, abw);
+            if (j + 1 < ninc) add(bv, bs, bbw);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    for (int idx = t; idx < R; idx += 64) {
+        const int64_t o = r0 + idx;
+        const double sum = s_rb[idx];
+        if (mode == 0)
+            values[o] = (TV)sum;
+        else {
+            double v2 = 0.0;  // stiffness, damping, mass (system_assembly.rs:197-235)
+            v2 += c * sum;
+            if (D2) v2 += cd * D2[o];
+            if (M) v2 += cm * M[o];
+            values[o] = (TV)v2;
+        }
+    }
+}
+
 // f += sum of element force blocks in color order (one thread per DOF)
 __global__ __launch_bounds__(128) void k_force_gather(int64_t nn, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_blk,
                                const int32_t* __restrict__ inc_loc, int n, const double* __restrict__ fe,
@@ -793,6 +895,19 @@ void launch_block_gather(const NodePattern& pat, const BlockScatter& sc, const T
                          double cm, KernelProf* prof) {
     const int64_t nblk = sc.ndest;
     if (nblk == 0) return;
+    if constexpr (sizeof(TB) == sizeof(double))
+        if (sc.by_rows) {
+            const size_t lds = (size_t)9 * pat.max_nbr * sizeof(double);
+            launch_timed(prof, k_block_gather_pf<TB, TV>, dim3((unsigned)pat.num_nodes), dim3(64), (uint32_t)lds, s,
+                         (const int32_t*)pat.d_nptr.get(), (const int32_t*)pat.d_rowptr.get(),
+                         (const uint8_t*)pat.d_diag_only.get(), (const int32_t*)sc.d_inc_ptr.get(),
+                         (const int32_t*)sc.d_inc_blk.get(), (const int32_t*)sc.d_inc_loc.get(),
+                         (const int32_t*)sc.d_m.get(), (const int64_t*)sc.d_val_off.get(),
+                         (const int64_t*)sc.d_slot_off.get(), (const int32_t*)sc.d_slot.get(), blocks, values, mode, c,
+                         M, zero_first ? 1 : 0, D2, cd, cm);
+            check_launch("k_block_gather_pf");
+            return;
+        }
     auto run = [&](auto kernel) {
         launch_timed(prof, kernel, dim3((unsigned)((3 * nblk + BS_THREADS - 1) / BS_THREADS)), dim3(BS_THREADS), 0, s, nblk,
                      sc.d_dest, sc.d_term_ptr, sc.d_term, sc.d_term_row, sc.row_stride, blocks,

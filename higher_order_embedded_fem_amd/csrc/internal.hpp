@@ -139,13 +139,11 @@ std::vector<std::vector<int32_t>> greedy_coloring(int64_t nsets, const int64_t* 
 constexpr int64_t SETUP_ENTRIES = 1 << 15;  // block entries worth a host thread (about 1 ms of one)
 struct BlockScatter {
     int64_t nblocks = 0;
-    int max_m = 0;
     std::vector<int32_t> m;         // nodes per block
     std::vector<int64_t> val_off;   // offset of block b's (3m)^2 dense values in the staging
     std::vector<int64_t> slot_off;  // offset of block b's m*m slot table
     std::vector<int32_t> slot;      // slot[slot_off[b] + a*m + c] = local index of node c in nbr(node a)
     std::vector<int32_t> inc_ptr;   // per pattern node
-    int max_inc = 0;                // most incident blocks of one node
     std::vector<int32_t> inc_blk, inc_loc;  // incident (block, local node) in color order
     // The same incidences seen from the pattern's node blocks (ncol entries): where block B's 3x3 values go,
     // and where its terms lie in the staging, in color order: term q in [term_ptr[B], term_ptr[B + 1]) has its
@@ -160,7 +158,8 @@ struct BlockScatter {
     const Dest* d_dest = nullptr;
     const int32_t *d_term_ptr = nullptr, *d_term_row = nullptr;
     const uint32_t* d_term = nullptr;
-    DevBuf<int32_t> d_m, d_inc_ptr, d_inc_blk, d_inc_loc;
+    bool by_rows = false;  // FP64 blocks are summed by k_block_gather_pf, which reads slot
+    DevBuf<int32_t> d_m, d_slot, d_inc_ptr, d_inc_blk, d_inc_loc;
     DevBuf<int64_t> d_val_off, d_slot_off;
     void build(const NodePattern& pat, int64_t nblocks, const int64_t* off, const int32_t* nodes,
                const std::vector<std::vector<int32_t>>* colors, int ncolor_lists);

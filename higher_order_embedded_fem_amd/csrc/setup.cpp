@@ -296,10 +296,8 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
     val_off.resize(nb + 1);
     slot_off.resize(nb + 1);
     val_off[0] = slot_off[0] = 0;
-    max_m = 0;
     for (int64_t b = 0; b < nb; ++b) {
         m[b] = (int32_t)(off[b + 1] - off[b]);
-        max_m = std::max(max_m, m[b]);
         val_off[b + 1] = val_off[b] + 9 * (int64_t)m[b] * m[b];
         slot_off[b + 1] = slot_off[b] + (int64_t)m[b] * m[b];
     }
@@ -318,7 +316,7 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
         for (const auto& color : color_lists[l])
             for (int32_t b : color)
                 for (int a = 0; a < m[b]; ++a) inc_ptr[nodes[off[b] + a] + 1]++;
-    max_inc = 0;
+    int max_inc = 0;  // most incident blocks of one node
     for (int64_t v = 0; v < pat.num_nodes; ++v) max_inc = std::max(max_inc, inc_ptr[v + 1]);
     for (int64_t v = 0; v < pat.num_nodes; ++v) inc_ptr[v + 1] += inc_ptr[v];
     inc_blk.resize(inc_ptr[pat.num_nodes]);
@@ -337,6 +335,10 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
     row_stride = nb > 0 ? 3 * m[0] : 0;
     for (int64_t b = 0; b < nb; ++b)
         if (3 * m[b] != row_stride) row_stride = 0;
+    // Blocks of 20 nodes past the caches, few of them at a node (Hex20): see k_block_gather_pf. Elsewhere the lists are
+    // faster: Tet20, up to 24 elements at a node, 171 us against 219 (cube of 12); Hex27 340 against 416 (36 cells).
+    constexpr int64_t BY_ROWS_BYTES = 128 << 20;
+    by_rows = row_stride == 60 && (int64_t)sizeof(double) * val_off[nb] > BY_ROWS_BYTES && max_inc <= 8 && pat.max_nbr <= 896;
     const int64_t nblk = pat.ncol.size(), nterms = slot_off[nb];
     if (nterms > INT32_MAX || val_off[nb] / 3 > UINT32_MAX)
         throw Error(HOEFEM_ERROR_INVALID_ARGUMENT, "too many element block entries");
@@ -388,6 +390,7 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
 
 void BlockScatter::upload(hipStream_t s) {
     d_m.upload(m, s);
+    if (by_rows) d_slot.upload(slot, s);
     d_lists.upload(lists, s);
     std::vector<int32_t>().swap(lists);
     d_dest = reinterpret_cast<const Dest*>(d_lists.get());

@@ -105,6 +105,45 @@ def test_stiffness_is_added_to_the_values(make, dtype):
     assert rel(once - host(values), K) < (1e-9 if dtype == torch.float64 else 1e-4)
 
 
+# Hex20 matrices on both sides of the size (about 26 cells) from which they are summed by rows: added to given values, and
+# combined into J = M + dt^2 K (in FP64 and rounded to FP32), with damping. K against the oracle as above; the
+# combination is the sum of its parts' values, each entry within a few roundings of its terms.
+@pytest.mark.parametrize("cells", [24, 28])
+@pytest.mark.parametrize("precision", [0, 3])
+def test_hex20_matrices_by_lists_and_by_rows(cells, precision):
+    from higher_order_embedded_fem_amd import fem
+
+    sc = scenes.cylinder_scene(cells, scenes.HEX20, 8)
+    om, gm = O.Model(sc), fem.ElasticityModel(sc)
+    mu, lam = scenes.lame_from_young_poisson(sc.young, sc.poisson)
+    mat = fem.StableNeoHookeanMaterial(mu=mu, lam=lam)
+    rng = np.random.default_rng(cells)
+    u = 0.005 * np.ptp(sc.vertices, axis=0).max() * rng.standard_normal(sc.ndof)
+    u.reshape(-1, 3)[sc.dirichlet_nodes] = 0.0
+    K = host(gm.assemble_stiffness_into(gm.zeros_matrix(), dev(u), mat))
+    if precision == 0:
+        assert rel(K, om.stiffness_add(mu, lam, u, np.zeros(om.nnz))) < 1e-9
+        start = np.abs(K).mean() * rng.standard_normal(om.nnz)
+        added = host(gm.assemble_stiffness_into(dev(start), dev(u), mat))
+        assert np.abs(added - (start + K)).max() <= 1e-14 * np.abs(K).max()
+    for damping in (0.0, 0.02):
+        sim = fem.NewtonCgIntegrator(gm, sc, schwarz=False, cg_max_iter=0, mixed_precision=precision, stiffness_damping=damping)
+        sim.set_state(0.0, dev(u), dev(np.zeros(sc.ndof)))
+        if damping:
+            sim.update_damping(dev(u))
+        sim.init_solve_jacobian_combination(-sc.dt * sc.dt, -sc.dt if damping else None)
+        sim.solve_jacobian_combination(dev(np.zeros(sc.ndof)), dev(np.zeros(sc.ndof)))
+        parts = [sc.dt * sc.dt * K, sc.dt * host(sim.damping()), host(sim.mass())]
+        rp, col = gm.pattern()
+        fixed = np.zeros(sc.ndof, bool)
+        fixed.reshape(-1, 3)[sc.dirichlet_nodes] = True
+        rows = np.repeat(np.arange(sc.ndof), np.diff(rp))
+        free = ~(fixed[rows] | fixed[col])
+        eps = 2.0 ** -52 if precision == 0 else 2.0 ** -23
+        off = np.abs(host(sim.jacobian()) - sum(parts))[free]
+        assert (off <= 4 * eps * sum(np.abs(p) for p in parts)[free]).all()
+
+
 # FP32 tangents of every element and material. A value sums at most a few hundred products with relative errors of
 # some eps, whose size the material's difference J - alpha raises up to tenfold: 500 eps = 3e-5 of the norm.
 @pytest.mark.parametrize("kind", [0, 1, 2])
