@@ -9,8 +9,8 @@
   substeps, simulation_toolbox/src/fem/newton_cg.rs:146-228) and one whose substepping gives up
   (Newton limit 1 at dt 0.2: status SUBSTEPPING): statuses, statistics and states equal the
   single-scene results, and the substepped scene matches the oracle in parity mode.
-* The FP32-operator precision modes (1 and 3) on a 12-scene batch: equal to each scene alone, bit
-  for bit.
+* The FP32-operator precision modes (1 and 3) on a 12-scene batch, by the resident grid and by the two-kernel
+  pools: equal to each scene alone, bit for bit.
 """
 
 import numpy as np
@@ -73,15 +73,18 @@ def test_batched_64_scenes_equal_each_scene_alone():
 
 
 @pytest.mark.timeout(600)
+@pytest.mark.parametrize("resident", [True, False], ids=["resident", "two_kernels"])
 @pytest.mark.parametrize("mode", [1, 3])
-def test_batched_fp32_operator_equals_each_scene_alone(mode):
+def test_batched_fp32_operator_equals_each_scene_alone(mode, resident):
     """The FP32-operator modes (1: FP32 tangents; 3: FP64 tangents rounded into the FP32 Jacobian) run
-    their batched solves on the FP32 CG kernels: 12 scenes of 2e3..3e4 DOFs, two batched steps, equal
-    to each scene stepped alone bit for bit."""
+    their batched solves on the FP32 CG kernels (scenes of this size on the resident grid, unless it is switched
+    off): 12 scenes of 2e3..3e4 DOFs, two batched steps, equal to each scene stepped alone bit for bit."""
     from higher_order_embedded_fem_amd import batch
 
     scs = batch.batched_scenes(12, seed=11, dof_range=(2e3, 3e4))
     stepper = batch.BatchedStepper(scs, newton_tolerance_factor=1e-6, mixed_precision=mode, autotune=True)
+    for m in stepper.models:
+        m.set_resident_solver(resident)
     steps = 2
     bstats = []
     for i in range(steps):
@@ -89,6 +92,7 @@ def test_batched_fp32_operator_equals_each_scene_alone(mode):
         assert all(s == 0 for s in r["status"]), r["status"]
         bstats.append(r["stats"])
     torch.cuda.synchronize()
+    assert all((m.resident_solver_stats()[0] > 0) == resident for m in stepper.models)
     print(f"mode {mode}: newton {[s['newton_iterations'] for s in bstats[-1]]}, "
           f"cg {[s['cg_iterations'] for s in bstats[-1]]}", flush=True)
     alone = run_alone(stepper, steps)

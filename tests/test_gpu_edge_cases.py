@@ -58,10 +58,13 @@ def fem():
     return F
 
 
-@pytest.fixture(scope="module")
-def tet1(fem):
+# both iterations of the conjugate gradients: the resident grid, which takes every system of this size by itself, and the
+# two kernels of larger ones
+@pytest.fixture(scope="module", params=[True, False], ids=["resident", "two_kernels"])
+def tet1(fem, request):
     sc = _single_tet()
     gm = fem.ElasticityModel(sc)
+    gm.set_resident_solver(request.param)
     rp, col = gm.pattern()
     assert len(col) == 144  # one element: every DOF couples with every DOF
     return sc, gm, rp, col
@@ -90,11 +93,13 @@ def test_cg_arbitrary_spd(fem, tet1):
     assert np.abs(host(x) - x0).max() <= 1e-12
 
 
-def test_cg_arbitrary_preconditioned_three_iterations(fem):
+@pytest.mark.parametrize("resident", [True, False])
+def test_cg_arbitrary_preconditioned_three_iterations(fem, resident):
     # Schwarz with the single subdomain {node 0}: its block of the update matrix is inv(p), so
     # the operator on node 0 is the reference's p; the other nodes are untreated with diagonal 1
     sc = _single_tet(subdomains=(0,), untreated=(1, 2, 3))
     gm = fem.ElasticityModel(sc)
+    gm.set_resident_solver(resident)
     rp, col = gm.pattern()
     a = np.array([[21.0, -1.0, -5.0], [-1.0, 11.0, -4.0], [-5.0, -4.0, 26.0]])
     p = np.array([[17.0, 6.0, 3.0], [6.0, 14.0, 9.0], [3.0, 9.0, 10.0]])
@@ -116,7 +121,7 @@ def test_cg_arbitrary_preconditioned_three_iterations(fem):
     xg[:3] = [2.0, 1.0, 0.0]  # the reference's initial guess
     x = dev(xg)
     it, st = fem.conjugate_gradient(gm, dev(_csr_values(rp, col, A)), dev(b), x, gsw, tol=1e-14, max_iter=100)
-    assert st == 0 and it == 3
+    assert st == 0 and it == 3 and gm.resident_solver_stats() == (int(resident), 0)
     assert np.abs(host(x) - x0).max() <= 1e-12
 
 

@@ -1,4 +1,5 @@
-"""The resident-grid PCG (every solve of a system that fits it) against the oracle's CG.
+"""The resident-grid PCG (every solve of a system that fits it) on systems with known solutions, each test beside the
+two-kernel iteration where both serve it.
 
 Sizes at its edges: fewer nodes than work-groups, one block per thread, blocks in registers, in LDS and in
 memory, rows of hundreds of blocks, several work-group counts; Schwarz and Jacobi; limits below, at and
@@ -57,13 +58,20 @@ def test_solution_matches_a_converged_residual(mesh, cells, element, subdomains,
     its, st = fem.conjugate_gradient(gm, Jd, b, x, pre, tol=1e-13, max_iter=20000)
     assert st == 0 and its > 0
     assert np.linalg.norm(x.cpu().numpy() - x_true) <= 1e-9 * np.linalg.norm(x_true)
+    assert gm.resident_solver_stats() == (1, 0)
     again = start.clone()  # the same launches: the same bits
     assert fem.conjugate_gradient(gm, Jd, b, again, pre, tol=1e-13, max_iter=20000) == (its, 0)
     assert torch.equal(x, again)
+    gm.set_resident_solver(False)
+    x = start.clone()
+    _, st = fem.conjugate_gradient(gm, Jd, b, x, pre, tol=1e-13, max_iter=20000)
+    assert st == 0 and gm.resident_solver_stats() == (2, 0)
+    assert np.linalg.norm(x.cpu().numpy() - x_true) <= 1e-9 * np.linalg.norm(x_true)
 
 
-@pytest.mark.parametrize("limit", [0, 1, 1023, 1024, 1025, 2300])
-def test_iteration_limits_across_launches(limit):
+# (the two kernels' launches are batches of 8 iterations; 2300 is the resident grid's third launch)
+@pytest.mark.parametrize("limit,resident", [(n, r) for r in (True, False) for n in (0, 1, 1023, 1024, 1025)] + [(2300, True)])
+def test_iteration_limits_across_launches(limit, resident):
     """A solve whose tolerance is never met stops at its limit, whether or not the limit is a launch's end; limits
     past a launch continue the same iteration: the iterate at 1025 is one step from the one at 1024."""
     from higher_order_embedded_fem_amd import fem
@@ -71,6 +79,7 @@ def test_iteration_limits_across_launches(limit):
     sc = scenes.cube_scene(3, scenes.TET10)
     _, _, J = system(sc, 1.0)
     gm = fem.ElasticityModel(sc)
+    gm.set_resident_solver(resident)
     Jd = torch.as_tensor(J, device="cuda")
     pre = fem.SchwarzPreconditioner.from_scene(gm, sc)
     pre.update(Jd)
@@ -80,6 +89,7 @@ def test_iteration_limits_across_launches(limit):
     # with tolerance 0 the iteration goes on after x has converged; p.Ap can then underflow to 0, which ends the
     # solve as an indefinite operator (status 6) before the limit
     assert (its, st) == (limit, 5) or (limit == 2300 and st == 6 and its > 1025)
+    assert gm.resident_solver_stats() == (int(resident), 0)
     assert bool(torch.isfinite(x).all())
     if limit == 0:
         assert not x.any()
@@ -93,20 +103,23 @@ def test_iteration_limits_across_launches(limit):
 
 
 def test_fp32_operator_matches_the_fp64_step():
-    """The FP32 operator inside the FP64 Newton loop (modes 1, 2, 3) reaches the FP64 step's solution: both
-    Newton loops stop at 1e-11 of the representative force, and the cube's Jacobian is well conditioned."""
+    """The FP32 operator inside the FP64 Newton loop (modes 1, 2, 3) reaches the FP64 step's solution, in either
+    iteration: both Newton loops stop at 1e-11 of the representative force, and the cube's Jacobian is well conditioned."""
     from higher_order_embedded_fem_amd import fem
 
     sc = scenes.cube_scene(7, scenes.TET10)
     ref = None
-    for mode in (0, 1, 2, 3):
+    for mode, resident in ((0, True), (1, True), (2, True), (3, True), (0, False), (1, False), (2, False), (3, False)):
         gm = fem.ElasticityModel(sc)
+        gm.set_resident_solver(resident)
         sim = fem.NewtonCgIntegrator(gm, sc, newton_tolerance_factor=1e-11, cg_tolerance=1e-7, cg_max_iter=5000,
                                      mixed_precision=mode)
         u = torch.zeros(sc.ndof, dtype=torch.float64, device="cuda")
         v = torch.zeros_like(u)
         sim.step(0.0, sc.dt, u, v)
-        if mode == 0:
+        solves, failures = gm.resident_solver_stats()
+        assert (solves > 0) == resident and failures == 0
+        if ref is None:
             ref = u.clone()
         else:
             assert float((u - ref).norm() / ref.norm()) < 1e-8

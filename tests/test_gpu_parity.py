@@ -196,12 +196,14 @@ def test_dirichlet_and_schwarz_match_oracle(fem, name):
     assert abs(it_g - it_o) <= max(2, it_o // 20)
 
 
+@pytest.mark.parametrize("resident", [True, False], ids=["resident", "two_kernels"])
 @pytest.mark.parametrize("name", ["cube3_tet10", "cyl8_hex20", "cyl8_hex20_emb"])
-def test_step_matches_oracle(fem, name):
+def test_step_matches_oracle(fem, name, resident):
     sc = SMALL_SCENES[name]()
     om = O.Model(sc)
     osim = O.Sim(om, newton_tolerance_factor=1e-9, cg_tolerance=1e-12, cg_max_iter=5000)
     gm = fem.ElasticityModel(sc)
+    gm.set_resident_solver(resident)
     gsim = fem.NewtonCgIntegrator(gm, sc, newton_tolerance_factor=1e-9, cg_tolerance=1e-12, cg_max_iter=5000)
     assert abs(gsim.representative_force - osim.representative_force) <= 1e-12 * osim.representative_force
     assert rel(host(gsim.mass()), osim.mass()) < 1e-12

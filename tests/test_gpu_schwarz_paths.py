@@ -59,8 +59,8 @@ def _hex27_cylinder():
     return sc, v, (1.0, 0.04, 0.03, 0.02)
 
 
-# 30 x 30 blocks (inverted on the matrix cores, k_spd_inverse_mf) and 81 x 81 blocks (in registers,
-# k_spd_inverse): each kernel's accepted, re-certified and rejected blocks
+# 30 x 30 and 81 x 81 blocks (two and six 16 x 16 tiles a side of k_spd_inverse_mf, by one wavefront and by eight):
+# each variant's accepted, re-certified and rejected blocks
 @pytest.mark.parametrize("make", [_tet10_cube, _hex27_cylinder], ids=["tet10_30x30", "hex27_81x81"])
 def test_block_inverse_paths(make):
     from higher_order_embedded_fem_amd import fem

@@ -2,7 +2,8 @@
 
 Two calls in a row on one GPU, the second on a smaller model (the scratch array keeps the first
 call's contents, which the second must not depend on), each compared with hoefem_pcg on the same
-system: same kernels and launch shapes, so the solution and the iteration count are identical.
+system: same kernels and launch shapes, so the solution and the iteration count are identical. By the resident grid,
+whose buffers an allocation-free call places in the scratch array, and by the two kernels.
 Also: the Jacobi variant, a zero right-hand side, the iteration limit, and the size limit.
 """
 
@@ -59,12 +60,17 @@ def fem():
     return F
 
 
-def test_noalloc_matches_pcg_on_two_calls_in_a_row(fem):
+PATHS = pytest.mark.parametrize("resident", [True, False], ids=["resident", "two_kernels"])
+
+
+@PATHS
+def test_noalloc_matches_pcg_on_two_calls_in_a_row(fem, resident):
     L = _lib.load()
     big = system(fem, scenes.cylinder_scene(8, scenes.HEX20, 8), 1)
     small = system(fem, scenes.cube_scene(3, scenes.TET10), 2)
     assert big[0].ndof > small[0].ndof
     for gm, sw, Jd, bd in (big, small):
+        gm.set_resident_solver(resident)
         for pre in (sw, None):  # Schwarz and Jacobi preconditioners
             st_r, it_r, x_r = solve(L.hoefem_pcg, gm, Jd, pre, bd, 1e-10, 5000)
             st_n, it_n, x_n = solve(L.hoefem_pcg_noalloc, gm, Jd, pre, bd, 1e-10, 5000)
@@ -76,11 +82,14 @@ def test_noalloc_matches_pcg_on_two_calls_in_a_row(fem):
                 assert st_r == 0
             assert it_n == it_r and it_r > 0
             assert np.array_equal(x_n, x_r)
+        assert gm.resident_solver_stats() == (4 if resident else 0, 0)
 
 
-def test_noalloc_limits_and_statuses(fem):
+@PATHS
+def test_noalloc_limits_and_statuses(fem, resident):
     L = _lib.load()
     gm, sw, Jd, bd = system(fem, scenes.cube_scene(3, scenes.TET10), 3)
+    gm.set_resident_solver(resident)
     # the iteration limit: the same status and partial solution as hoefem_pcg
     st_r, it_r, x_r = solve(L.hoefem_pcg, gm, Jd, sw, bd, 1e-14, 3)
     st_n, it_n, x_n = solve(L.hoefem_pcg_noalloc, gm, Jd, sw, bd, 1e-14, 3)
