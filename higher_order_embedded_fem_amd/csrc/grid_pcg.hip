@@ -572,6 +572,7 @@ constexpr int GRID_BLOCKS_PER_THREAD = 6, GRID_BLOCKS_ON_CHIP = 12, GRID_WIDE = 
 constexpr int GRID_MAX_SLOTS = 32;                 // bits of a thread's row-end mask
 constexpr size_t GRID_MAX_LDS = 143 * 1024;  // beside 16.3 KiB of fixed arrays
 constexpr int GRID_MAX_NODES = GRID_THREADS / 3;   // per work-group
+constexpr int64_t GRID_SETUP_BLOCKS = 1 << 16;     // blocks worth a host thread (about 0.3 ms of one)
 constexpr int GRID_SPARE = 8;                      // spare partial sums (row_sum)
 constexpr int64_t GRID_STATE_WORDS = (sizeof(GridState) + 255) / 256 * 32;
 
@@ -706,7 +707,7 @@ void GridPlan::build(const NodePattern& J, const NodePattern* P, int cus, hipStr
         }
     };
     // large patterns on a few host threads
-    const int nt = total < 100000 ? 1 : thread_count(total, 1);
+    const int nt = thread_count(total, GRID_SETUP_BLOCKS);
     run_on_threads(nt, [&](int i) { work(i, nt); });
     size_t nhalo = 0, ncol = 0, nrp = 0;
     lds_bytes = 0;

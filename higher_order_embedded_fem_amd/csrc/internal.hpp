@@ -5,6 +5,8 @@
 #include <hip/hip_ext.h>
 
 #include <cstdint>
+#include <cstring>
+#include <functional>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -69,6 +71,51 @@ struct DevBuf {
     T* get() const { return p; }
 };
 
+// An array inside a DevPack
+template <class T>
+struct DevView {
+    T* p = nullptr;
+    T* get() const { return p; }
+};
+
+// Host arrays that are uploaded together, at setup, into one allocation: an allocation and a copy for each of some
+// thirty arrays took a quarter of a small model's setup. Up to STAGE bytes go in one copy.
+class DevPack {
+public:
+    template <class T>
+    void add(const std::vector<T>& v, DevView<T>& out) {
+        items_.push_back({v.data(), v.size() * sizeof(T), total_, [&out](char* at) { out.p = reinterpret_cast<T*>(at); }});
+        total_ += (v.size() * sizeof(T) + 255) / 256 * 256;
+    }
+    void upload(hipStream_t s) {  // blocking, as DevBuf::upload
+        buf_.alloc(total_ ? total_ : 1);
+        HIP_CHECK(hipStreamSynchronize(s));
+        if (total_ <= STAGE) {
+            std::vector<char> all(total_);
+            for (const Item& i : items_)
+                if (i.bytes) std::memcpy(all.data() + i.at, i.src, i.bytes);
+            if (total_) HIP_CHECK(hipMemcpy(buf_.get(), all.data(), total_, hipMemcpyHostToDevice));
+        } else {
+            for (const Item& i : items_)
+                if (i.bytes) HIP_CHECK(hipMemcpy(buf_.get() + i.at, i.src, i.bytes, hipMemcpyHostToDevice));
+        }
+        for (const Item& i : items_) i.set(buf_.get() + i.at);
+        items_.clear();
+        total_ = 0;
+    }
+
+private:
+    static constexpr size_t STAGE = 1 << 20;
+    struct Item {
+        const void* src;
+        size_t bytes, at;
+        std::function<void(char*)> set;
+    };
+    std::vector<Item> items_;
+    size_t total_ = 0;
+    DevBuf<char> buf_;
+};
+
 template <class T>
 struct PinnedBuf {
     T* p = nullptr;
@@ -112,16 +159,15 @@ struct NodePattern {
     std::vector<uint8_t> diag_only;   // per node
     int max_nbr = 0;
     int tuned_group = 0;  // lanes per node row block chosen by autotune_spmv (0: heuristic)
-    DevBuf<int32_t> d_nptr, d_ncol, d_rowptr, d_col, d_diag_pos;
-    DevBuf<uint8_t> d_diag_only;
+    DevPack pack;  // the arrays on the device
+    DevView<int32_t> d_nptr, d_ncol, d_rowptr, d_col, d_diag_pos;
+    DevView<uint8_t> d_diag_only;
     std::vector<NodeEntry> entries;   // block nodes, then diagonal-only nodes
     int64_t n_block = 0, n_diag = 0;
-    DevBuf<NodeEntry> d_entries;
+    DevView<NodeEntry> d_entries;
     int64_t nnz() const { return (int64_t)col.size(); }
     int64_t ndof() const { return 3 * num_nodes; }
     int32_t find(int32_t a, int32_t b) const;  // local index of b in nbr(a), or -1
-    // slot[i m + j] = find(node i, node j) for the m nodes of a set
-    void find_pairs(const int32_t* set, int m, int32_t* slot) const;
     void upload(hipStream_t s);
 };
 
@@ -136,7 +182,7 @@ std::vector<std::vector<int32_t>> greedy_coloring(int64_t nsets, const int64_t* 
 
 // Color-ordered incidence of dense blocks ("element matrices") into a node pattern; shared
 // by the stiffness / mass assembly and the Schwarz preconditioner assembly.
-constexpr int64_t SETUP_ENTRIES = 1 << 15;  // block entries worth a host thread (about 1 ms of one)
+constexpr int64_t SETUP_ENTRIES = 1 << 16;  // block entries worth a host thread (about 0.3 ms of one)
 struct BlockScatter {
     int64_t nblocks = 0;
     std::vector<int32_t> m;         // nodes per block
@@ -154,15 +200,20 @@ struct BlockScatter {
     int64_t ndest = 0;
     int row_stride = 0;
     std::vector<int32_t> lists;  // dest (two words each), term_ptr, term, term_row
-    DevBuf<int32_t> d_lists;
+    DevPack pack;  // the arrays on the device
+    DevView<int32_t> d_lists;
     const Dest* d_dest = nullptr;
     const int32_t *d_term_ptr = nullptr, *d_term_row = nullptr;
     const uint32_t* d_term = nullptr;
     bool by_rows = false;  // FP64 blocks are summed by k_block_gather_pf, which reads slot
-    DevBuf<int32_t> d_m, d_slot, d_inc_ptr, d_inc_blk, d_inc_loc;
-    DevBuf<int64_t> d_val_off, d_slot_off;
+    DevView<int32_t> d_m, d_slot, d_inc_ptr, d_inc_blk, d_inc_loc;
+    DevView<int64_t> d_val_off, d_slot_off;
     void build(const NodePattern& pat, int64_t nblocks, const int64_t* off, const int32_t* nodes,
                const std::vector<std::vector<int32_t>>* colors, int ncolor_lists);
+    // out, laid out as slot: the blocks' nodes in the rows v0 .. v1 - 1 of another pattern, -1 where it does not couple
+    // them. pos: a work array of -1 per node, left so.
+    void slots_in(const NodePattern& pat, const int64_t* off, const int32_t* nodes, int64_t v0, int64_t v1,
+                  std::vector<int32_t>& pos, int32_t* out) const;
     void upload(hipStream_t s);
 };
 
@@ -325,8 +376,9 @@ struct Schwarz {
     GridPlan grid;                 // resident-grid solves of the model's matrix with this preconditioner
     BlockScatter scatter;          // blocks -> P pattern
     std::vector<int32_t> jslot;    // per block entry (a, c): local index of node c in J's nbr(node a)
-    DevBuf<int32_t> d_jslot, d_untreated, d_nodes;
-    DevBuf<int64_t> d_off;
+    DevPack pack;                  // the index arrays on the device
+    DevView<int32_t> d_jslot, d_untreated, d_nodes;
+    DevView<int64_t> d_off;
     bool fp32 = false;             // P stored in FP32 (mixed precision)
     DevBuf<double> d_vals;         // P values (FP64)
     DevBuf<float> d_vals32;        // P values (FP32)

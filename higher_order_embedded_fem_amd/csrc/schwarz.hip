@@ -45,10 +45,8 @@ void schwarz_setup(Schwarz& s, Model& m, int64_t nsub, const int64_t* off, const
     int64_t panel_total = 0;
     const int nt = thread_count((int64_t)s.jslot.size(), SETUP_ENTRIES);
     run_on_threads(nt, [&](int t) {
-        for (int64_t b = t * nsub / nt; b < (t + 1) * nsub / nt; ++b) {
-            m.pattern.find_pairs(s.nodes.data() + s.off[b], (int)(s.off[b + 1] - s.off[b]),
-                                 s.jslot.data() + s.scatter.slot_off[b]);
-        }
+        std::vector<int32_t> pos(m.nv, -1);
+        s.scatter.slots_in(m.pattern, s.off.data(), s.nodes.data(), t * m.nv / nt, (t + 1) * m.nv / nt, pos, s.jslot.data());
     });
     for (int64_t b = 0; b < nsub; ++b) {
         const int mb = (int)(s.off[b + 1] - s.off[b]);
@@ -68,10 +66,11 @@ void schwarz_setup(Schwarz& s, Model& m, int64_t nsub, const int64_t* off, const
     s.P.upload(m.stream);
     s.grid.build(m.pattern, &s.P, grid_device_cus(), m.stream);
     s.scatter.upload(m.stream);
-    s.d_jslot.upload(s.jslot, m.stream);
-    s.d_untreated.upload(s.untreated, m.stream);
-    s.d_off.upload(s.off, m.stream);
-    s.d_nodes.upload(s.nodes, m.stream);
+    s.pack.add(s.jslot, s.d_jslot);
+    s.pack.add(s.untreated, s.d_untreated);
+    s.pack.add(s.off, s.d_off);
+    s.pack.add(s.nodes, s.d_nodes);
+    s.pack.upload(m.stream);
     if (s.fp32) {
         s.d_vals32.ensure(std::max<int64_t>(s.P.nnz(), 1));
         HIP_CHECK(hipMemsetAsync(s.d_vals32.get(), 0, sizeof(float) * s.d_vals32.n, m.stream));

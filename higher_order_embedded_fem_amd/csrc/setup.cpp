@@ -81,29 +81,13 @@ int32_t NodePattern::find(int32_t a, int32_t b) const {
     return (int32_t)(it - lo);
 }
 
-void NodePattern::find_pairs(const int32_t* set, int m, int32_t* slot) const {
-    std::vector<std::pair<int32_t, int32_t>> sorted(m);  // node, place in the set
-    for (int j = 0; j < m; ++j) sorted[j] = {set[j], j};
-    std::sort(sorted.begin(), sorted.end());
-    for (int i = 0; i < m; ++i) {  // the set's nodes and the row's neighbours are both in order
-        const int32_t *nb = ncol.data() + nptr[set[i]], *end = ncol.data() + nptr[set[i] + 1], *p = nb;
-        for (const auto& [node, j] : sorted) {
-            if (end - p > 16)
-                p = std::lower_bound(p, end, node);
-            else
-                while (p < end && *p < node) ++p;
-            slot[(int64_t)i * m + j] = p < end && *p == node ? (int32_t)(p - nb) : -1;
-        }
-    }
-}
-
 void NodePattern::upload(hipStream_t s) {
-    d_nptr.upload(nptr, s);
-    d_ncol.upload(ncol, s);
-    d_rowptr.upload(rowptr, s);
-    d_col.upload(col, s);
-    d_diag_pos.upload(diag_pos, s);
-    d_diag_only.upload(diag_only, s);
+    pack.add(nptr, d_nptr);
+    pack.add(ncol, d_ncol);
+    pack.add(rowptr, d_rowptr);
+    pack.add(col, d_col);
+    pack.add(diag_pos, d_diag_pos);
+    pack.add(diag_only, d_diag_only);
     entries.clear();
     for (int64_t v = 0; v < num_nodes; ++v)
         if (!diag_only[v])
@@ -112,7 +96,8 @@ void NodePattern::upload(hipStream_t s) {
     for (int64_t v = 0; v < num_nodes; ++v)
         if (diag_only[v]) entries.push_back(NodeEntry{(int32_t)v, 0, 0, rowptr[3 * v]});
     n_diag = (int64_t)entries.size() - n_block;
-    d_entries.upload(entries, s);
+    pack.add(entries, d_entries);
+    pack.upload(s);
 }
 
 uint64_t next_pattern_id() {
@@ -289,6 +274,21 @@ std::vector<std::vector<int32_t>> greedy_coloring(int64_t nsets, const int64_t* 
     return colors;
 }
 
+// A row's places are put down per node once and looked up by all the blocks at the row's node
+void BlockScatter::slots_in(const NodePattern& pat, const int64_t* off, const int32_t* nodes, int64_t v0, int64_t v1,
+                            std::vector<int32_t>& pos, int32_t* out) const {
+    for (int64_t v = v0; v < v1; ++v) {
+        const int32_t *row = pat.ncol.data() + pat.nptr[v], k = pat.nptr[v + 1] - pat.nptr[v];
+        for (int32_t j = 0; j < k; ++j) pos[row[j]] = j;
+        for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
+            const int32_t b = inc_blk[it], *g = nodes + off[b];
+            int32_t* sl = out + slot_off[b] + (int64_t)inc_loc[it] * m[b];
+            for (int32_t c = 0; c < m[b]; ++c) sl[c] = pos[g[c]];
+        }
+        for (int32_t j = 0; j < k; ++j) pos[row[j]] = -1;
+    }
+}
+
 void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off, const int32_t* nodes,
                          const std::vector<std::vector<int32_t>>* color_lists, int ncolor_lists) {
     nblocks = nb;
@@ -302,15 +302,6 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
         slot_off[b + 1] = slot_off[b] + (int64_t)m[b] * m[b];
     }
     slot.resize(slot_off[nb]);
-    const int nt = thread_count(slot_off[nb], SETUP_ENTRIES);
-    run_on_threads(nt, [&](int t) {
-        for (int64_t b = t * nb / nt; b < (t + 1) * nb / nt; ++b) {
-            int32_t* sl = slot.data() + slot_off[b];
-            pat.find_pairs(nodes + off[b], m[b], sl);
-            if (std::find(sl, sl + (int64_t)m[b] * m[b], -1) != sl + (int64_t)m[b] * m[b])
-                throw Error(HOEFEM_ERROR_PATTERN, "block entry missing from CSR pattern");
-        }
-    });
     inc_ptr.assign(pat.num_nodes + 1, 0);
     for (int l = 0; l < ncolor_lists; ++l)
         for (const auto& color : color_lists[l])
@@ -355,9 +346,11 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
         first[v + 1] = first[v];
         for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) first[v + 1] += m[inc_blk[it]];
     }
+    const int nt = thread_count(nterms, SETUP_ENTRIES);
     run_on_threads(nt, [&](int t) {
-        std::vector<int32_t> at;
+        std::vector<int32_t> pos(nn, -1), at;
         for (int64_t v = t * nn / nt; v < (t + 1) * nn / nt; ++v) {
+            slots_in(pat, off, nodes, v, v + 1, pos, slot.data());
             const int32_t b0 = pat.nptr[v], k = pat.nptr[v + 1] - b0;
             for (int j = 0; j < k; ++j)
                 dest[b0 + j] = pat.diag_only[v] ? Dest{0, 0} : Dest{pat.rowptr[3 * v] + 3 * j, 3 * k};
@@ -365,7 +358,10 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
             for (int32_t it = inc_ptr[v]; it < inc_ptr[v + 1]; ++it) {
                 const int32_t b = inc_blk[it], mb = m[b];
                 const int32_t* sl = slot.data() + slot_off[b] + (int64_t)inc_loc[it] * mb;
-                for (int c = 0; c < mb; ++c) at[sl[c]]++;
+                for (int c = 0; c < mb; ++c) {
+                    if (sl[c] < 0) throw Error(HOEFEM_ERROR_PATTERN, "block entry missing from CSR pattern");
+                    at[sl[c]]++;
+                }
             }
             int32_t end = first[v];
             for (int j = 0; j < k; ++j) {
@@ -389,19 +385,20 @@ void BlockScatter::build(const NodePattern& pat, int64_t nb, const int64_t* off,
 }
 
 void BlockScatter::upload(hipStream_t s) {
-    d_m.upload(m, s);
-    if (by_rows) d_slot.upload(slot, s);
-    d_lists.upload(lists, s);
+    pack.add(m, d_m);
+    if (by_rows) pack.add(slot, d_slot);
+    pack.add(lists, d_lists);
+    pack.add(inc_ptr, d_inc_ptr);
+    pack.add(inc_blk, d_inc_blk);
+    pack.add(inc_loc, d_inc_loc);
+    pack.add(val_off, d_val_off);
+    pack.add(slot_off, d_slot_off);
+    pack.upload(s);
     std::vector<int32_t>().swap(lists);
     d_dest = reinterpret_cast<const Dest*>(d_lists.get());
     d_term_ptr = d_lists.get() + 2 * ndest;
     d_term = reinterpret_cast<const uint32_t*>(d_term_ptr + ndest + 1);
     d_term_row = d_term_ptr + ndest + 1 + slot_off[nblocks];
-    d_inc_ptr.upload(inc_ptr, s);
-    d_inc_blk.upload(inc_blk, s);
-    d_inc_loc.upload(inc_loc, s);
-    d_val_off.upload(val_off, s);
-    d_slot_off.upload(slot_off, s);
 }
 
 }  // namespace hoefem
