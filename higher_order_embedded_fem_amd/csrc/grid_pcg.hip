@@ -34,9 +34,9 @@
 // before anyone can poll phase m + 2.
 //
 // Residency. The work-groups wait for each other, so all of a launch's must be resident: launches are
-// admitted against the device's number of CUs (GridSlots below), one work-group per CU. Every wait is
-// bounded (GRID_POLL_LIMIT polls); a launch that cannot make progress ends with an error status and the caller
-// falls back to the two-kernel path.
+// admitted in order against the CUs of every XCD (GridSlots below), one work-group per CU. Every wait is
+// bounded (GRID_POLL_LIMIT polls); a launch that cannot make progress, because another process holds CUs, ends with
+// an error status, the caller falls back to the two-kernel path, and so do its next solves (GridRest).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -55,7 +55,8 @@ constexpr unsigned long long GRID_EMPTY = 0x7ff4deadbeef0001ull;  // slot sentin
 constexpr int GRID_POLL_LIMIT = 1 << 21;                           // about 2 s of polling
 constexpr int GRID_WAVES = GRID_THREADS / 64;
 // copies of the partial sums, each read by an eighth of the work-groups: 256 work-groups polling one array
-// queue at its few memory channels (3.1 us per exchange at 256 work-groups against 2.4 with 8 copies)
+// queue at its few memory channels (an exchange of partial sums alone takes 1.5 us at 8 work-groups, 2.3 at 256 with 8
+// copies and 3.1 with one)
 constexpr int GRID_COPIES = 8;
 
 __device__ inline double agent_load(const double* p) {
@@ -562,8 +563,9 @@ __global__ __launch_bounds__(GRID_THREADS) __attribute__((amdgpu_waves_per_eu(2,
 }
 
 // ------------------------------------------------------------------ plan
-// W: a phase's exchange grows from 2.9 us at 8 work-groups to 5.1 us at 256 while its products shrink with
-// 1/W (about 0.13 us per block of a thread), so small systems take few work-groups: enough for
+// W: an exchange with its vector entries takes 2.6 us at 8 work-groups, 2.9 at 80 and 3.9 at 216 to 240 (5.1 where it
+// waits for work-groups whose halo is past the entries taken in meanwhile), the two phases' products together 2.0, 2.4 and 3.5 us with
+// 4, 7 and 13 blocks per thread, and both grow or shrink with W, so small systems take few work-groups: enough for
 // GRID_BLOCKS_PER_THREAD blocks per thread, at least 8. Past GRID_WIDE work-groups the two balance over a wide
 // range of W, and a system takes no more than what still keeps its blocks on the chip
 // (GRID_BLOCKS_ON_CHIP per thread): alone it is as fast (48 to 74 thousand DOFs: -4 to +2.5 %), and two of a
