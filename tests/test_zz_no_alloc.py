@@ -85,6 +85,19 @@ def test_noalloc_matches_pcg_on_two_calls_in_a_row(fem, resident):
         assert gm.resident_solver_stats() == (4 if resident else 0, 0)
 
 
+def test_noalloc_matches_pcg_where_blocks_are_kept_in_memory(fem):
+    """A cube of 107,811 DOFs, more blocks per thread than the chip holds: those past the registers and the LDS of its
+    resident grid do not fit the fixed array."""
+    L = _lib.load()
+    gm, sw, Jd, bd = system(fem, scenes.cube_scene(16, scenes.TET10), 4)
+    for pre in (sw, None):
+        st_r, it_r, x_r = solve(L.hoefem_pcg, gm, Jd, pre, bd, 1e-10, 3000)
+        for _ in range(2):
+            st_n, it_n, x_n = solve(L.hoefem_pcg_noalloc, gm, Jd, pre, bd, 1e-10, 3000)
+            assert st_n == st_r == 0 and it_n == it_r > 0 and np.array_equal(x_n, x_r)
+    assert gm.resident_solver_stats() == (6, 0)
+
+
 @PATHS
 def test_noalloc_limits_and_statuses(fem, resident):
     L = _lib.load()
